@@ -87,3 +87,31 @@ def test_learned_scheduler_without_cdf_cache(C):
     print("held-out regret (no CDF cache)", r)
     assert r["chunks"] > 100
     assert r["mlp"] < r["heuristic"], r
+
+
+@pytest.mark.parametrize("n", [1, 31, 127, 128, 129, 300])
+def test_gradient_tile_edges(C, n):
+    """Minibatch sizes around the parameter kernel's 128-row tiles: gradients
+    (grad) and the update of one whole-batch step (train) against FP64."""
+    m = C.Mlp(9)
+    X, T, M = data(n, 40 + n)
+    M[0, 0] = 1.0
+    p0 = m.params()
+    w = MO.bf16_round(p0)
+    _, wg = MO.loss_grad(w, X, T, M)
+    # FP32 chains of at most n rows over values from chains of at most 64 + 64
+    # + 16 + 8 terms; 8 covers the growth through the three layers
+    y, (_, a1, h1, a2, h2) = MO.forward(w, X)
+    dy = np.abs((y - T) * M) / M.sum()
+    P = MO.unpack(w)
+    d2 = dy @ np.abs(P["W3"])
+    d1 = d2 @ np.abs(P["W2"])
+    size = max((d1.T @ np.abs(X)).max(), (d2.T @ h1).max(), (dy.T @ h2).max(), d1.sum(0).max(), d2.sum(0).max(),
+               dy.sum(0).max())
+    tol = 8 * (n + 152) * 2.0 ** -24 * size
+    loss, g = m.grad(X, T, M)
+    assert np.abs(g - wg).max() <= tol
+    lr = 0.5
+    m.train(X, T, M, epochs=1, batch=n, lr=lr)
+    step = (p0.astype(np.float64) - m.params()) / lr
+    assert np.abs(step - wg).max() <= tol + 2.0 ** -23 * np.abs(p0).max() / lr
