@@ -92,7 +92,8 @@ struct GraphDev {
 struct ReqDev {
   int32_t fanout[CSAW_MAX_HOPS];
   int32_t depth, bias, dedup, samples;
-  uint32_t key_lo, key_hi, request_id, pad;
+  uint32_t key_lo, key_hi, request_id;
+  uint32_t slot;  // the request's row of the bounds table (HopDev)
   int64_t gbase;
 };
 
@@ -134,6 +135,10 @@ struct HopDev {
   int32_t chunk_min;    // smallest chunk piece (a power of two, kChunkMin .. kBlockEntries)
   int32_t group_min;    // smallest sub-wave group (kGroupMin .. 32)
   int32_t only_kind;    // 1 + a bias kind: expand only that kind's entries (0: all)
+  // edge bounds of each request's hops, bounds[(slot * CSAW_MAX_HOPS + hop) * 2 + {0, 1}]
+  // (null: not wanted), so that a host needs one copy to place every request
+  int64_t* bounds;
+  int32_t n_req;
 };
 
 // Hops of a batched plan with at most this many frontier entries skip the

@@ -113,6 +113,8 @@ static void plan_free(csaw_plan* p) {
     if (p->join[i]) (void)hipEventDestroy(p->join[i]);
   }
   if (p->fork) (void)hipEventDestroy(p->fork);
+  if (p->begin) (void)hipEventDestroy(p->begin);
+  if (p->end) (void)hipEventDestroy(p->end);
   delete p;
 }
 
@@ -137,6 +139,7 @@ static int build_unit(csaw_plan* p, Unit& u) {
     d.key_lo = (uint32_t)r.seed;
     d.key_hi = (uint32_t)(r.seed >> 32);
     d.request_id = r.request_id;
+    d.slot = (uint32_t)ri;
     d.gbase = u.G;
     u.gbase.push_back(u.G);
     rd.push_back(d);
@@ -239,6 +242,8 @@ static HopDev make_hop(csaw_plan* p, Unit& u, int h) {
   H.chunk_min = p->L.chunk_min;
   H.group_min = p->L.group_min;
   H.only_kind = 0;
+  H.bounds = p->bounds;
+  H.n_req = (int32_t)u.reqs.size();
   return H;
 }
 
@@ -266,7 +271,7 @@ static int run_unit(csaw_plan* p, Unit& u, hipStream_t st, TimingHook* th) {
     CSAW_TRY(launch_count(L, G, u.d_req, u.d_gs2req, H, bin, u.nmax[h]));
     if (th) th->end(kKernCount, st);
     if (th) th->begin(kKernScan, st);
-    CSAW_TRY(launch_scans(L, H, p->totals + h, u.nmax[h]));
+    CSAW_TRY(launch_scans(L, H, u.d_req, p->totals + h, u.nmax[h]));
     if (th) th->end(kKernScan, st);
     if (bin) {
       ChooseArgs A;
@@ -419,8 +424,13 @@ extern "C" int csaw_plan_create(csaw_graph* g, const csaw_request* reqs, int32_t
     CSAW_HIP(hipMalloc(&p->local_excl, sizeof(uint32_t) * nmax));
     CSAW_HIP(hipMalloc(&p->blk_excl, sizeof(uint32_t) * nblk));
     CSAW_HIP(hipMalloc(&p->grp_excl, sizeof(uint64_t) * ngrp));
-    CSAW_HIP(hipMalloc(&p->counters, sizeof(uint32_t) * kCtrCount));
-    CSAW_HIP(hipMemset(p->counters, 0, sizeof(uint32_t) * kCtrCount));
+    const size_t state = kCtrBytes + kBoundsBytes * (size_t)n_req;
+    CSAW_HIP(hipMalloc(&p->counters, state));
+    CSAW_HIP(hipMemset(p->counters, 0, state));
+    p->bounds = reinterpret_cast<int64_t*>(reinterpret_cast<char*>(p->counters) + kCtrBytes);
+    p->h_state.assign(state / sizeof(uint32_t), 0u);
+    CSAW_HIP(hipEventCreate(&p->begin));
+    CSAW_HIP(hipEventCreate(&p->end));
     CSAW_HIP(hipMalloc(&p->totals, sizeof(int64_t) * depth));
     CSAW_HIP(hipMalloc(&p->bytes_acc, sizeof(unsigned long long) * kNumKernKinds));
     CSAW_HIP(hipMemset(p->bytes_acc, 0, sizeof(unsigned long long) * kNumKernKinds));
@@ -468,11 +478,10 @@ extern "C" int csaw_plan_run(csaw_plan* p, void* stream, int sync) {
   hipStream_t st = stream ? (hipStream_t)stream : p->stream;
   p->hop_logs.clear();
   p->pending_log_hops.clear();
-  hipEvent_t e0, e1;
-  CSAW_HIP(hipEventCreate(&e0));
-  CSAW_HIP(hipEventCreate(&e1));
-  CSAW_HIP(hipEventRecord(e0, st));
+  p->bounds_known = false;
   TimingHook* th = p->timer.enabled ? &p->timer : nullptr;
+  const bool wait = sync || th;
+  if (wait) CSAW_HIP(hipEventRecord(p->begin, st));
   if (th) {
     LaunchCfg L = p->L;
     L.stream = st;
@@ -501,16 +510,19 @@ extern "C" int csaw_plan_run(csaw_plan* p, void* stream, int sync) {
     }
     CSAW_HIP(hipGraphLaunch(p->gexec, st));
   } else {
-    for (auto& u : p->units) {
-      CSAW_TRY(run_unit(p, u, st, th));
-      if (p->opts.mode == CSAW_MODE_PLAIN) CSAW_HIP(hipStreamSynchronize(st));
+    for (size_t i = 0; i < p->units.size(); ++i) {
+      CSAW_TRY(run_unit(p, p->units[i], st, th));
+      // (the last one's wait is the run's own, below)
+      if (p->opts.mode == CSAW_MODE_PLAIN && !(wait && i + 1 == p->units.size())) CSAW_HIP(hipStreamSynchronize(st));
     }
   }
-  CSAW_HIP(hipEventRecord(e1, st));
-  if (sync || th) {
-    CSAW_HIP(hipEventSynchronize(e1));
+  if (wait) {
+    CSAW_HIP(hipEventRecord(p->end, st));
+    CSAW_HIP(hipMemcpyAsync(p->h_state.data(), p->counters, sizeof(uint32_t) * p->h_state.size(), hipMemcpyDeviceToHost,
+                            st));
+    CSAW_HIP(hipStreamSynchronize(st));
     float ms = 0.f;
-    CSAW_HIP(hipEventElapsedTime(&ms, e0, e1));
+    CSAW_HIP(hipEventElapsedTime(&ms, p->begin, p->end));
     p->last_ms = ms;
     if (th) {
       p->timer.collect();
@@ -518,33 +530,31 @@ extern "C" int csaw_plan_run(csaw_plan* p, void* stream, int sync) {
       CSAW_HIP(hipMemcpy(b, p->bytes_acc, sizeof(b), hipMemcpyDeviceToHost));
       for (int k = 0; k < kNumKernKinds; ++k) p->timer.total_bytes[k] += (double)b[k];
     }
-    uint32_t flags = 0;
-    CSAW_HIP(hipMemcpy(&flags, p->counters + kCtrFlags, sizeof(uint32_t), hipMemcpyDeviceToHost));
-    if (flags & 1u) {
+    if (p->h_state[kCtrFlags] & 1u) {
       set_last_error("chunk descriptor capacity exceeded");
-      (void)hipEventDestroy(e0);
-      (void)hipEventDestroy(e1);
       return CSAW_ERR_CAPACITY;
     }
+    p->bounds_known = true;
   }
-  CSAW_HIP(hipEventDestroy(e0));
-  CSAW_HIP(hipEventDestroy(e1));
   p->runs += 1;
   return CSAW_OK;
 }
 
 // Per-request hop boundaries: hop h edges of request r are
-// [eo_h[gbase], eo_h[gbase + S]) of its unit's hop-h arrays.
+// [eo_h[gbase], eo_h[gbase + S]) of its unit's hop-h arrays.  A synchronised
+// run has brought them to the host; after any other they are read here.
 static int request_bounds(const csaw_plan* p, int32_t req, std::vector<int64_t>& lo, std::vector<int64_t>& hi) {
   if (req < 0 || req >= (int32_t)p->reqs.size()) return CSAW_ERR_INVALID_ARG;
-  const auto [ui, k] = p->req_unit[req];
-  const Unit& u = p->units[ui];
-  const csaw_request& r = p->reqs[req];
-  lo.assign(r.depth, 0);
-  hi.assign(r.depth, 0);
-  for (int h = 0; h < r.depth; ++h) {
-    CSAW_HIP(hipMemcpy(&lo[h], u.d_eo[h] + u.gbase[k], sizeof(int64_t), hipMemcpyDeviceToHost));
-    CSAW_HIP(hipMemcpy(&hi[h], u.d_eo[h] + u.gbase[k] + r.samples, sizeof(int64_t), hipMemcpyDeviceToHost));
+  const int32_t depth = p->reqs[req].depth;
+  int64_t read[2 * CSAW_MAX_HOPS];
+  const char* known = reinterpret_cast<const char*>(p->h_state.data()) + kCtrBytes + kBoundsBytes * (size_t)req;
+  if (p->bounds_known) memcpy(read, known, kBoundsBytes);
+  else CSAW_HIP(hipMemcpy(read, p->bounds + (size_t)req * 2 * CSAW_MAX_HOPS, kBoundsBytes, hipMemcpyDeviceToHost));
+  lo.resize(depth);
+  hi.resize(depth);
+  for (int h = 0; h < depth; ++h) {
+    lo[h] = read[2 * h];
+    hi[h] = read[2 * h + 1];
   }
   return CSAW_OK;
 }
@@ -588,17 +598,6 @@ extern "C" int csaw_plan_copy(const csaw_plan* p, int32_t req, int32_t* src, int
   return CSAW_OK;
 }
 
-namespace csaw {
-__global__ void k_sub_i32(int32_t* __restrict__ x, int64_t n, int32_t sub) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    x[i] -= sub;
-}
-__global__ void k_add_i64(const int64_t* __restrict__ in, int64_t n, int64_t add, int64_t* __restrict__ out) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    out[i] = in[i] + add;
-}
-}  // namespace csaw
-
 // csaw_plan_copy into device buffers, on the device (for callers that keep
 // the edge lists on the GPU, e.g. as framework tensors).
 extern "C" int csaw_plan_copy_device(const csaw_plan* p, int32_t req, int32_t* src, int32_t* dst, int32_t* sample,
@@ -610,28 +609,27 @@ extern "C" int csaw_plan_copy_device(const csaw_plan* p, int32_t req, int32_t* s
   const Unit& u = p->units[ui];
   const csaw_request& r = p->reqs[req];
   hipStream_t st = stream ? (hipStream_t)stream : p->stream;
-  auto grid = [&](int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 4096)); };
+  CopyArgs A;
+  memset(&A, 0, sizeof(A));
   int64_t at = 0;
   for (int h = 0; h < r.depth; ++h) {
-    const int64_t n = hi[h] - lo[h];
-    if (n > 0) {
-      if (src) CSAW_HIP(hipMemcpyAsync(src + at, u.d_src[h] + lo[h], sizeof(int32_t) * n, hipMemcpyDeviceToDevice, st));
-      if (dst) CSAW_HIP(hipMemcpyAsync(dst + at, u.d_dst[h] + lo[h], sizeof(int32_t) * n, hipMemcpyDeviceToDevice, st));
-      if (sample) {
-        CSAW_HIP(hipMemcpyAsync(sample + at, u.d_smp[h] + lo[h], sizeof(int32_t) * n, hipMemcpyDeviceToDevice, st));
-        if (u.gbase[k]) {
-          k_sub_i32<<<grid(n), 256, 0, st>>>(sample + at, n, (int32_t)u.gbase[k]);
-          CSAW_LAUNCH_CHECK();
-        }
-      }
-    }
-    if (hop_offsets) {
-      k_add_i64<<<grid(r.samples + 1), 256, 0, st>>>(u.d_eo[h] + u.gbase[k], r.samples + 1, at - lo[h],
-                                                     hop_offsets + (int64_t)h * (r.samples + 1));
-      CSAW_LAUNCH_CHECK();
-    }
-    at += n;
+    A.col[0][h] = u.d_src[h];
+    A.col[1][h] = u.d_dst[h];
+    A.col[2][h] = u.d_smp[h];
+    A.eo[h] = u.d_eo[h] + u.gbase[k];
+    A.lo[h] = lo[h];
+    A.n[h] = hi[h] - lo[h];
+    A.at[h] = at;
+    at += A.n[h];
   }
+  A.out[0] = src;
+  A.out[1] = dst;
+  A.out[2] = sample;
+  A.hop_offsets = hop_offsets;
+  A.rows = (int64_t)r.samples + 1;
+  A.depth = r.depth;
+  A.sub = (int32_t)u.gbase[k];
+  CSAW_TRY(launch_copy_edges(st, A));
   if (sync) CSAW_HIP(hipStreamSynchronize(st));
   return CSAW_OK;
 }

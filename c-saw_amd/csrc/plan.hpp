@@ -16,6 +16,9 @@ enum : int {
   kCtrFlags = kCtrQhead + kNumQueues,
   kCtrCount = kCtrFlags + 1
 };
+static_assert(kCtrCount <= 64, "the bounds table starts 64 words after the counters");
+constexpr size_t kCtrBytes = 64 * sizeof(uint32_t);  // counters, padded
+constexpr size_t kBoundsBytes = 2 * CSAW_MAX_HOPS * sizeof(int64_t);  // one request's edge bounds
 
 struct EventTimer : TimingHook {
   struct Rec {
@@ -80,7 +83,13 @@ struct csaw_plan {
   uint64_t* grp_excl = nullptr;
   csaw::Chunk* chunks = nullptr;
   uint32_t chunk_cap = 0;
+  // counter block, then the requests' edge bounds (kCtrBytes + n_req *
+  // kBoundsBytes): one copy into h_state after a synchronised run brings the
+  // overflow flag and every request's place to the host
   uint32_t* counters = nullptr;
+  int64_t* bounds = nullptr;          // in the same allocation
+  std::vector<uint32_t> h_state;
+  bool bounds_known = false;          // h_state is of the last run
   uint32_t* queues = nullptr;
   int64_t queue_cap = 0;
   int64_t* totals = nullptr;
@@ -100,6 +109,7 @@ struct csaw_plan {
   hipEvent_t fork = nullptr;
   hipEvent_t join[kSide] = {};
   csaw::EventTimer timer;
+  hipEvent_t begin = nullptr, end = nullptr;  // of a synchronised run
   double last_ms = 0.0;
   int64_t runs = 0;
   std::vector<csaw::HopLog> hop_logs;

@@ -231,14 +231,71 @@ __global__ __launch_bounds__(256) void k_scan_groups(HopDev H, int64_t* __restri
   if (tid == 0) *total = (int64_t)carry;
 }
 
-// per-sample edge offsets for samples [0, gb] of this hop
-__global__ void k_offsets(HopDev H, const int64_t* __restrict__ total) {
+// per-sample edge offsets for samples [0, gb] of this hop, and the bounds of
+// the requests active in it (the offsets at their first and past their last
+// sample)
+__global__ void k_offsets(HopDev H, const ReqDev* __restrict__ R, const int64_t* __restrict__ total) {
   const int64_t n = *H.n_ptr;
-  for (int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; g <= H.gb; g += (int64_t)gridDim.x * blockDim.x) {
+  auto offset = [&](int64_t g) -> int64_t {
     const int64_t x = H.fo[g];
-    H.eo[g] = x >= n ? *total
-                     : (int64_t)H.grp_excl[x >> kGroupShift] + H.blk_excl[x >> kBlockShift] + H.local_excl[x];
+    return x >= n ? *total
+                  : (int64_t)H.grp_excl[x >> kGroupShift] + H.blk_excl[x >> kBlockShift] + H.local_excl[x];
+  };
+  const int64_t t0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t g = t0; g <= H.gb; g += step) H.eo[g] = offset(g);
+  if (!H.bounds) return;
+  for (int64_t i = t0; i < 2 * (int64_t)H.n_req; i += step) {
+    const ReqDev& r = R[i >> 1];
+    if (r.depth > H.hop)
+      H.bounds[((int64_t)r.slot * CSAW_MAX_HOPS + H.hop) * 2 + (i & 1)] = offset(r.gbase + (i & 1 ? r.samples : 0));
   }
+}
+
+// ---------------------------------------------------------------- copy-out
+// One request's edges out of its hops' arrays, in one launch: blockIdx.y is a
+// (hop, column) pair, column 3 the per-sample offsets.  Stores are 16-byte
+// aligned (the first elements up to the boundary go one by one); the loads
+// follow the request's own alignment, which dword-aligned 16-byte loads allow.
+// Bound: HBM for a large request, the launch for a small one (a request of two
+// hops took six copies, two adds and a subtraction, each its own launch).
+struct __attribute__((packed, aligned(4))) Quad {
+  int32_t v[4];
+};
+__global__ __launch_bounds__(256) void k_copy_edges(CopyArgs A) {
+  const int h = blockIdx.y >> 2, col = blockIdx.y & 3;
+  const int64_t t0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+  if (col == 3) {
+    if (!A.hop_offsets) return;
+    const int64_t* __restrict__ in = A.eo[h];
+    int64_t* __restrict__ out = A.hop_offsets + h * A.rows;
+    const int64_t add = A.at[h] - A.lo[h];
+    for (int64_t i = t0; i < A.rows; i += step) out[i] = in[i] + add;
+    return;
+  }
+  int32_t* __restrict__ out = A.out[col];
+  if (!out) return;
+  out += A.at[h];
+  const int32_t* __restrict__ in = A.col[col][h] + A.lo[h];
+  const int32_t sub = col == 2 ? A.sub : 0;
+  const int64_t n = A.n[h];
+  const int64_t head = min(n, (int64_t)((16 - ((uintptr_t)out & 15)) & 15) >> 2);
+  const int64_t quads = (n - head) >> 2, tail = head + 4 * quads;
+  if (t0 < head) out[t0] = in[t0] - sub;
+  for (int64_t i = t0; i < quads; i += step) {
+    const Quad q = *reinterpret_cast<const Quad*>(in + head + 4 * i);
+    *reinterpret_cast<int4*>(out + head + 4 * i) = make_int4(q.v[0] - sub, q.v[1] - sub, q.v[2] - sub, q.v[3] - sub);
+  }
+  if (t0 < n - tail) out[tail + t0] = in[tail + t0] - sub;
+}
+
+int launch_copy_edges(hipStream_t st, const CopyArgs& A) {
+  if (A.depth <= 0) return CSAW_OK;
+  int64_t most = A.hop_offsets ? A.rows : 0;
+  for (int h = 0; h < A.depth; ++h) most = std::max(most, (A.n[h] + 3) / 4);
+  const int grid = (int)std::max<int64_t>(1, std::min<int64_t>((most + 1023) / 1024, 4096));
+  k_copy_edges<<<dim3(grid, 4 * A.depth), 256, 0, st>>>(A);
+  CSAW_LAUNCH_CHECK();
+  return CSAW_OK;
 }
 
 // ------------------------------------------------------------ digest
@@ -766,7 +823,7 @@ int launch_bin_list(const LaunchCfg& L, const GraphDev& G, const ReqDev* R, cons
   return CSAW_OK;
 }
 
-int launch_scans(const LaunchCfg& L, const HopDev& H, int64_t* total, int64_t max_entries) {
+int launch_scans(const LaunchCfg& L, const HopDev& H, const ReqDev* R, int64_t* total, int64_t max_entries) {
   int64_t nb = (max_entries + kBlockEntries - 1) / kBlockEntries;
   int64_t ng = (nb + 1023) / 1024;
   int grid = (int)std::max<int64_t>(1, std::min<int64_t>(ng, grid_of(L, 4)));
@@ -774,9 +831,9 @@ int launch_scans(const LaunchCfg& L, const HopDev& H, int64_t* total, int64_t ma
   CSAW_LAUNCH_CHECK();
   k_scan_groups<<<1, 256, 0, L.stream>>>(H, total);
   CSAW_LAUNCH_CHECK();
-  int64_t gs = H.gb + 1;
+  int64_t gs = std::max<int64_t>(H.gb + 1, H.bounds ? 2 * (int64_t)H.n_req : 0);
   int g2 = (int)std::max<int64_t>(1, std::min<int64_t>((gs + 255) / 256, grid_of(L, 8)));
-  k_offsets<<<g2, 256, 0, L.stream>>>(H, total);
+  k_offsets<<<g2, 256, 0, L.stream>>>(H, R, total);
   CSAW_LAUNCH_CHECK();
   return CSAW_OK;
 }

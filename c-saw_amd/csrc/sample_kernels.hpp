@@ -88,7 +88,22 @@ int launch_count(const LaunchCfg& L, const GraphDev& G, const ReqDev* R, const i
 // Bins the n entries list[0 .. n) into chunks (H.order by list position).
 int launch_bin_list(const LaunchCfg& L, const GraphDev& G, const ReqDev* R, const int32_t* gs2req, const HopDev& H,
                     const int32_t* list, int64_t n);
-int launch_scans(const LaunchCfg& L, const HopDev& H, int64_t* total, int64_t max_entries);
+int launch_scans(const LaunchCfg& L, const HopDev& H, const ReqDev* R, int64_t* total, int64_t max_entries);
+// One request's hops (k_copy_edges): hop h's edges are [lo[h], lo[h] + n[h])
+// of its columns col[0 .. 2][h] (src, dst, sample) and go to out[c] + at[h];
+// eo[h] are its rows = samples + 1 offsets, written to hop_offsets[h * rows ..]
+// relative to the request's first edge; sub is taken off the sample ids.
+// out[c] and hop_offsets may be null.
+struct CopyArgs {
+  const int32_t* col[3][CSAW_MAX_HOPS];
+  const int64_t* eo[CSAW_MAX_HOPS];
+  int64_t lo[CSAW_MAX_HOPS], n[CSAW_MAX_HOPS], at[CSAW_MAX_HOPS];
+  int32_t* out[3];
+  int64_t* hop_offsets;
+  int64_t rows;
+  int32_t depth, sub;
+};
+int launch_copy_edges(hipStream_t st, const CopyArgs& A);
 int launch_fill(const LaunchCfg& L, uint32_t* p, uint32_t v, int64_t n);
 int launch_digest(hipStream_t st, int num_cu, const int32_t* src, const int32_t* dst, const int32_t* smp, int64_t lo,
                   int64_t hi, int64_t pos0, int64_t gbase, unsigned long long* out);

@@ -685,7 +685,7 @@ extern "C" int csaw_stream_sample_opts(csaw_host_graph* hg, const csaw_request* 
         H.group_min = L.group_min;
       }
       CSAW_TRY(launch_count(L, G, d_req, d_gs2req, H, false, nmax[h]));
-      CSAW_TRY(launch_scans(L, H, d_tot + h, nmax[h]));
+      CSAW_TRY(launch_scans(L, H, d_req, d_tot + h, nmax[h]));
       // bin the frontier by partition
       CSAW_TRY(launch_fill(L, d_cnt, 0u, 3 * P));
       CSAW_TRY(launch_fill(L, reinterpret_cast<uint32_t*>(d_pbytes), 0u, 2 * P));

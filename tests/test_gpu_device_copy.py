@@ -55,3 +55,40 @@ def test_plan_copy_device(C):
                 for b in bufs:
                     hip.L.hipFree(b)
         p.close()
+
+
+@pytest.mark.parametrize("shift", [0, 1, 2, 3])
+@pytest.mark.parametrize("sync", [True, False])
+def test_plan_copy_device_alignments(C, shift, sync):
+    """Requests of 1 to 13 samples packed one after another from `shift`
+    elements into the buffers: every alignment of source and destination, heads
+    and tails shorter than four elements, a request without edges, and the
+    bounds of a run that was not waited for by the call itself."""
+    hip = Hip()
+    g = C.Graph.rmat(10, 4)
+    off, adj = g.csr()
+    deg = np.diff(off)
+    specs = [{"seeds": g.seeds(n, request=n), "fanouts": [3, 2], "bias": n % 2, "dedup": n % 2, "request": n}
+             for n in range(1, 14)]
+    specs.append({"seeds": np.nonzero(deg == 0)[0][:5].astype(np.int32), "fanouts": [2, 2], "bias": 0, "request": 20})
+    p = C.Plan(g, specs, mode=C.MODE_BATCHED, use_graph=True, cdf_cache=True)
+    p.run(sync=sync)
+    if not sync:
+        assert hip.L.hipDeviceSynchronize() == 0
+    want = [p.result(r) for r in range(len(specs))]
+    total = sum(len(w["src"]) for w in want) + shift
+    bufs = [hip.alloc(4 * (total + 4)) for _ in range(3)]
+    try:
+        at = shift
+        for r in range(len(specs)):
+            st = C.lib().csaw_plan_copy_device(p.h, r, bufs[0].value + 4 * at, bufs[1].value + 4 * at,
+                                               bufs[2].value + 4 * at, None, None, 1)
+            assert st == 0, C.last_error()
+            at += len(want[r]["src"])
+        for buf, k in zip(bufs, ("src", "dst", "smp")):
+            got = hip.to_host(buf, at, np.int32)[shift:]
+            assert np.array_equal(got, np.concatenate([w[k] for w in want])), k
+    finally:
+        for b in bufs:
+            hip.L.hipFree(b)
+    p.close()
