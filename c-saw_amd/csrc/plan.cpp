@@ -340,11 +340,10 @@ static int run_unit(csaw_plan* p, Unit& u, hipStream_t st, TimingHook* th) {
             remap |= r.dedup == 2;
           }
         }
-        // region-remap requests resolve their slots with whole waves (gs = 0)
-        const int gs = remap ? 0 : group_size_for(fmax, L.group_min);
+        const int gs = group_size_for(fmax, L.group_min);
         H.only_kind = nk > 1 ? 1 + kind : 0;
         if (th) th->begin(kKernPlain, st);
-        CSAW_TRY(launch_expand_plain(L, kind, G, hv, u.d_req, u.d_gs2req, H, u.nmax[h], gs));
+        CSAW_TRY(launch_expand_plain(L, kind, G, hv, u.d_req, u.d_gs2req, H, u.nmax[h], gs, remap));
         if (th) th->end(kKernPlain, st);
       }
     }

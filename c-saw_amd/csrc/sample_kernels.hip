@@ -345,13 +345,17 @@ __global__ void k_fill_u32(uint32_t* __restrict__ p, uint32_t v, int64_t n) {
 // the CDF cache and its 16-ary index (searched through the index).  KEYS:
 // kKeys32 when no integer cache of the view is 64-bit (the 64-bit searches
 // compiled out of the group path).
-template <int KIND, bool IDX, int KEYS>
+// REMAP: the hop's requests of this kind use the region-remap mode.
+template <int KIND, bool IDX, int KEYS, bool REMAP = false>
 __global__ __launch_bounds__(256) void k_expand_plain(GraphDev G, csaw_graph_view hv, const ReqDev* __restrict__ R,
                                                       const int32_t* __restrict__ gs2req, HopDev H, int gs) {
-  constexpr bool kGroupOk = KIND != kInt || IDX;            // no per-entry CDF build needed
+  constexpr bool kGroupOk = KIND != kInt || IDX;  // no per-entry CDF build needed
   constexpr bool kGroupLds = KIND == kF32 || (KIND == kInt && IDX);  // small cached CDFs staged in LDS
-  __shared__ uint64_t cdf[KIND == kInt ? 4 * kWaveIntCap : 1];
-  __shared__ uint32_t bms[4 * (kWaveBitmapCap / 32)];
+  // (a region-remap build always has a group size: the whole-wave path and its
+  // 40 KB of LDS per workgroup are left out)
+  constexpr bool kGroupOnly = kGroupOk && KEYS == kKeys32 && REMAP;
+  __shared__ uint64_t cdf[KIND == kInt && !kGroupOnly ? 4 * kWaveIntCap : 1];
+  __shared__ uint32_t bms[kGroupOnly ? 1 : 4 * (kWaveBitmapCap / 32)];
   __shared__ uint32_t glds[kGroupLds ? 4 * kGroupLdsWords : 1];
   const int64_t n = *H.n_ptr;
   const int wid = threadIdx.x / kWave;
@@ -359,7 +363,7 @@ __global__ __launch_bounds__(256) void k_expand_plain(GraphDev G, csaw_graph_vie
   // batch size adapts to the frontier: one entry (one group round) per wave
   // when it is small (all waves busy), up to 64 entries per metadata round
   // when it is large
-  const bool grp = kGroupOk && gs > 0;
+  const bool grp = kGroupOnly || (kGroupOk && gs > 0);
   const int64_t per = grp ? kWave / gs : 1;
   const int64_t bs = min((int64_t)kWave, max(per, (n + nw - 1) / nw));
   uint32_t* gl = kGroupLds ? glds + wid * kGroupLdsWords : nullptr;
@@ -367,12 +371,13 @@ __global__ __launch_bounds__(256) void k_expand_plain(GraphDev G, csaw_graph_vie
     const int cnt = (int)min(bs, n - e0);
     if constexpr (kGroupOk) {
       if (grp) {
-        group_expand_batch<KIND, KEYS>(G, hv, R, gs2req, H, nullptr, e0, cnt, gs, gl);
+        group_expand_batch<KIND, KEYS, REMAP>(G, hv, R, gs2req, H, nullptr, e0, cnt, gs, gl);
         continue;
       }
     }
-    wave_expand_batch<KIND, IDX>(G, hv, R, gs2req, H, nullptr, e0, cnt, KIND == kInt ? cdf + wid * kWaveIntCap : nullptr,
-                                 bms + wid * (kWaveBitmapCap / 32));
+    if constexpr (!kGroupOnly)
+      wave_expand_batch<KIND, IDX>(G, hv, R, gs2req, H, nullptr, e0, cnt,
+                                   KIND == kInt ? cdf + wid * kWaveIntCap : nullptr, bms + wid * (kWaveBitmapCap / 32));
   }
 }
 
@@ -677,15 +682,15 @@ __global__ __launch_bounds__(256) void k_expand_wave(GraphDev G, csaw_graph_view
   }
 }
 
-// Region-remap entries (dedup == 2, heur_normalize's collision policy): one
-// wave per entry, whole-wave selection (wave_select_remap); the integer CDF
-// is built in LDS (d <= kWaveIntCap) or read from the hub cache or the CDF
-// cache, the taken set is an LDS bitmap.
-template <int KIND>
+// Region-remap entries (dedup == 2, heur_normalize's collision policy).  G32
+// (CDF keys all 32-bit, none to build): sub-wave groups; else one wave per
+// entry, the integer CDF built in LDS (d <= kWaveIntCap) or read from the hub
+// cache or the 64-bit CDF cache.
+template <int KIND, bool G32>
 __global__ __launch_bounds__(256) void k_expand_remap(GraphDev G, csaw_graph_view hv, const ReqDev* __restrict__ R,
                                                       const int32_t* __restrict__ gs2req, HopDev H, ExpandArgs A) {
-  __shared__ uint64_t cdf[KIND == kInt ? 4 * kWaveIntCap : 1];
-  __shared__ uint32_t bms[4 * (kWaveBitmapCap / 32)];
+  __shared__ uint64_t cdf[KIND == kInt && !G32 ? 4 * kWaveIntCap : 1];
+  __shared__ uint32_t glds[G32 && KIND != kUniform ? 4 * kGroupLdsWords : 1];
   const int wid = threadIdx.x / kWave;
   WaveClaim wc;
   for (;;) {
@@ -693,9 +698,17 @@ __global__ __launch_bounds__(256) void k_expand_remap(GraphDev G, csaw_graph_vie
     if (!cc.valid) break;
     const uint64_t t0 = wall_clock64();
     const Chunk c = H.chunks[cc.ci];
-    for (int k0 = 0; k0 < c.len; k0 += kWave)
-      wave_expand_batch<KIND, true>(G, hv, R, gs2req, H, H.order, (int64_t)c.start + k0, min(kWave, (int)c.len - k0),
-                                    KIND == kInt ? cdf + wid * kWaveIntCap : nullptr, bms + wid * (kWaveBitmapCap / 32));
+    for (int k0 = 0; k0 < c.len; k0 += kWave) {
+      const int64_t first = (int64_t)c.start + k0;
+      const int cnt = min(kWave, (int)c.len - k0);
+      if constexpr (G32)
+        group_expand_batch<KIND, kKeys32, true>(G, hv, R, gs2req, H, H.order, first, cnt,
+                                                group_size_for(c.max_f, H.group_min),
+                                                KIND != kUniform ? glds + wid * kGroupLdsWords : nullptr);
+      else
+        wave_expand_batch<KIND, true>(G, hv, R, gs2req, H, H.order, first, cnt,
+                                      KIND == kInt ? cdf + wid * kWaveIntCap : nullptr, nullptr);
+    }
     log_chunk_wave(A, H, cc.ci, CSAW_VAR_WAVE_BITMAP, t0);
   }
 }
@@ -847,20 +860,30 @@ int launch_fill(const LaunchCfg& L, uint32_t* p, uint32_t v, int64_t n) {
 }
 
 int launch_expand_plain(const LaunchCfg& L, int kind, const GraphDev& G, const csaw_graph_view& hv, const ReqDev* R,
-                        const int32_t* gs2req, const HopDev& H, int64_t max_entries, int gs) {
+                        const int32_t* gs2req, const HopDev& H, int64_t max_entries, int gs, bool remap) {
   int64_t nwg = (max_entries + 3) / 4;
   int grid = (int)std::max<int64_t>(1, std::min<int64_t>(nwg, grid_of(L, L.expand_per_cu)));
   if (L.grid_override > 0) grid = L.grid_override;
   // the CDF cache (and its index) is in the view: plain sampling with cdf_cache
   const bool idx = G.cdf_idx || G.int_idx32[0] || G.int_idx32[1] || G.int_idx[0] || G.int_idx[1];
   const bool wide = G.int_cdf[0] || G.int_cdf[1];  // a 64-bit integer cache in the view
-  if (kind == kUniform) k_expand_plain<kUniform, false, kKeys32><<<grid, 256, 0, L.stream>>>(G, hv, R, gs2req, H, gs);
-  else if (kind == kInt && idx && !wide)
-    k_expand_plain<kInt, true, kKeys32><<<grid, 256, 0, L.stream>>>(G, hv, R, gs2req, H, gs);
-  else if (kind == kInt && idx) k_expand_plain<kInt, true, kKeysAny><<<grid, 256, 0, L.stream>>>(G, hv, R, gs2req, H, gs);
-  else if (kind == kInt) k_expand_plain<kInt, false, kKeysAny><<<grid, 256, 0, L.stream>>>(G, hv, R, gs2req, H, 0);
-  else if (idx) k_expand_plain<kF32, true, kKeys32><<<grid, 256, 0, L.stream>>>(G, hv, R, gs2req, H, gs);
-  else k_expand_plain<kF32, false, kKeys32><<<grid, 256, 0, L.stream>>>(G, hv, R, gs2req, H, gs);
+  auto go = [&](auto kern, int group) { kern<<<grid, 256, 0, L.stream>>>(G, hv, R, gs2req, H, group); };
+  if (kind == kUniform) {
+    if (remap) go(k_expand_plain<kUniform, false, kKeys32, true>, gs);
+    else go(k_expand_plain<kUniform, false, kKeys32>, gs);
+  } else if (kind == kInt) {
+    // (region remap over 64-bit keys or CDFs to build: whole waves, group 0)
+    if (idx && !wide && remap) go(k_expand_plain<kInt, true, kKeys32, true>, gs);
+    else if (idx && !wide) go(k_expand_plain<kInt, true, kKeys32>, gs);
+    else if (idx) go(k_expand_plain<kInt, true, kKeysAny>, remap ? 0 : gs);
+    else go(k_expand_plain<kInt, false, kKeysAny>, 0);
+  } else if (remap) {
+    if (idx) go(k_expand_plain<kF32, true, kKeys32, true>, gs);
+    else go(k_expand_plain<kF32, false, kKeys32, true>, gs);
+  } else {
+    if (idx) go(k_expand_plain<kF32, true, kKeys32>, gs);
+    else go(k_expand_plain<kF32, false, kKeys32>, gs);
+  }
   CSAW_LAUNCH_CHECK();
   return CSAW_OK;
 }
@@ -930,9 +953,12 @@ int launch_expand_chunks(const LaunchCfg& L, const GraphDev& G, const csaw_graph
   }
   CSAW_TRY(go(kKernCopy, k_expand_copy, L.expand_per_cu));
   if (A.remap) {
-    if (kinds_present[kUniform]) CSAW_TRY(go(kKernWave, k_expand_remap<kUniform>, L.expand_per_cu));
-    if (kinds_present[kInt]) CSAW_TRY(go(kKernWave, k_expand_remap<kInt>, L.expand_per_cu));
-    if (kinds_present[kF32]) CSAW_TRY(go(kKernWave, k_expand_remap<kF32>, L.expand_per_cu));
+    if (kinds_present[kUniform]) CSAW_TRY(go(kKernWave, k_expand_remap<kUniform, true>, L.expand_per_cu));
+    if (kinds_present[kInt]) {
+      if (g32) CSAW_TRY(go(kKernWave, k_expand_remap<kInt, true>, L.expand_per_cu));
+      else CSAW_TRY(go(kKernWave, k_expand_remap<kInt, false>, L.expand_per_cu));
+    }
+    if (kinds_present[kF32]) CSAW_TRY(go(kKernWave, k_expand_remap<kF32, true>, L.expand_per_cu));
   }
   return CSAW_OK;
 }

@@ -17,6 +17,7 @@
 #pragma once
 #include "cdf_index.hpp"
 #include "common.hpp"
+#include "remap.hpp"
 
 namespace csaw {
 
@@ -270,9 +271,106 @@ __device__ int32_t wave_select(int64_t E, const Entry& en, const Picker& pk, uin
 // each attempt draws r; on a collision with the picked interval [A, B) r is
 // remapped with the reference's float sequence (A = p_{i-1}, 0 for i = 0;
 // B = p_i) and picks again; after kReselect attempts the cyclic fallback.
-// Every lane runs the same sequence (the results agree across lanes); lane
-// j keeps slot j.  Taken set: the LDS bitmap, or the resolved lanes.
+// Attempt 0 of every slot is drawn at once, slot j on lane j: a slot whose draw
+// repeats no earlier slot's keeps it, and only the others run the sequence
+// above, in slot order (remap_resolve).
 // ---------------------------------------------------------------------------
+__device__ __forceinline__ int32_t shfl_abs(int32_t v, int src) { return __builtin_amdgcn_ds_bpermute(src << 2, v); }
+__device__ __forceinline__ uint32_t shfl_abs_u(uint32_t v, int src) { return (uint32_t)shfl_abs((int32_t)v, src); }
+__device__ __forceinline__ uint64_t shfl_abs_u64(uint64_t v, int src) {
+  return (uint64_t)shfl_abs_u((uint32_t)v, src) | ((uint64_t)shfl_abs_u((uint32_t)(v >> 32), src) << 32);
+}
+__device__ __forceinline__ float shfl_abs_f(float v, int src) { return __int_as_float(shfl_abs(__float_as_int(v), src)); }
+
+// Slots of one entry on the gs lanes from gbase (gmask; lane gl of them holds
+// slot gl, F <= gs), all of which follow the same path.  draw(j, a): the float
+// of slot j's attempt a; pick(r): the index r picks; p(i): the normalised CDF.
+// Returns the lane's index (-1 for gl >= F).
+// Bound: the latency of the longest sequences (degrees just above the fanout
+// with most of the weight on taken neighbours: a thousand attempts).  Only the
+// bounds chain from attempt to attempt, two divisions long; draws, picks and
+// their checks do not, so a batch of attempts runs them lane by lane around it.
+// 8,191 seeds of fanouts {10, 10} under degree bias on RMAT-22: 7.3 ms with a
+// wave per entry and every lane on the same attempt, 1.1 ms here.
+template <class Draw, class Pick, class Norm>
+__device__ __forceinline__ int32_t remap_resolve(int F, int32_t d, int gs, int gl, int gbase, uint64_t gmask,
+                                                 const Draw& draw, const Pick& pick, const Norm& p) {
+  const float r0 = gl < F ? draw(gl, 0) : 0.0f;
+  const int32_t cand = gl < F ? pick(r0) : -1;
+  bool dup = false;
+  for (int i = 0; i + 1 < F; ++i) dup |= (cand == shfl_abs(cand, gbase + i)) & (gl > i);
+  // pending: slots whose attempt 0 an earlier slot holds (a slot that leaves
+  // its draw for another index leaves it to the earlier holder, so only the
+  // index it moves to can make a later slot pending)
+  uint64_t pending = ballot(dup && gl < F) & gmask;
+  int32_t res = cand;
+  while (pending) {
+    const int jl = __builtin_ctzll(pending), jj = jl - gbase;
+    pending &= pending - 1ull;
+    auto taken = [&](int32_t c) -> bool {  // by slots 0 .. jj-1 (every lane of the group takes part)
+      bool hit = false;
+#pragma unroll 4
+      for (int m = 0; m < jj; ++m) hit |= c == shfl_abs(res, gbase + m);
+      return hit;
+    };
+    float lb = 0.0f, hb = 1.0f;
+    int32_t chosen = -1, last = 0;
+    // attempts a0 .. a0 + nb - 1, lane k on attempt a0 + k (attempt 0, whose
+    // draw is known to be taken, by itself: its second pick mostly decides)
+    for (int a0 = 0, nb = 1; chosen < 0 && a0 < kReselect; a0 += nb, nb = min(gs, kReselect - a0)) {
+      float r;
+      int32_t i;
+      uint64_t free = 0;  // attempts whose first pick is free
+      if (a0 == 0) {
+        r = shfl_abs_f(r0, jl);
+        i = shfl_abs(cand, jl);
+      } else {
+        r = gl < nb ? draw(jj, a0 + gl) : 0.0f;
+        i = gl < nb ? pick(r) : 0;
+        const bool tk = taken(i);
+        free = ballot(gl < nb && !tk) & gmask;
+      }
+      const int n = free ? __builtin_ctzll(free) - gbase : nb;  // attempts that remap
+      const float A = i > 0 ? p(i - 1) : 0.0f, B = p(i);
+      float q = 0.0f, my_lb = 0.0f, my_hb = 1.0f;
+      for (int k = 0; k < n; ++k) {
+        const float Ak = shfl_abs_f(A, gbase + k), Bk = shfl_abs_f(B, gbase + k), rk = shfl_abs_f(r, gbase + k);
+        const float lambda = __fdiv_rn(__fsub_rn(Ak, lb), __fsub_rn(__fadd_rn(__fsub_rn(Ak, lb), hb), Bk));
+        const float qk = __fdiv_rn(rk, lambda);
+        if (gl == k) {
+          q = qk;
+          my_lb = lb;
+          my_hb = hb;
+        }
+        if (qk < Ak) hb = Ak;
+        else lb = Bk;
+      }
+      // the second picks, in the bounds of before their own attempt
+      const float r2 = q < A ? q : __fadd_rn(q, __fdiv_rn(__fsub_rn(B, A), __fsub_rn(my_hb, my_lb)));
+      const int32_t i2 = gl < n ? pick(r2) : 0;
+      const bool tk2 = taken(i2);
+      const uint64_t free2 = ballot(gl < n && !tk2) & gmask;
+      if (free2) chosen = shfl_abs(i2, __builtin_ctzll(free2));
+      else if (free) chosen = shfl_abs(i, __builtin_ctzll(free));
+      else last = shfl_abs(i2, gbase + nb - 1);
+    }
+    if (chosen < 0) {
+      for (int q = 0; q < d; q += gs) {
+        const int32_t c = (int32_t)(((int64_t)last + 1 + q + gl) % d);
+        const bool tk = taken(c);
+        const uint64_t free = ballot(q + gl < d && !tk) & gmask;
+        if (free) {
+          chosen = shfl_abs(c, __builtin_ctzll(free));
+          break;
+        }
+      }
+    }
+    if (gl == jj) res = chosen;
+    pending |= ballot(gl > jj && gl < F && cand == chosen) & gmask;
+  }
+  return res;
+}
+
 __device__ __forceinline__ float remap_p(const Picker& pk, int32_t i) {
   switch (pk.mode) {
     case kPickUniform:
@@ -296,64 +394,10 @@ __device__ __forceinline__ int32_t remap_pick(const Picker& pk, float r) {
   return lo < pk.d ? lo : pk.d - 1;
 }
 
-__device__ int32_t wave_select_remap(const Entry& en, const Picker& pk, uint32_t* bm) {
-  const int lane = lane_id();
-  const int F = en.F;
-  const int32_t d = en.d;
-  int32_t res = -1;
-  if (bm) {
-    const int words = (d + 31) >> 5;
-    for (int i = lane; i < words; i += kWave) bm[i] = 0u;
-    wave_fence();
-  }
-  auto taken = [&](int32_t c, int jj) -> bool {
-    return bm ? ((bm[c >> 5] >> (c & 31)) & 1u) != 0u : ballot(res == c) != 0ull;
-  };
-  for (int jj = 0; jj < F; ++jj) {
-    float lb = 0.0f, hb = 1.0f;
-    int32_t i = 0, chosen = -1;
-    for (int a = 0; a < kReselect; ++a) {
-      float r = philox_u24(draw(en, jj, a));
-      i = remap_pick(pk, r);
-      if (!taken(i, jj)) {
-        chosen = i;
-        break;
-      }
-      const float A = i > 0 ? remap_p(pk, i - 1) : 0.0f;
-      const float B = remap_p(pk, i);
-      const float lambda = __fdiv_rn(__fsub_rn(A, lb), __fsub_rn(__fadd_rn(__fsub_rn(A, lb), hb), B));
-      const float delta = __fdiv_rn(__fsub_rn(B, A), __fsub_rn(hb, lb));
-      r = __fdiv_rn(r, lambda);
-      if (r < A) {
-        hb = A;
-      } else {
-        r = __fadd_rn(r, delta);
-        lb = B;
-      }
-      i = remap_pick(pk, r);
-      if (!taken(i, jj)) {
-        chosen = i;
-        break;
-      }
-    }
-    if (chosen < 0) {
-      for (int q = 0; q < d; q += kWave) {
-        const int32_t c = (int32_t)(((int64_t)i + 1 + q + lane) % d);
-        const bool fr = (q + lane < d) && !wave_taken_lane(c, res, jj, bm);
-        const uint64_t m = ballot(fr);
-        if (m) {
-          chosen = readlane(c, __builtin_ctzll(m));
-          break;
-        }
-      }
-    }
-    if (bm) {
-      if (lane == 0) bm[chosen >> 5] |= 1u << (chosen & 31);
-      wave_fence();
-    }
-    if (lane == jj) res = chosen;
-  }
-  return res;
+__device__ int32_t wave_select_remap(const Entry& en, const Picker& pk) {
+  return remap_resolve(
+      en.F, en.d, kWave, lane_id(), 0, ~0ull, [&](int j, int a) { return philox_u24(draw(en, j, a)); },
+      [&](float r) { return remap_pick(pk, r); }, [&](int32_t i) { return remap_p(pk, i); });
 }
 
 // Builds the integer CDF of entry en in LDS with one wave (d <= cap).
@@ -397,7 +441,7 @@ __device__ void expand_entry_wave(const GraphDev& G, const csaw_graph_view& hv, 
     pk.mode = pk.T > 0 ? kPickLds : kPickUniform;
   }
   uint32_t* tb = (bm && en.d <= kWaveBitmapCap) ? bm : nullptr;
-  const int32_t res = en.dedup == 2 ? wave_select_remap(en, pk, tb) : wave_select<IDX>(G.E, en, pk, tb);
+  const int32_t res = en.dedup == 2 ? wave_select_remap(en, pk) : wave_select<IDX>(G.E, en, pk, tb);
   if (lane_id() < en.F) write_edge(G, hv, H, en, en.pos + lane_id(), res);
 }
 
@@ -477,12 +521,6 @@ __device__ void wave_expand_batch(const GraphDev& G, const csaw_graph_view& hv, 
 // 64/GS entries in flight per wave instead of one.  Every shuffle reads lanes
 // of the shuffling group only, and all lanes of a group follow the same path.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ int32_t shfl_abs(int32_t v, int src) { return __builtin_amdgcn_ds_bpermute(src << 2, v); }
-__device__ __forceinline__ uint32_t shfl_abs_u(uint32_t v, int src) { return (uint32_t)shfl_abs((int32_t)v, src); }
-__device__ __forceinline__ uint64_t shfl_abs_u64(uint64_t v, int src) {
-  return (uint64_t)shfl_abs_u((uint32_t)v, src) | ((uint64_t)shfl_abs_u((uint32_t)(v >> 32), src) << 32);
-}
-
 // One frontier entry as the group path keeps it (16 dwords, so a batch of 64
 // costs 16 registers per lane, and one shuffle per dword to fetch).
 struct GEntry {
@@ -491,7 +529,7 @@ struct GEntry {
   int32_t F, g;
   int64_t pos;
   uint32_t c1, c2, c3, k0, k1;
-  uint32_t flags;  // bit 0 dedup, bit 1 user-bias cache, bits 4-7 PickMode
+  uint32_t flags;  // bit 0 dedup, bit 1 user-bias cache, bit 2 region remap, bits 4-7 PickMode
   uint64_t T;      // integer CDF total, or the FP32 total's bits
 };
 
@@ -529,7 +567,7 @@ __device__ __forceinline__ GEntry make_gentry(const GraphDev& G, const Entry& en
       }
     }
   }
-  ge.flags = (en.dedup ? 1u : 0u) | (ck << 1) | (mode << 4);
+  ge.flags = (en.dedup ? 1u : 0u) | (ck << 1) | (en.dedup == 2 ? 4u : 0u) | (mode << 4);
   return ge;
 }
 
@@ -615,10 +653,68 @@ __device__ __forceinline__ int32_t gpick_small(const GEntry& en, const uint32_t*
   }
 }
 
+// Region remap in a group (32-bit keys).  A CDF that fits the group's LDS slot
+// is normalised into it once, and picks search the quotients.  Otherwise the
+// draw's threshold key (remap_key) is searched in the CDF; draws whose key does
+// not settle and totals out of its range take the search over p_i.
+template <int KIND>
+__device__ __forceinline__ int32_t group_select_remap(const GraphDev& G, const GEntry& en, int gs, int gl, int gbase,
+                                                      uint64_t gmask, uint32_t* lc, bool small) {
+  const int32_t d = en.d;
+  const uint32_t mode = (en.flags >> 4) & 15u;
+  const bool user = (en.flags >> 1) & 1u;
+  const uint32_t T = (uint32_t)en.T;
+  const uint32_t* C = KIND == kF32 ? reinterpret_cast<const uint32_t*>(G.cdf) + en.o
+                                   : (KIND == kInt ? (user ? G.int_cdf32[1] : G.int_cdf32[0]) + en.o : nullptr);
+  auto norm = [&](uint32_t c) -> float {
+    if (KIND == kF32) return (float)((double)__uint_as_float(c) / (double)__uint_as_float(T));
+    return (float)((double)c / (double)T);
+  };
+  float* lp = reinterpret_cast<float*>(lc);
+  if (small) {
+    for (int i = gl; i < d; i += gs) lp[i] = norm(C[i]);
+    wave_fence();
+  }
+  auto p = [&](int32_t i) -> float {
+    if (KIND == kUniform || mode == kPickUniform) return (float)((double)(i + 1) / (double)d);
+    return small ? lp[i] : norm(C[i]);
+  };
+  auto pick = [&](float r) -> int32_t {
+    if (!(r < 1.0f)) return d - 1;  // p never exceeds 1 (and nothing exceeds NaN)
+    if (!(r >= 0.0f)) return 0;     // p_0 >= 0
+    r = __uint_as_float(__float_as_uint(r) & 0x7fffffffu);  // -0 as 0
+    if (KIND == kUniform || mode == kPickUniform) {
+      uint32_t key;
+      if (remap_key(r, (uint32_t)d, &key)) return (int32_t)key - 1;
+    } else if (small) {
+      return (int32_t)min(upper_bound_dev<float>(lp, d, r), (int64_t)d - 1);
+    } else if (KIND == kF32) {
+      float x;
+      if (remap_key(r, __uint_as_float(T), &x)) {
+        if (mode == kPickF32Idx) return cdf_index_search<float>(G.cdf, G.cdf_idx, G.E, en.o, d, x);
+        return (int32_t)upper_bound_dev<float>(G.cdf + en.o, d, x);
+      }
+    } else {
+      uint32_t key;
+      if (remap_key(r, T, &key))
+        return cdf_index_search<uint32_t>(user ? G.int_cdf32[1] : G.int_cdf32[0], user ? G.int_idx32[1] : G.int_idx32[0],
+                                          G.E, en.o, d, key - 1u);
+    }
+    int32_t lo = 0, hi = d;
+    while (lo < hi) {
+      const int32_t mid = (lo + hi) >> 1;
+      if (p(mid) > r) hi = mid; else lo = mid + 1;
+    }
+    return lo < d ? lo : d - 1;
+  };
+  return remap_resolve(
+      en.F, d, gs, gl, gbase, gmask, [&](int j, int a) { return philox_u24(gdraw(en, j, a)); }, pick, p);
+}
+
 // lc: the group's LDS slot of cap words (null: no small path)
 // gs: group size (4 .. 32, or 64), a run-time value so one build serves all;
 // the group is lanes gbase .. gbase + gs - 1 (gmask)
-template <int KIND, int KEYS>
+template <int KIND, int KEYS, bool REMAP>
 __device__ int32_t group_select(const GraphDev& G, const GEntry& en, int gs, int gl, int gbase, uint64_t gmask,
                                 uint32_t* lc, int cap, int32_t* cl) {
   const int F = en.F;
@@ -627,6 +723,8 @@ __device__ int32_t group_select(const GraphDev& G, const GEntry& en, int gs, int
   const uint32_t mode = (en.flags >> 4) & 15u;
   const bool small = KIND != kUniform && lc && d <= cap &&
                      (mode == kPickInt32Idx || mode == kPickF32 || mode == kPickF32Idx);
+  if constexpr (REMAP)
+    if (en.flags & 4u) return group_select_remap<KIND>(G, en, gs, gl, gbase, gmask, lc, small);
   if (small) {
     const uint32_t* C = KIND == kF32 ? reinterpret_cast<const uint32_t*>(G.cdf)
                                      : ((en.flags >> 1) & 1u ? G.int_cdf32[1] : G.int_cdf32[0]);
@@ -724,11 +822,13 @@ constexpr int kGroupLdsWords = (kWave / kGroupMin) * kGroupSmallCap;
 // lanes never select, so their slot pointer is never dereferenced)
 constexpr int kCandSlotWords = 128;
 
-template <int KIND, int KEYS = kKeysAny>
+// REMAP: entries of region-remap requests may be among them (32-bit keys only).
+template <int KIND, int KEYS = kKeysAny, bool REMAP = false>
 __device__ void group_expand_batch(const GraphDev& G, const csaw_graph_view& hv, const ReqDev* __restrict__ R,
                                    const int32_t* __restrict__ gs2req, const HopDev& H,
                                    const int32_t* __restrict__ order, int64_t first, int count, int gs,
                                    uint32_t* lds) {
+  static_assert(!REMAP || KEYS == kKeys32, "region remap in groups searches 32-bit keys");
   const int NG = kWave / gs;
   const int lane = lane_id();
   const int gi = lane / gs;  // group; gi == NG: the idle remainder lanes
@@ -817,7 +917,7 @@ __device__ void group_expand_batch(const GraphDev& G, const csaw_graph_view& hv,
     const GEntry en = shfl_gentry(mine, src);
     int32_t idx = -1;
     if (e < nsel) {
-      const int32_t res = group_select<KIND, KEYS>(G, en, gs, gl, gbase, gmask, lc, cap, gcl);
+      const int32_t res = group_select<KIND, KEYS, REMAP>(G, en, gs, gl, gbase, gmask, lc, cap, gcl);
       idx = gl < en.F ? res : -1;
     }
     if (have) {

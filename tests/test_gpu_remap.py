@@ -99,3 +99,33 @@ def test_remap_rejects_bad_dedup(C, g13):
     g, _ = g13
     with pytest.raises(C.CsawError):
         C.sample(g, g.seeds(4), [2], dedup=3)
+
+
+@pytest.mark.parametrize("fan", [1, 4, 5, 16, 17, 32, 33, 64])
+def test_remap_group_sizes(C, O, fan):
+    """Fanouts at the group sizes' edges (groups of 4 to 32 lanes, the whole
+    wave above), degrees from just over the fanout (collisions in every slot,
+    the fallback) past the LDS copies of small CDFs, zero weights in runs."""
+    rng = np.random.default_rng(fan)
+    degs = [fan + 1, fan + 2, 2 * fan + 1, 64, 65, 85, 86, 170, 171, 512, 513, 1024, 1025, 3000]
+    degs = [d for d in degs if d > fan]
+    V = 4000
+    lists = [np.sort(rng.choice(V, d, replace=False)) for d in degs]
+    lists += [np.sort(rng.choice(V, rng.integers(0, 6), replace=False)) for _ in range(V - len(degs))]
+    off = np.concatenate([[0], np.cumsum([len(x) for x in lists])]).astype(np.int64)
+    adj = np.concatenate(lists).astype(np.int32)
+    w = rng.random(len(adj)).astype(np.float32)
+    w[rng.random(len(adj)) < 0.4] = 0
+    g = C.Graph.from_csr(off, adj, w)
+    og = O.OracleGraph(off, adj, weights=w)
+    seeds = rng.integers(0, len(degs), 150).astype(np.int32)
+    for bias in (0, 1, 2):
+        want = O.sample(og, seeds, [fan, 2], bias=bias, dedup=2)
+        for mode in (C.MODE_PLAIN, C.MODE_BATCHED):
+            for cache in (False, True):
+                for sched in ((C.SCHED_HEURISTIC, C.SCHED_FORCED) if mode == C.MODE_BATCHED else (C.SCHED_HEURISTIC,)):
+                    p = C.Plan(g, [{"seeds": seeds, "fanouts": [fan, 2], "bias": bias, "dedup": 2, "request": 0}],
+                               mode=mode, cdf_cache=cache, sched=sched, variant=C.VAR_WAVE_HASH)
+                    p.run()
+                    same(p.result(0), want, f"bias {bias} mode {mode} cache {cache} sched {sched}")
+                    p.close()
