@@ -5,10 +5,12 @@
 // then a uniform neighbour nb of u = frontier[q] (draw (t, 1, ...)); a degree-0
 // pick consumes the step (main.cu:162-163); emit (u, nb); frontier[q] = nb.
 //
-// One wave per sample; frontier and its VertexBias values live in LDS, the
-// total T is kept incrementally and the slot search streams a wave scan over
-// the bias values (no stored CDF).  Unlike the reference (D11: only thread 0
-// of the grid commits), every sample is walked.
+// One wave per sample.  Every frontier slot keeps its vertex, offset, degree and
+// VertexBias (in lane q's registers for up to 64 slots, else in LDS), and the
+// wave keeps the running totals of the biases (of runs of slots when there are
+// more than 64), so a step finds its slot with a ballot and adds the change of
+// one bias to the totals after it.  Unlike the reference (D11: only thread 0 of
+// the grid commits), every sample is walked.
 #include <algorithm>
 #include <cstring>
 #include <mutex>
@@ -21,16 +23,52 @@ namespace csaw {
 
 constexpr int kMdrwMaxFs = 4096;
 
+// Where a sample's frontier is kept: in the wave's registers (up to 64 slots),
+// in LDS sized to it at the launch (20 bytes per slot, up to 64 KB), or in the
+// full static array.
+enum MdrwFrontier { kMdrwRegs = 0, kMdrwLds = 1, kMdrwLdsMax = 2 };
+constexpr int kMdrwSlotBytes = 20;
+constexpr int kMdrwDynFs = 65536 / kMdrwSlotBytes;
+
+struct MdrwSlot {
+  int64_t o;
+  int32_t v, d;
+  uint32_t w;
+};
+
+__device__ __forceinline__ MdrwSlot mdrw_slot(const GraphDev& G, const csaw_graph_view& hv, int32_t v) {
+  MdrwSlot x;
+  x.v = v;
+  x.o = G.off[v];
+  x.d = (int32_t)(G.off[v + 1] - x.o);
+  x.w = VertexBias(v, &hv);
+  return x;
+}
+
 // bad: null when the host has validated the seeds; otherwise a sample with
 // a seed outside [0, V) emits nothing and sets *bad (seeds read on the device).
+// Bound: two dependent memory round trips a step, the neighbour and then its
+// offset and bias (which are loaded together).  4,096 samples of 64 slots x 200
+// steps on RMAT-22: 0.205 ms; 1.25 ms with the degree, offset and bias of the
+// picked vertex loaded in turn, a scan of the biases and two Philox calls a step
+// (64 steps' draws are now one call each, a lane per step), and 32 KB of LDS per
+// wave whatever the frontier's size (5 waves per CU).
+template <int MODE>
 __global__ __launch_bounds__(64) void k_mdrw(GraphDev G, csaw_graph_view hv, uint32_t k0, uint32_t k1, uint32_t request,
                                             int32_t S, int32_t fs, int32_t depth, const int32_t* __restrict__ seeds,
                                             int32_t* __restrict__ src, int32_t* __restrict__ dst,
                                             int32_t* __restrict__ cnt, uint32_t* __restrict__ bad) {
-  __shared__ int32_t front[kMdrwMaxFs];
-  __shared__ uint32_t wts[kMdrwMaxFs];
+  extern __shared__ __align__(16) unsigned char dyn[];
+  __shared__ __align__(16) unsigned char fix[MODE == kMdrwLdsMax ? kMdrwMaxFs * kMdrwSlotBytes : 8];
+  unsigned char* base = MODE == kMdrwLdsMax ? fix : dyn;
+  int64_t* so = reinterpret_cast<int64_t*>(base);
+  int32_t* sv = reinterpret_cast<int32_t*>(so + fs);
+  int32_t* sd = sv + fs;
+  uint32_t* sw = reinterpret_cast<uint32_t*>(sd + fs);
   const int lane = lane_id();
   const uint32_t c3 = (kDomMdrw << 28) | request;
+  // lane l owns the slots [l * run, (l + 1) * run)
+  const int run = MODE == kMdrwRegs ? 1 : (fs + kWave - 1) / kWave;
   for (int32_t s = blockIdx.x; s < S; s += gridDim.x) {
     if (bad) {
       bool out = false;
@@ -46,57 +84,107 @@ __global__ __launch_bounds__(64) void k_mdrw(GraphDev G, csaw_graph_view hv, uin
         continue;
       }
     }
-    uint64_t T = 0;
-    for (int q0 = 0; q0 < fs; q0 += kWave) {
-      const int q = q0 + lane;
-      uint32_t w = 0;
-      if (q < fs) {
-        const int32_t v = seeds[(int64_t)s * fs + q];
-        front[q] = v;
-        w = VertexBias(v, &hv);
-        wts[q] = w;
+    MdrwSlot mine{0, 0, 0, 0u};
+    uint64_t tot = 0;  // the lane's run, then the runs up to and including it
+    if (MODE == kMdrwRegs) {
+      if (lane < fs) mine = mdrw_slot(G, hv, seeds[(int64_t)s * fs + lane]);
+      tot = mine.w;
+    } else {
+      for (int q = lane; q < fs; q += kWave) {
+        const MdrwSlot x = mdrw_slot(G, hv, seeds[(int64_t)s * fs + q]);
+        so[q] = x.o;
+        sv[q] = x.v;
+        sd[q] = x.d;
+        sw[q] = x.w;
       }
-      T += readlane_u64(wave_incl_scan_u64((uint64_t)w), kWave - 1);
+      wave_fence();
+      for (int q = lane * run; q < min(fs, (lane + 1) * run); ++q) tot += sw[q];
     }
-    wave_fence();
-    int32_t c = 0;
+    tot = wave_incl_scan_u64(tot);
+    int32_t c = 0, bu = 0, bn = 0;  // edges so far; lane c mod 64 holds edge c until 64 are written out
+    uint64_t ts = 0, tn = 0;        // targets of step t0 + lane: slot, neighbour
     for (int32_t t = 0; t < depth; ++t) {
-      const U4 o = philox4x32_10((uint32_t)t, 0u, (uint32_t)s, c3, k0, k1);
-      int32_t q = 0;
+      const int at = t & (kWave - 1);
+      if (at == 0) {
+        ts = philox_t64(philox4x32_10((uint32_t)(t + lane), 0u, (uint32_t)s, c3, k0, k1));
+        tn = philox_t64(philox4x32_10((uint32_t)(t + lane), 1u, (uint32_t)s, c3, k0, k1));
+      }
+      const uint64_t T = readlane_u64(tot, kWave - 1), target = readlane_u64(ts, at);
+      int l, q;  // the slot and its lane
       if (T == 0) {
-        q = (int32_t)mulhi64(philox_t64(o), (uint64_t)fs);
+        q = (int)mulhi64(target, (uint64_t)fs);
+        l = MODE == kMdrwRegs ? q : q / run;
       } else {
-        const uint64_t x = mulhi64(philox_t64(o), T);
-        uint64_t acc = 0;
-        for (int q0 = 0; q0 < fs; q0 += kWave) {
-          const int qi = q0 + lane;
-          const uint64_t w = qi < fs ? wts[qi] : 0u;
-          const uint64_t sc = wave_incl_scan_u64(w);
-          const uint64_t tot = readlane_u64(sc, kWave - 1);
-          if (acc + tot > x) {
-            q = q0 + __builtin_ctzll(ballot(acc + sc > x));
-            break;
-          }
-          acc += tot;
+        const uint64_t x = mulhi64(target, T);
+        l = __builtin_ctzll(ballot(tot > x));
+        q = l;
+        if (MODE != kMdrwRegs) {
+          const uint64_t before = l ? readlane_u64(tot, l - 1) : 0ull;
+          const int qi = l * run + lane;
+          const uint64_t sc = wave_incl_scan_u64(lane < run && qi < fs ? (uint64_t)sw[qi] : 0ull);
+          q = l * run + __builtin_ctzll(ballot(before + sc > x));
         }
       }
-      const int32_t u = front[q];
-      const int32_t d = G.deg[u];
-      if (d == 0) continue;
-      const U4 o2 = philox4x32_10((uint32_t)t, 1u, (uint32_t)s, c3, k0, k1);
-      const int32_t nb = G.adj[G.off[u] + (int64_t)mulhi64(philox_t64(o2), (uint64_t)d)];
-      if (lane == 0) {
-        src[(int64_t)s * depth + c] = u;
-        dst[(int64_t)s * depth + c] = nb;
-        front[q] = nb;
-        wts[q] = VertexBias(nb, &hv);
+      MdrwSlot u;
+      if (MODE == kMdrwRegs) {
+        u.v = readlane(mine.v, q);
+        u.d = readlane(mine.d, q);
+        u.o = (int64_t)readlane_u64((uint64_t)mine.o, q);
+        u.w = readlane_u(mine.w, q);
+      } else {
+        u.v = sv[q];
+        u.d = sd[q];
+        u.o = so[q];
+        u.w = sw[q];
       }
-      T = T - (uint64_t)VertexBias(u, &hv) + (uint64_t)VertexBias(nb, &hv);
+      if (u.d == 0) continue;
+      const int32_t nb = G.adj[u.o + (int64_t)mulhi64(readlane_u64(tn, at), (uint64_t)u.d)];
+      const MdrwSlot x = mdrw_slot(G, hv, nb);
+      if (lane == (c & (kWave - 1))) {
+        bu = u.v;
+        bn = nb;
+      }
       ++c;
-      wave_fence();
+      if ((c & (kWave - 1)) == 0) {
+        src[(int64_t)s * depth + c - kWave + lane] = bu;
+        dst[(int64_t)s * depth + c - kWave + lane] = bn;
+      }
+      if (MODE == kMdrwRegs) {
+        if (lane == q) mine = x;
+      } else {
+        if (lane == 0) {
+          so[q] = x.o;
+          sv[q] = x.v;
+          sd[q] = x.d;
+          sw[q] = x.w;
+        }
+        wave_fence();
+      }
+      if (lane >= l) tot += (uint64_t)x.w - (uint64_t)u.w;
+    }
+    const int32_t rest = c & (kWave - 1);
+    if (lane < rest) {
+      src[(int64_t)s * depth + c - rest + lane] = bu;
+      dst[(int64_t)s * depth + c - rest + lane] = bn;
     }
     if (lane == 0) cnt[s] = c;
+    if (MODE != kMdrwRegs) wave_fence();  // the next sample overwrites the slots
   }
+}
+
+// One wave per workgroup, as many as the frontier's LDS lets a CU hold (16).
+static int launch_mdrw(hipStream_t st, const csaw_graph* g, uint64_t seed, uint32_t request, int32_t samples, int32_t fs,
+                       int32_t depth, const int32_t* seeds, int32_t* src, int32_t* dst, int32_t* cnt, uint32_t* bad) {
+  const int grid = std::min<int>(samples, g->num_cu * 16);
+  auto go = [&](auto kern, size_t lds) {
+    kern<<<grid, 64, lds, st>>>(g->view(), g->hook_view(), (uint32_t)seed, (uint32_t)(seed >> 32), request, samples, fs,
+                                depth, seeds, src, dst, cnt, bad);
+  };
+  if (fs <= kWave) go(k_mdrw<kMdrwRegs>, 0);
+  else if (fs <= kMdrwDynFs) go(k_mdrw<kMdrwLds>, (size_t)fs * kMdrwSlotBytes);
+  else go(k_mdrw<kMdrwLdsMax>, 0);
+  CSAW_LAUNCH_CHECK();
+  return CSAW_OK;
 }
 
 // Per-sample edge offsets from the per-sample counts: one workgroup of 1024
@@ -217,10 +305,8 @@ extern "C" int csaw_mdrw(csaw_graph* g, uint64_t seed, uint32_t request_id, int3
     CSAW_HIP(hipEventCreate(&e1));
     CSAW_HIP(hipEventRecord(e0, g->stream));
     if (samples > 0) {
-      const int grid = std::min<int>(samples, g->num_cu * 16);
-      k_mdrw<<<grid, 64, 0, g->stream>>>(g->view(), g->hook_view(), (uint32_t)seed, (uint32_t)(seed >> 32), request_id,
-                                         samples, frontier_size, depth, d_seeds, d_src, d_dst, d_cnt, nullptr);
-      CSAW_LAUNCH_CHECK();
+      CSAW_TRY(launch_mdrw(g->stream, g, seed, request_id, samples, frontier_size, depth, d_seeds, d_src, d_dst, d_cnt,
+                           nullptr));
     }
     CSAW_HIP(hipEventRecord(e1, g->stream));
     CSAW_HIP(hipEventSynchronize(e1));
@@ -285,10 +371,7 @@ extern "C" int csaw_mdrw_noalloc(csaw_graph* g, uint64_t seed, uint32_t request_
   k_mdrw_clear<<<1, 64, 0, st>>>(bad);
   CSAW_LAUNCH_CHECK();
   if (samples > 0) {
-    const int grid = std::min<int>(samples, g->num_cu * 16);
-    k_mdrw<<<grid, 64, 0, st>>>(g->view(), g->hook_view(), (uint32_t)seed, (uint32_t)(seed >> 32), request_id, samples,
-                                frontier_size, depth, d_seeds, ssrc, sdst, cnt, bad);
-    CSAW_LAUNCH_CHECK();
+    CSAW_TRY(launch_mdrw(st, g, seed, request_id, samples, frontier_size, depth, d_seeds, ssrc, sdst, cnt, bad));
   }
   k_mdrw_offsets<<<1, 1024, 0, st>>>(cnt, samples, d_offsets);
   CSAW_LAUNCH_CHECK();

@@ -406,3 +406,20 @@ def test_limits_fanout_64_depth_8(C, O, g14, cdf_cache):
         {"seeds": g.seeds(30, request=4), "fanouts": [2, 64, 2], "bias": 3, "dedup": 1, "request": 4},
     ]
     _check_cache_plans(C, O, g, og, specs, "limits", cdf_cache=cdf_cache)
+
+
+@pytest.mark.parametrize("fs", [1, 2, 63, 64, 65, 129, 1000, 3276, 3277, 4096])
+def test_mdrw_frontier_sizes(C, O, g14, fs):
+    """Frontiers in registers (up to 64 slots), in LDS sized to them and in the
+    full array, with runs of slots that do not divide evenly; step counts around
+    the 64 steps drawn at once; frontiers whose biases are all zero."""
+    g, og, off, *_ = g14
+    for S, D in ((3, 63), (2, 64), (5, 65), (2, 131)):
+        seeds = g.seeds(S * fs, request=D)
+        zero = np.nonzero(np.diff(off) == 0)[0].astype(np.int32)
+        seeds[:fs] = np.resize(zero, fs)  # sample 0 starts from vertices without neighbours
+        if fs > 1:
+            seeds[fs - 1] = int(np.argmax(np.diff(off)))
+        so, do, oo = O.mdrw(og, seeds, S, fs, D, request=D)
+        src, dst, offs = C.mdrw(g, seeds, S, fs, D, request=D)
+        assert np.array_equal(offs, oo) and np.array_equal(src, so) and np.array_equal(dst, do), (S, D)
