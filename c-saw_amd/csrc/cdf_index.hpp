@@ -24,6 +24,8 @@
 #pragma once
 #include <string.h>
 
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace csaw {
@@ -78,6 +80,39 @@ __host__ __device__ __forceinline__ void load16(const T* __restrict__ p, T* v) {
   }
 }
 
+// Bit i: v[i] above the target x.  32-bit keys take three VALU instructions a
+// key (compare by a subtraction, shift the bit in) instead of a compare, two
+// range tests and their mask logic through VCC, which also waits two states
+// between writing and reading it.  FP32: bits of non-negative floats order as
+// integers, a negative key is below every target (targets are non-negative),
+// and every key counts as above a NaN target.  1,048,576 FP32 walks of 80 steps
+// on RMAT-22: 4.30 -> 4.13 ms; FP32 neighbour sampling 739 -> 677 us.
+template <typename T>
+__host__ __device__ __forceinline__ uint32_t above16(const T* v, T x) {
+  uint32_t m = 0;
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (std::is_same<T, uint32_t>::value) {
+#pragma unroll
+    for (int i = 15; i >= 0; --i) {
+      // min(max(v - x, 0), 1), written out: the compiler turns it back into a compare
+      uint32_t t;
+      asm("v_sub_u32_e64 %0, %1, %2 clamp\n\tv_min_u32_e32 %0, 1, %0" : "=&v"(t) : "v"(v[i]), "v"(x));
+      m = (m << 1) | t;
+    }
+    return m;
+  } else if constexpr (std::is_same<T, float>::value) {
+    const int32_t xb = x == x ? __float_as_int(x) : -1;
+#pragma unroll
+    for (int i = 15; i >= 0; --i)
+      m = __builtin_amdgcn_alignbit(m, (uint32_t)(xb - max(__float_as_int(v[i]), 0)), 31);
+    return m;
+  }
+#endif
+#pragma unroll
+  for (int i = 15; i >= 0; --i) m = (m << 1) | (uint32_t)!(v[i] <= x);
+  return m;
+}
+
 // #{c : end_c < o or (end_c <= last and v[c] <= x)}, end_c = ((16 b + c + 1) << sh) - 1.
 // end_c < o  <=>  c < (o >> sh) - 16 b, and end_c <= last  <=>  c < ((last + 1) >> sh) - 16 b.
 template <typename T>
@@ -85,10 +120,14 @@ __host__ __device__ __forceinline__ int count16(const T* v, int64_t b, int sh, i
   const int64_t lo64 = (o >> sh) - 16 * b, hi64 = ((last + 1) >> sh) - 16 * b;
   const int lo = (int)(lo64 < 0 ? 0 : (lo64 > 16 ? 16 : lo64));
   const int hi = (int)(hi64 < 0 ? 0 : (hi64 > 16 ? 16 : hi64));
-  int c = 0;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) c += (i < lo) | ((i < hi) & (v[i] <= x));
-  return c;
+  // the keys passed inside the range, then the ends before it
+  uint32_t m = ~above16(v, x);
+  m = (m & ((1u << hi) - 1u)) | ((1u << lo) - 1u);
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __popc(m);
+#else
+  return __builtin_popcount(m);
+#endif
 }
 
 // upper_bound over C[o .. o+d) through the index K of the array C (E entries).
