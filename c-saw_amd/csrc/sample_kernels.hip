@@ -346,17 +346,21 @@ __global__ void k_fill_u32(uint32_t* __restrict__ p, uint32_t v, int64_t n) {
 // kKeys32 when no integer cache of the view is 64-bit (the 64-bit searches
 // compiled out of the group path).
 // REMAP: the hop's requests of this kind use the region-remap mode.
+// The group-only builds are held to 128 registers, four waves per SIMD: their
+// waves wait for memory most of the time (FP32 {15, 10, 5} from 30,011 seeds:
+// 645 us at three waves, 565 us at four).
 template <int KIND, bool IDX, int KEYS, bool REMAP = false>
-__global__ __launch_bounds__(256) void k_expand_plain(GraphDev G, csaw_graph_view hv, const ReqDev* __restrict__ R,
+__global__ __launch_bounds__(256, KEYS == kKeys32 && !REMAP ? 4 : 1) void k_expand_plain(GraphDev G, csaw_graph_view hv, const ReqDev* __restrict__ R,
                                                       const int32_t* __restrict__ gs2req, HopDev H, int gs) {
   constexpr bool kGroupOk = KIND != kInt || IDX;  // no per-entry CDF build needed
   constexpr bool kGroupLds = KIND == kF32 || (KIND == kInt && IDX);  // small cached CDFs staged in LDS
-  // (a region-remap build always has a group size: the whole-wave path and its
-  // 40 KB of LDS per workgroup are left out)
-  constexpr bool kGroupOnly = kGroupOk && KEYS == kKeys32 && REMAP;
+  // (32-bit-key builds are always given a group size: the whole-wave path and
+  // its 40 KB of LDS per workgroup are left out)
+  constexpr bool kGroupOnly = kGroupOk && KEYS == kKeys32;
+  constexpr int kGroupStride = kGroupLds ? kGroupWords : kGroupBaseWords;
   __shared__ uint64_t cdf[KIND == kInt && !kGroupOnly ? 4 * kWaveIntCap : 1];
   __shared__ uint32_t bms[kGroupOnly ? 1 : 4 * (kWaveBitmapCap / 32)];
-  __shared__ uint32_t glds[kGroupLds ? 4 * kGroupLdsWords : 1];
+  __shared__ __align__(16) uint32_t glds[kGroupOk ? 4 * kGroupStride : 4];
   const int64_t n = *H.n_ptr;
   const int wid = threadIdx.x / kWave;
   const int64_t nw = (int64_t)gridDim.x * 4;
@@ -366,12 +370,12 @@ __global__ __launch_bounds__(256) void k_expand_plain(GraphDev G, csaw_graph_vie
   const bool grp = kGroupOnly || (kGroupOk && gs > 0);
   const int64_t per = grp ? kWave / gs : 1;
   const int64_t bs = min((int64_t)kWave, max(per, (n + nw - 1) / nw));
-  uint32_t* gl = kGroupLds ? glds + wid * kGroupLdsWords : nullptr;
   for (int64_t e0 = (blockIdx.x * 4 + wid) * bs; e0 < n; e0 += nw * bs) {
     const int cnt = (int)min(bs, n - e0);
     if constexpr (kGroupOk) {
       if (grp) {
-        group_expand_batch<KIND, KEYS, REMAP>(G, hv, R, gs2req, H, nullptr, e0, cnt, gs, gl);
+        group_expand_batch<KIND, KEYS, REMAP>(G, hv, R, gs2req, H, nullptr, e0, cnt, gs, glds + wid * kGroupStride,
+                                              kGroupLds);
         continue;
       }
     }
@@ -642,12 +646,15 @@ __global__ __launch_bounds__(256) void k_expand_thread(GraphDev G, csaw_graph_vi
 // groups (GS = 64 for fanouts above 32) and the whole-wave path, LDS CDF
 // builds and uint64 searches are compiled out.
 template <int KIND, bool BITMAP, bool G32>
-__global__ __launch_bounds__(256) void k_expand_wave(GraphDev G, csaw_graph_view hv, const ReqDev* __restrict__ R,
+__global__ __launch_bounds__(256, G32 ? 4 : 1) void k_expand_wave(GraphDev G, csaw_graph_view hv, const ReqDev* __restrict__ R,
                                                      const int32_t* __restrict__ gs2req, HopDev H, ExpandArgs A) {
-  __shared__ uint64_t cdf[!G32 && KIND == kInt ? 4 * kWaveIntCap : 1];
+  // a wave's scratch: the group path's (with small-degree CDF slots for the
+  // biased kinds), or in the generic integer kernel the CDF built for one entry
+  constexpr bool kSmall = KIND != kUniform;
+  constexpr int kWords = kSmall ? kGroupWords : kGroupBaseWords;
+  static_assert(G32 || KIND != kInt || 2 * kWaveIntCap <= kWords, "the built CDF fits the scratch");
+  __shared__ __align__(16) uint32_t scratch[4 * kWords];
   __shared__ uint32_t bms[!G32 && BITMAP ? 4 * (kWaveBitmapCap / 32) : 1];
-  // small-degree CDF slots (the generic integer kernel reuses its CDF region)
-  __shared__ uint32_t glds[KIND == kF32 || (G32 && KIND == kInt) ? 4 * kGroupLdsWords : 1];
   const int var = BITMAP ? CSAW_VAR_WAVE_BITMAP : CSAW_VAR_WAVE_HASH;
   const int q = var * 3 + KIND;
   const int wid = threadIdx.x / kWave;
@@ -655,9 +662,7 @@ __global__ __launch_bounds__(256) void k_expand_wave(GraphDev G, csaw_graph_view
   // chunks whose fanouts fit a sub-wave group (and need no CDF build) run
   // 64 / GS entries at a time
   const bool groups_ok = KIND != kInt || A.int_cache;
-  uint32_t* gl = nullptr;
-  if (KIND == kF32 || (G32 && KIND == kInt)) gl = glds + wid * kGroupLdsWords;
-  else if (KIND == kInt) gl = reinterpret_cast<uint32_t*>(cdf + wid * kWaveIntCap);
+  uint32_t* mine = scratch + wid * kWords;
   WaveClaim wc;
   for (;;) {
     const ChunkCursor cc = next_chunk_wave(A, q, wc);
@@ -669,12 +674,12 @@ __global__ __launch_bounds__(256) void k_expand_wave(GraphDev G, csaw_graph_view
       const int64_t first = (int64_t)c.start + k0;
       const int cnt = min(kWave, (int)c.len - k0);
       if constexpr (G32) {
-        group_expand_batch<KIND, kKeys32>(G, hv, R, gs2req, H, H.order, first, cnt, gs, gl);
+        group_expand_batch<KIND, kKeys32>(G, hv, R, gs2req, H, H.order, first, cnt, gs, mine, kSmall);
       } else {
-        if (groups_ok && gs < kWave) group_expand_batch<KIND>(G, hv, R, gs2req, H, H.order, first, cnt, gs, gl);
+        if (groups_ok && gs < kWave) group_expand_batch<KIND>(G, hv, R, gs2req, H, H.order, first, cnt, gs, mine, kSmall);
         else
           wave_expand_batch<KIND, true>(G, hv, R, gs2req, H, H.order, first, cnt,
-                                        KIND == kInt ? cdf + wid * kWaveIntCap : nullptr,
+                                        KIND == kInt ? reinterpret_cast<uint64_t*>(mine) : nullptr,
                                         BITMAP ? bms + wid * (kWaveBitmapCap / 32) : nullptr);
       }
     }
@@ -689,8 +694,9 @@ __global__ __launch_bounds__(256) void k_expand_wave(GraphDev G, csaw_graph_view
 template <int KIND, bool G32>
 __global__ __launch_bounds__(256) void k_expand_remap(GraphDev G, csaw_graph_view hv, const ReqDev* __restrict__ R,
                                                       const int32_t* __restrict__ gs2req, HopDev H, ExpandArgs A) {
+  constexpr int kWords = KIND != kUniform ? kGroupWords : kGroupBaseWords;
   __shared__ uint64_t cdf[KIND == kInt && !G32 ? 4 * kWaveIntCap : 1];
-  __shared__ uint32_t glds[G32 && KIND != kUniform ? 4 * kGroupLdsWords : 1];
+  __shared__ __align__(16) uint32_t glds[G32 ? 4 * kWords : 4];
   const int wid = threadIdx.x / kWave;
   WaveClaim wc;
   for (;;) {
@@ -703,8 +709,8 @@ __global__ __launch_bounds__(256) void k_expand_remap(GraphDev G, csaw_graph_vie
       const int cnt = min(kWave, (int)c.len - k0);
       if constexpr (G32)
         group_expand_batch<KIND, kKeys32, true>(G, hv, R, gs2req, H, H.order, first, cnt,
-                                                group_size_for(c.max_f, H.group_min),
-                                                KIND != kUniform ? glds + wid * kGroupLdsWords : nullptr);
+                                                group_size_for(c.max_f, H.group_min), glds + wid * kWords,
+                                                KIND != kUniform);
       else
         wave_expand_batch<KIND, true>(G, hv, R, gs2req, H, H.order, first, cnt,
                                       KIND == kInt ? cdf + wid * kWaveIntCap : nullptr, nullptr);
@@ -717,10 +723,13 @@ __global__ __launch_bounds__(256) void k_expand_remap(GraphDev G, csaw_graph_vie
 // entries in LDS), wave 0 resolves the slots.  G32: the group-only build (see
 // k_expand_wave), for views whose CDF keys are all 32-bit.
 template <int KIND, bool BITMAP, bool G32>
-__global__ __launch_bounds__(256) void k_expand_block(GraphDev G, csaw_graph_view hv, const ReqDev* __restrict__ R,
+__global__ __launch_bounds__(256, G32 ? 4 : 1) void k_expand_block(GraphDev G, csaw_graph_view hv, const ReqDev* __restrict__ R,
                                                       const int32_t* __restrict__ gs2req, HopDev H, ExpandArgs A) {
-  // (G32: only the four waves' small-CDF slots, 4 x kGroupLdsWords words)
-  __shared__ uint64_t cdf[KIND == kInt ? (G32 ? 2 * kGroupLdsWords : kBlockIntCap) : 1];
+  // the CDF built for one entry, or the four waves' group scratch
+  constexpr bool kSmall = KIND == kInt;
+  constexpr int kWords = kSmall ? kGroupWords : kGroupBaseWords;
+  static_assert(4 * kWords <= 2 * kBlockIntCap, "the group scratch fits the CDF's array");
+  __shared__ __align__(16) uint64_t cdf[KIND == kInt && !G32 ? kBlockIntCap : 2 * kWords];
   __shared__ uint32_t bms[BITMAP && !G32 ? kBlockBitmapCap / 32 : 1];
   __shared__ uint64_t wsum[4];
   __shared__ uint64_t carry;
@@ -732,7 +741,7 @@ __global__ __launch_bounds__(256) void k_expand_block(GraphDev G, csaw_graph_vie
   // workgroup to share: its four waves then split the chunk into 64-entry
   // batches expanded in sub-wave groups.
   const bool groups_ok = KIND != kInt || A.int_cache;
-  uint32_t* gl = KIND == kInt ? reinterpret_cast<uint32_t*>(cdf) + wid * kGroupLdsWords : nullptr;
+  uint32_t* mine = reinterpret_cast<uint32_t*>(cdf) + wid * kWords;
   for (;;) {
     const ChunkCursor cc = next_chunk(A, q, &slot);
     if (!cc.valid) break;
@@ -743,8 +752,8 @@ __global__ __launch_bounds__(256) void k_expand_block(GraphDev G, csaw_graph_vie
       for (int k0 = wid * kWave; k0 < c.len; k0 += 4 * kWave) {
         const int64_t first = (int64_t)c.start + k0;
         const int cnt = min(kWave, (int)c.len - k0);
-        if constexpr (G32) group_expand_batch<KIND, kKeys32>(G, hv, R, gs2req, H, H.order, first, cnt, gs, gl);
-        else group_expand_batch<KIND>(G, hv, R, gs2req, H, H.order, first, cnt, gs, gl);
+        if constexpr (G32) group_expand_batch<KIND, kKeys32>(G, hv, R, gs2req, H, H.order, first, cnt, gs, mine, kSmall);
+        else group_expand_batch<KIND>(G, hv, R, gs2req, H, H.order, first, cnt, gs, mine, kSmall);
       }
       __syncthreads();
       log_chunk(A, H, cc.ci, var, t0);
@@ -799,6 +808,7 @@ __global__ __launch_bounds__(256) void k_expand_block(GraphDev G, csaw_graph_vie
 // group copying neighbour i (coalesced reads and writes)
 __global__ __launch_bounds__(256) void k_expand_copy(GraphDev G, csaw_graph_view hv, const ReqDev* __restrict__ R,
                                                      const int32_t* __restrict__ gs2req, HopDev H, ExpandArgs A) {
+  __shared__ __align__(16) uint32_t scratch[4 * kGroupBaseWords];
   WaveClaim wc;
   for (;;) {
     const ChunkCursor cc = next_chunk_wave(A, kQueueCopy, wc);
@@ -807,7 +817,8 @@ __global__ __launch_bounds__(256) void k_expand_copy(GraphDev G, csaw_graph_view
     const int gs = group_size_for(c.max_f, H.group_min);
     for (int k0 = 0; k0 < c.len; k0 += kWave)
       group_expand_batch<kUniform, kKeys32>(G, hv, R, gs2req, H, H.order, (int64_t)c.start + k0,
-                                            min(kWave, (int)c.len - k0), gs, nullptr);
+                                            min(kWave, (int)c.len - k0), gs,
+                                            scratch + (threadIdx.x / kWave) * kGroupBaseWords, false);
   }
 }
 

@@ -601,37 +601,167 @@ __device__ __forceinline__ int32_t gpick(const GraphDev& G, const GEntry& en, co
   return (int32_t)upper_bound_dev<uint64_t>(C + en.o, en.d, x);
 }
 
-__device__ __forceinline__ GEntry shfl_gentry(const GEntry& m, int src) {
+// A batch's selecting entries wait in LDS, 64 bytes each: the lanes of a group
+// read theirs with four broadcast ds_read_b128 instead of holding a lane's own
+// entry in 17 registers and fetching one with 17 shuffles a round.
+__device__ __forceinline__ void store_gentry(int4* p, const GEntry& e) {
+  p[0] = make_int4(e.v, e.g, (int)(uint32_t)e.o, (int)(uint32_t)((uint64_t)e.o >> 32));
+  p[1] = make_int4(e.d, e.F, (int)(uint32_t)e.pos, (int)(uint32_t)((uint64_t)e.pos >> 32));
+  p[2] = make_int4((int)e.c1, (int)e.c2, (int)e.c3, (int)e.flags);
+  p[3] = make_int4((int)e.k0, (int)e.k1, (int)(uint32_t)e.T, (int)(uint32_t)(e.T >> 32));
+}
+__device__ __forceinline__ int64_t pack_i64(int lo, int hi) {
+  return (int64_t)((uint64_t)(uint32_t)lo | ((uint64_t)(uint32_t)hi << 32));
+}
+__device__ __forceinline__ GEntry fetch_gentry(const int4* p) {
+  const int4 a = p[0], b = p[1], c = p[2], t = p[3];
   GEntry e;
-  e.v = shfl_abs(m.v, src);
-  e.d = shfl_abs(m.d, src);
-  e.o = (int64_t)shfl_abs_u64((uint64_t)m.o, src);
-  e.F = shfl_abs(m.F, src);
-  e.g = shfl_abs(m.g, src);
-  e.pos = (int64_t)shfl_abs_u64((uint64_t)m.pos, src);
-  e.c1 = shfl_abs_u(m.c1, src);
-  e.c2 = shfl_abs_u(m.c2, src);
-  e.c3 = shfl_abs_u(m.c3, src);
-  e.k0 = shfl_abs_u(m.k0, src);
-  e.k1 = shfl_abs_u(m.k1, src);
-  e.flags = shfl_abs_u(m.flags, src);
-  e.T = shfl_abs_u64(m.T, src);
+  e.v = a.x;
+  e.g = a.y;
+  e.o = pack_i64(a.z, a.w);
+  e.d = b.x;
+  e.F = b.y;
+  e.pos = pack_i64(b.z, b.w);
+  e.c1 = (uint32_t)c.x;
+  e.c2 = (uint32_t)c.y;
+  e.c3 = (uint32_t)c.z;
+  e.flags = (uint32_t)c.w;
+  e.k0 = (uint32_t)t.x;
+  e.k1 = (uint32_t)t.y;
+  e.T = (uint64_t)pack_i64(t.z, t.w);
   return e;
 }
 
-__device__ __forceinline__ void gwrite_edge(const GraphDev& G, const csaw_graph_view& hv, const HopDev& H,
-                                            const GEntry& en, int64_t p, int32_t idx) {
-  H.src[p] = en.v;
-  H.dst[p] = Update(&hv, G.adj[en.o + idx], en.v);
-  H.smp[p] = en.g;
-}
-
-// ci equal to one of the group's resolved slots 0 .. jj-1 (res of lane gbase+m)
-__device__ __forceinline__ bool group_taken(int32_t ci, int32_t res, int jj, int gbase) {
-  bool hit = false;
-#pragma unroll 8
-  for (int m = 0; m < jj; ++m) hit |= (ci == shfl_abs(res, gbase + m));
-  return hit;
+// Ordered resolution of one entry's slots on the gs lanes from gbase (gmask;
+// lane gl of them holds slot gl, F <= gs), which all follow the same path: slot
+// j keeps its attempt-0 draw `cand` unless an earlier slot's final index equals
+// it, and else takes its first later attempt that none of them equals (after
+// kReselect attempts the first free index scanning upward from the last draw).
+// cl, bits: 16-byte-aligned LDS words of the group, F rounded up to four of them
+// and four.
+// pick(j, a, valid): slot j's attempt a; lanes with valid == false take part.
+// spec: attempts a slot draws at first (the group's size where draws cost no
+// memory reads).
+//
+// A slot whose draw repeats no earlier draw is final at once.  A pending slot's
+// draw is held by an earlier slot whatever that one's own fate (a slot only
+// leaves an index that an earlier one keeps), so the indexes of cl can be
+// compared with as they stand, and only the index a slot moves to can make a
+// later one pending.  All pending slots draw together, gs / P attempts each, so
+// an entry's redraws cost one round of searches rather than one per collision;
+// a slot that finds nothing free in its share gets every lane for itself.
+// Bound: the latency of those searches and of the group's LDS round trips.
+// Searches that read memory draw kSpecDraws attempts at first: most slots need
+// one, and every further one costs its reads (53e9 random ones a second are the
+// card's limit).  FP32 fanouts {15, 10, 5} from 30,011 seeds on RMAT-22: 717 us
+// for the hops with every slot after the first collision stepped through and one
+// collision redrawn at a time, 645 us here, 565 us with the batch's entries in
+// LDS and registers for four waves per SIMD (128) instead of three.
+constexpr int kSpecDraws = 3;
+constexpr int kTakenMaskCap = 128;  // degrees whose taken set fits four words
+template <class Pick>
+__device__ __forceinline__ int32_t resolve_slots(int F, int32_t d, int gs, int gl, int gbase, uint64_t gmask, int32_t* cl,
+                                                 uint32_t* bits, int32_t cand, int spec, const Pick& pick) {
+  const bool act = gl < F;
+  // duplicate check: the group's draws read back four at a time (one broadcast
+  // ds_read_b128 per four slots)
+  cl[gl] = cand;
+  wave_fence();
+  auto held = [&](int32_t c, int before) -> bool {  // c among the slots 0 .. before-1
+    bool hit = false;
+#pragma unroll 2
+    for (int i0 = 0; i0 < before; i0 += 4) {
+      const int4 q = *reinterpret_cast<const int4*>(cl + i0);
+      hit |= (c == q.x) | (before > i0 + 1 && c == q.y) | (before > i0 + 2 && c == q.z) | (before > i0 + 3 && c == q.w);
+    }
+    return hit;
+  };
+  const bool dup = held(cand, act ? gl : 0);
+  uint64_t pending = ballot(dup) & gmask;
+  int32_t res = cand;
+  auto settle = [&](int at, int32_t c) -> uint64_t {  // slot `at` takes c; the slots this makes pending
+    if (gl == at) {
+      res = c;
+      cl[gl] = c;
+    }
+    return ballot(act && gl > at && cand == c) & gmask & ~pending;
+  };
+  while (pending) {
+    // lane gl draws attempt 1 + k for the p-th pending slot
+    const int np = __popcll(pending);
+    const int share = np == 1 ? gs : gs / np, m = min(share, spec);
+    const int p = np == 1 ? 0 : gl / share, k = gl - p * share;
+    int jj;
+    if (np == 1) {
+      jj = __builtin_ctzll(pending) - gbase;
+    } else {
+      // the pending slots' numbers to the lanes of their ranks (the others'
+      // beyond them, so that every lane has a destination of its own)
+      const bool mine = (pending >> (gbase + gl)) & 1ull;
+      const int rank = __popcll(pending & ((1ull << (gbase + gl)) - 1ull));
+      const int list = __builtin_amdgcn_ds_permute((gbase + (mine ? rank : np + gl - rank)) << 2, gl);
+      jj = shfl_abs(list, gbase + min(p, np - 1));
+    }
+    int32_t ci = pick(jj, 1 + k, p < np && k < m);
+    bool free = p < np && k < m && !held(ci, jj);
+    bool none = false;  // the first slot left found nothing free in its m attempts
+    for (int t = 0; t < np; ++t) {
+      const uint64_t fm = ballot(free && p == t) & gmask;
+      if (fm == 0ull) {
+        none = true;
+        break;
+      }
+      const int32_t c = shfl_abs(ci, __builtin_ctzll(fm));
+      const int at = __builtin_ctzll(pending) - gbase;
+      pending &= pending - 1ull;
+      free &= ci != c;
+      const uint64_t moved = settle(at, c);
+      pending |= moved;
+      if (moved) break;  // a new pending slot may come before the next of this round
+    }
+    wave_fence();
+    if (!none) continue;
+    // every lane for this slot, from its attempt m + 1 on; up to kTakenMaskCap
+    // neighbours the earlier slots' indexes are gathered into a mask first
+    const int at = __builtin_ctzll(pending) - gbase;
+    pending &= pending - 1ull;
+    const bool masked = d <= kTakenMaskCap;
+    uint64_t lo = 0, hi = 0;
+    if (masked) {
+      if (gl < 4) bits[gl] = 0u;
+      wave_fence();
+      if (gl < at) atomicOr(&bits[res >> 5], 1u << (res & 31));
+      wave_fence();
+      const uint4 q = *reinterpret_cast<const uint4*>(bits);
+      lo = (uint64_t)q.x | ((uint64_t)q.y << 32);
+      hi = (uint64_t)q.z | ((uint64_t)q.w << 32);
+      wave_fence();
+    }
+    auto hit = [&](int32_t c) -> bool {
+      return masked ? ((c < 64 ? lo >> c : hi >> (c - 64)) & 1ull) != 0ull : held(c, at);
+    };
+    int32_t c = -1, last = 0;
+    for (int a0 = m + 1; a0 < kReselect; a0 += gs) {
+      const bool in = a0 + gl < kReselect;
+      ci = pick(at, a0 + gl, in);
+      const uint64_t fm = ballot(in && !hit(ci)) & gmask;
+      if (fm) {
+        c = shfl_abs(ci, __builtin_ctzll(fm));
+        break;
+      }
+      if (kReselect - 1 - a0 < gs) last = shfl_abs(ci, gbase + kReselect - 1 - a0);
+    }
+    for (int q = 0; c < 0; q += gs) {  // (k = min(F, d) slots: some index is free)
+      const int32_t i = (int32_t)(((int64_t)last + 1 + q + gl) % d);
+      const uint64_t fm = ballot(q + gl < d && !hit(i)) & gmask;
+      if (fm) c = shfl_abs(i, __builtin_ctzll(fm));
+      else if (q + gs >= d) break;
+    }
+    pending |= settle(at, c);
+    wave_fence();
+  }
+  wave_fence();  // every lane has read cl before the group's next entry writes it
+  return res;
 }
 
 // Small-degree entries with 32-bit CDF keys: the group copies the entry's CDF
@@ -716,7 +846,7 @@ __device__ __forceinline__ int32_t group_select_remap(const GraphDev& G, const G
 // the group is lanes gbase .. gbase + gs - 1 (gmask)
 template <int KIND, int KEYS, bool REMAP>
 __device__ int32_t group_select(const GraphDev& G, const GEntry& en, int gs, int gl, int gbase, uint64_t gmask,
-                                uint32_t* lc, int cap, int32_t* cl) {
+                                uint32_t* lc, int cap, int32_t* cl, uint32_t* bits) {
   const int F = en.F;
   const int32_t d = en.d;
   const bool act = gl < F;
@@ -740,107 +870,41 @@ __device__ int32_t group_select(const GraphDev& G, const GEntry& en, int gs, int
   int32_t cand = pick(gl, 0, act);
   if (!act) cand = -1;
   if (!(en.flags & 1u)) return cand;
-  // duplicate check: every lane writes its candidate into the group's
-  // 16-byte-aligned LDS slot, then reads the group's candidates back four
-  // at a time (one broadcast ds_read_b128 per four slots instead of one
-  // ds_bpermute per slot) and compares with the slots before its own
-  cl[gl] = cand;
-  wave_fence();
-  bool dup = false;
-  for (int i0 = 0; i0 + 1 < F; i0 += 4) {
-    const int4 q = *reinterpret_cast<const int4*>(cl + i0);
-    dup |= (gl > i0 && cand == q.x) | (gl > i0 + 1 && cand == q.y) | (gl > i0 + 2 && cand == q.z) |
-           (gl > i0 + 3 && cand == q.w);
-  }
-  dup &= act;
-  wave_fence();  // every lane has read the slot before the next round writes it
-  const uint64_t dm = ballot(dup) & gmask;
-  if (dm == 0ull) return cand;
-  const int j0 = __builtin_ctzll(dm) - gbase;
-  int32_t res = gl < j0 ? cand : -1;
-  // Taken set: for d <= 128 a 128-bit mask held identically by the group's
-  // lanes (O(1) tests, no shuffles; where collisions are frequent), else the
-  // resolved lanes' registers.
-  const bool use_mask = d <= 128;
-  uint64_t mlo = 0, mhi = 0;
-  if (use_mask) {
-    for (int m = 0; m < j0; ++m) {  // the resolved slots 0 .. j0-1
-      const int32_t cm = shfl_abs(cand, gbase + m);
-      if (cm < 64) mlo |= 1ull << cm;
-      else mhi |= 1ull << (cm - 64);
-    }
-  }
-  auto in_mask = [&](int32_t ci) -> bool { return ((ci < 64 ? mlo >> ci : mhi >> (ci - 64)) & 1ull) != 0ull; };
-  for (int jj = j0; jj < F; ++jj) {
-    int32_t c = shfl_abs(cand, gbase + jj);
-    const bool c_taken = use_mask ? in_mask(c) : ((ballot(res == c) & gmask) != 0ull);
-    if (c_taken) {
-      int32_t chosen = -1, last = c;
-      for (int a0 = 1; a0 < kReselect; a0 += gs) {
-        const int a = a0 + gl;
-        int32_t ci = pick(jj, a, a < kReselect);
-        if (a >= kReselect) ci = 0;
-        const bool tk = use_mask ? in_mask(ci) : group_taken(ci, res, jj, gbase);
-        const uint64_t m = ballot((a < kReselect) && !tk) & gmask;
-        if (m) {
-          chosen = shfl_abs(ci, __builtin_ctzll(m));
-          break;
-        }
-        const int ll = kReselect - 1 - a0;
-        if (ll < gs) last = shfl_abs(ci, gbase + ll);
-      }
-      if (chosen < 0) {
-        for (int q = 0; q < d; q += gs) {
-          const int32_t i = (int32_t)(((int64_t)last + 1 + q + gl) % d);
-          const bool tk = use_mask ? in_mask(i) : group_taken(i, res, jj, gbase);
-          const uint64_t m = ballot((q + gl < d) && !tk) & gmask;
-          if (m) {
-            chosen = shfl_abs(i, __builtin_ctzll(m));
-            break;
-          }
-        }
-      }
-      c = chosen;
-    }
-    if (use_mask) {
-      if (c < 64) mlo |= 1ull << c;
-      else mhi |= 1ull << (c - 64);
-    }
-    if (gl == jj) res = c;
-  }
-  return res;
+  return resolve_slots(F, d, gs, gl, gbase, gmask, cl, bits, cand, small || KIND == kUniform ? gs : kSpecDraws, pick);
 }
 
 // Expands `count` (<= 64) entries, all with F <= gs, in groups of gs lanes
 // (4 <= gs <= 32, or 64): 64 / gs groups, the remaining 64 mod gs lanes idle.
 // Needs no per-entry CDF build: uniform, FP32, or integer biases with the CDF
-// cache.  lds: the wave's kGroupLdsWords words for small-degree CDFs (null:
-// searches only).
+// cache.  lds: the wave's scratch, kGroupBaseWords words (kGroupWords with
+// small: small-degree CDFs are staged in it too), 16-byte aligned.
 constexpr int kGroupLdsWords = (kWave / kGroupMin) * kGroupSmallCap;
-// per-wave candidate slots: NG groups of gs lanes rounded up to four words,
-// NG * round4(gs) <= 64 + 3 * NG <= 112 for gs >= 4 (the idle remainder
-// lanes never select, so their slot pointer is never dereferenced)
+// candidate slots: NG groups of gs lanes rounded up to four words, NG *
+// round4(gs) <= 64 + 3 * NG <= 112 for gs >= 4 (the idle remainder lanes never
+// select, so their slot pointer is never dereferenced)
 constexpr int kCandSlotWords = 128;
+// a batch's entries, the candidate slots, four words of taken set per group
+constexpr int kGroupBaseWords = kWave * 16 + kCandSlotWords + 4 * (kWave / kGroupMin);
+constexpr int kGroupWords = kGroupBaseWords + kGroupLdsWords;
 
 // REMAP: entries of region-remap requests may be among them (32-bit keys only).
 template <int KIND, int KEYS = kKeysAny, bool REMAP = false>
 __device__ void group_expand_batch(const GraphDev& G, const csaw_graph_view& hv, const ReqDev* __restrict__ R,
                                    const int32_t* __restrict__ gs2req, const HopDev& H,
-                                   const int32_t* __restrict__ order, int64_t first, int count, int gs,
-                                   uint32_t* lds) {
+                                   const int32_t* __restrict__ order, int64_t first, int count, int gs, uint32_t* lds,
+                                   bool small) {
   static_assert(!REMAP || KEYS == kKeys32, "region remap in groups searches 32-bit keys");
   const int NG = kWave / gs;
   const int lane = lane_id();
   const int gi = lane / gs;  // group; gi == NG: the idle remainder lanes
   const int gl = lane - gi * gs, gbase = gi * gs;
   const int cap = kGroupLdsWords / NG;  // LDS slot words per group
-  uint32_t* lc = lds && gi < NG ? lds + gi * cap : nullptr;
-  // candidate slots of the duplicate check: per wave, each group's gs words
-  // rounded up to four (16-byte aligned); the idle remainder lanes' slot
-  // follows the groups'
-  __shared__ __align__(16) int32_t cand_slots[4][kCandSlotWords];
-  const int gstride = (gs + 3) & ~3;
-  int32_t* gcl = &cand_slots[(threadIdx.x / kWave) & 3][gi * gstride];
+  int4* ents = reinterpret_cast<int4*>(lds);
+  // candidate slots of the duplicate check: each group's gs words rounded up to
+  // four (16-byte aligned); the idle remainder lanes' slot follows the groups'
+  int32_t* gcl = reinterpret_cast<int32_t*>(lds + kWave * 16) + gi * ((gs + 3) & ~3);
+  uint32_t* gbits = lds + kWave * 16 + kCandSlotWords + 4 * min(gi, NG - 1);
+  uint32_t* lc = small && gi < NG ? lds + kGroupBaseWords + gi * cap : nullptr;
   const uint64_t gmask = gs >= kWave ? ~0ull : (((1ull << gs) - 1ull) << gbase);
   GEntry mine;
   mine.d = 0;
@@ -899,12 +963,9 @@ __device__ void group_expand_batch(const GraphDev& G, const csaw_graph_view& hv,
   const bool selects = live && !cp;
   const uint64_t sm = ballot(selects);
   const int nsel = __popcll(sm);
-  // lane r receives the lane of the r-th selecting entry (ds_permute pushes
-  // every lane to a distinct destination: selecting lanes to their rank,
-  // the others after them)
-  const int rank = __popcll(sm & ((1ull << lane) - 1ull));
-  const int dest = selects ? rank : nsel + (lane - rank);
-  const int sel_lane = __builtin_amdgcn_ds_permute(dest << 2, lane);
+  wave_fence();  // the previous batch's rounds have read theirs
+  if (selects) store_gentry(ents + 4 * __popcll(sm & ((1ull << lane) - 1ull)), mine);
+  wave_fence();
   // Software pipeline: a round's neighbour load is consumed (written out) only
   // after the next round's selection, so its latency overlaps that round's
   // searches instead of adding to them.
@@ -913,11 +974,11 @@ __device__ void group_expand_batch(const GraphDev& G, const csaw_graph_view& hv,
   int64_t pp = 0;
   for (int e0 = 0; e0 < nsel; e0 += NG) {
     const int e = gi < NG ? e0 + gi : nsel;
-    const int src = shfl_abs(sel_lane, e < nsel ? e : 0);
-    const GEntry en = shfl_gentry(mine, src);
+    const int4* ep = ents + 4 * (e < nsel ? e : 0);
     int32_t idx = -1;
     if (e < nsel) {
-      const int32_t res = group_select<KIND, KEYS, REMAP>(G, en, gs, gl, gbase, gmask, lc, cap, gcl);
+      const GEntry en = fetch_gentry(ep);
+      const int32_t res = group_select<KIND, KEYS, REMAP>(G, en, gs, gl, gbase, gmask, lc, cap, gcl, gbits);
       idx = gl < en.F ? res : -1;
     }
     if (have) {
@@ -927,10 +988,11 @@ __device__ void group_expand_batch(const GraphDev& G, const csaw_graph_view& hv,
     }
     have = idx >= 0;
     if (have) {
-      pv = en.v;
-      pg = en.g;
-      pp = en.pos + gl;
-      pnb = Update(&hv, G.adj[en.o + idx], en.v);
+      const int4 a = ep[0], b = ep[1];  // read again rather than held over the selection
+      pv = a.x;
+      pg = a.y;
+      pp = pack_i64(b.z, b.w) + gl;
+      pnb = Update(&hv, G.adj[pack_i64(a.z, a.w) + idx], pv);
     }
   }
   if (have) {
