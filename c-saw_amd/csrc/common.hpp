@@ -135,6 +135,7 @@ struct HopDev {
   int32_t chunk_min;    // smallest chunk piece (a power of two, kChunkMin .. kBlockEntries)
   int32_t group_min;    // smallest sub-wave group (kGroupMin .. 32)
   int32_t only_kind;    // 1 + a bias kind: expand only that kind's entries (0: all)
+  uint8_t* kind_mask;   // bit k of entry [64 i, 64 i + 64)'s byte: some entry of kind k emits edges (null: one kind)
   // edge bounds of each request's hops, bounds[(slot * CSAW_MAX_HOPS + hop) * 2 + {0, 1}]
   // (null: not wanted), so that a host needs one copy to place every request
   int64_t* bounds;
@@ -142,8 +143,8 @@ struct HopDev {
 };
 
 // Hops of a batched plan with at most this many frontier entries skip the
-// binning and the variant kernels (whose fixed costs dominate a small hop):
-// one whole-hop kernel per bias kind expands them in frontier order.
+// binning and the variant kernels (whose fixed costs dominate a small hop)
+// whatever their kinds need; see plan_bins_hop for the others.
 constexpr int64_t kSmallHopEntries = 65536;
 
 // Entries per chunk for a hop of n frontier entries: whole 1024-entry buckets

@@ -96,6 +96,7 @@ static void plan_free(csaw_plan* p) {
   }
   (void)hipFree(p->local_excl);
   (void)hipFree(p->order);
+  (void)hipFree(p->kind_mask);
   (void)hipFree(p->blk_excl);
   (void)hipFree(p->grp_excl);
   (void)hipFree(p->chunks);
@@ -242,9 +243,26 @@ static HopDev make_hop(csaw_plan* p, Unit& u, int h) {
   H.chunk_min = p->L.chunk_min;
   H.group_min = p->L.group_min;
   H.only_kind = 0;
+  H.kind_mask = p->kind_mask;
   H.bounds = p->bounds;
   H.n_req = (int32_t)u.reqs.size();
   return H;
+}
+
+// Whether a batched hop of at most nmax entries is binned into chunks with a
+// kernel variant each, or expanded in frontier order by one whole-hop kernel per
+// bias kind.  Frontier order writes each wave's edges next to one another; a
+// block's chunks are spread over the chip and fill the same output lines from
+// several XCDs, which cost more than the variants gained wherever no entry has a
+// CDF to build: 256 mixed requests over RMAT-22 take 22.7 ms binned, 17.3 ms in
+// frontier order, 8 of 64 to 1,024 seeds 0.89 and 0.41.  Binning stays for integer
+// biases without a 32-bit CDF cache (the workgroup variants share the builds),
+// and for what asks for chunks: forced and random variants, chunk logs.
+static bool plan_bins_hop(const csaw_plan* p, const Unit& u, int64_t nmax) {
+  if (p->opts.mode != CSAW_MODE_BATCHED) return false;
+  if (p->opts.log_chunks || (p->opts.sched != CSAW_SCHED_HEURISTIC && p->opts.sched != CSAW_SCHED_MLP)) return true;
+  if (nmax <= kSmallHopEntries) return false;
+  return u.kinds[kInt] && !(p->opts.cdf_cache && !p->g->int_cdf[0] && !p->g->int_cdf[1]);
 }
 
 static int run_unit(csaw_plan* p, Unit& u, hipStream_t st, TimingHook* th) {
@@ -252,16 +270,9 @@ static int run_unit(csaw_plan* p, Unit& u, hipStream_t st, TimingHook* th) {
   const csaw_graph_view hv = p->g->hook_view();
   LaunchCfg L = p->L;
   L.stream = st;
-  const bool batched = p->opts.mode == CSAW_MODE_BATCHED;
   for (int h = 0; h < u.depth_max; ++h) {
     HopDev H = make_hop(p, u, h);
-    // a small hop of a batched plan (its entry bound known on the host) is
-    // not binned: one whole-hop kernel per bias kind, as in the plain sampler
-    // (schedules that ask for particular variants, forced or random, and
-    // chunk logging keep the binned path)
-    const bool small = batched && u.nmax[h] <= kSmallHopEntries && !p->opts.log_chunks &&
-                       (p->opts.sched == CSAW_SCHED_HEURISTIC || p->opts.sched == CSAW_SCHED_MLP);
-    const bool bin = batched && !small;
+    const bool bin = u.bin[h];
     if (bin) {
       if (th) th->begin(kKernFill, st);
       CSAW_TRY(launch_fill(L, p->counters, 0u, kCtrCount - 1));  // keeps the flags word
@@ -325,10 +336,18 @@ static int run_unit(csaw_plan* p, Unit& u, hipStream_t st, TimingHook* th) {
     } else {
       // one launch per bias kind present (one for a plain unit, whose single
       // request has one kind); with several kinds each launch expands only
-      // its own kind's entries
+      // its own kind's entries, side by side on the plan's streams so that
+      // one kind's last waves overlap the others' work
       int nk = 0;
       for (int k = 0; k < 3; ++k) nk += u.kinds[k] ? 1 : 0;
-      for (int kind = 0; kind < 3; ++kind) {
+      const bool fan = nk > 1 && p->side[0];
+      if (fan) {
+        CSAW_HIP(hipEventRecord(p->fork, st));
+        for (int i = 0; i + 1 < nk; ++i) CSAW_HIP(hipStreamWaitEvent(p->side[i], p->fork, 0));
+      }
+      int next = 0;
+      // integer and FP32 kinds first: their chains are the long ones
+      for (int kind : {(int)kInt, (int)kF32, (int)kUniform}) {
         if (!u.kinds[kind]) continue;
         // sub-wave group size from the largest fanout of the kind's requests
         int fmax = 0;
@@ -342,9 +361,16 @@ static int run_unit(csaw_plan* p, Unit& u, hipStream_t st, TimingHook* th) {
         }
         const int gs = group_size_for(fmax, L.group_min);
         H.only_kind = nk > 1 ? 1 + kind : 0;
-        if (th) th->begin(kKernPlain, st);
-        CSAW_TRY(launch_expand_plain(L, kind, G, hv, u.d_req, u.d_gs2req, H, u.nmax[h], gs, remap));
-        if (th) th->end(kKernPlain, st);
+        LaunchCfg K = L;
+        if (fan && next > 0) K.stream = p->side[next - 1];
+        if (th) th->begin(kKernPlain, K.stream);
+        CSAW_TRY(launch_expand_plain(K, kind, G, hv, u.d_req, u.d_gs2req, H, u.nmax[h], gs, remap));
+        if (th) th->end(kKernPlain, K.stream);
+        if (fan && next > 0) {
+          CSAW_HIP(hipEventRecord(p->join[next - 1], K.stream));
+          CSAW_HIP(hipStreamWaitEvent(st, p->join[next - 1], 0));
+        }
+        ++next;
       }
     }
     if (bin && p->opts.log_chunks) {
@@ -389,6 +415,13 @@ extern "C" int csaw_plan_create(csaw_graph* g, const csaw_request* reqs, int32_t
   p->opts = o;
   p->L.num_cu = g->num_cu;
   if (o.tuning) apply_tuning(p->L, o.tuning);
+  // Whole-hop kernels: a plain plan's takes the tuned shape (8 by default: 4 to
+  // 16 within 2% from 3,000 to 1,048,576 seeds, 32 up to 8% slower for degree bias).
+  // A batched plan's tuned expand_per_cu is that of its side-by-side variant
+  // kernels; its kinds' kernels skip one another's batches, and 32 evens out what
+  // is left (32 requests of 64 to 4,096 seeds: 906 us at 32, 1,022 at 8).
+  if (o.mode == CSAW_MODE_BATCHED) p->L.frontier_per_cu = 32;
+  else if (o.tuning && o.tuning->expand_per_cu > 0) p->L.frontier_per_cu = o.tuning->expand_per_cu;
   auto body = [&]() -> int {
     for (int i = 0; i < n_req; ++i) {
       CSAW_TRY(graph_prepare_bias(g, reqs[i].bias));
@@ -409,10 +442,16 @@ extern "C" int csaw_plan_create(csaw_graph* g, const csaw_request* reqs, int32_t
         p->units.back().reqs.push_back(i);
       }
     }
-    int64_t nmax = 1, depth = 1;
+    int64_t nmax = 1, depth = 1, bin_max = 0;
+    bool several = false;
     for (auto& u : p->units) {
       CSAW_TRY(build_unit(p, u));
-      for (int64_t v : u.nmax) nmax = std::max(nmax, v);
+      for (int64_t v : u.nmax) {
+        nmax = std::max(nmax, v);
+        u.bin.push_back(plan_bins_hop(p, u, v));
+        if (u.bin.back()) bin_max = std::max(bin_max, v);
+      }
+      several |= u.kinds[0] + u.kinds[1] + u.kinds[2] > 1;
       depth = std::max<int64_t>(depth, u.depth_max);
     }
     p->req_unit.assign(n_req, {-1, -1});
@@ -433,15 +472,19 @@ extern "C" int csaw_plan_create(csaw_graph* g, const csaw_request* reqs, int32_t
     CSAW_HIP(hipMalloc(&p->totals, sizeof(int64_t) * depth));
     CSAW_HIP(hipMalloc(&p->bytes_acc, sizeof(unsigned long long) * kNumKernKinds));
     CSAW_HIP(hipMemset(p->bytes_acc, 0, sizeof(unsigned long long) * kNumKernKinds));
-    if (o.mode == CSAW_MODE_BATCHED) {
-      CSAW_HIP(hipMalloc(&p->order, sizeof(int32_t) * nblk * kBlockEntries));
+    if (several) CSAW_HIP(hipMalloc(&p->kind_mask, (nmax + kWave - 1) / kWave));
+    if (bin_max > 0) {
+      const int64_t bblk = (bin_max + kBlockEntries - 1) / kBlockEntries;
+      CSAW_HIP(hipMalloc(&p->order, sizeof(int32_t) * bblk * kBlockEntries));
       const int64_t waves = (int64_t)p->L.num_cu * p->L.expand_per_cu * 4;
-      p->chunk_cap = (uint32_t)std::min<int64_t>(nblk * kChunksPerBlock + waves, 0xFFFFFFF0LL);
+      p->chunk_cap = (uint32_t)std::min<int64_t>(bblk * kChunksPerBlock + waves, 0xFFFFFFF0LL);
       CSAW_HIP(hipMalloc(&p->chunks, sizeof(Chunk) * p->chunk_cap));
       p->queue_cap = p->chunk_cap;
       CSAW_HIP(hipMalloc(&p->queues, sizeof(uint32_t) * (int64_t)kNumQueues * p->queue_cap));
       CSAW_HIP(hipMalloc(&p->chosen, p->chunk_cap));
       if (o.log_chunks) CSAW_HIP(hipMalloc(&p->log, sizeof(ChunkLog) * p->chunk_cap));
+    }
+    if (o.mode == CSAW_MODE_BATCHED) {
       if (o.sched == CSAW_SCHED_MLP) {
         if (!o.mlp) {
           set_last_error("CSAW_SCHED_MLP needs a trained csaw_mlp");

@@ -47,6 +47,7 @@ struct Unit {
   std::vector<int32_t> gb;      // per hop: first inactive global sample
   std::vector<int64_t> cap;     // per hop: edge capacity
   std::vector<int64_t> nmax;    // per hop: frontier entries upper bound
+  std::vector<char> bin;        // per hop: binned into chunks (plan_bins_hop)
   ReqDev* d_req = nullptr;
   int32_t* d_gs2req = nullptr;
   int32_t* d_fv0 = nullptr;
@@ -79,6 +80,7 @@ struct csaw_plan {
   std::vector<csaw::Unit> units;
   uint32_t* local_excl = nullptr;
   int32_t* order = nullptr;
+  uint8_t* kind_mask = nullptr;  // whole-hop kernels of several kinds (HopDev)
   uint32_t* blk_excl = nullptr;
   uint64_t* grp_excl = nullptr;
   csaw::Chunk* chunks = nullptr;

@@ -54,6 +54,7 @@ __global__ __launch_bounds__(256) void k_count(GraphDev G, const ReqDev* __restr
     // hands out keep runs of neighbouring entries (siblings, whose edges
     // are neighbours in the output) together in a chunk
     uint32_t k[4];
+    int ek[4];  // bias kind of an entry that emits edges
     int bk[4];
     uint32_t slot[4];
     int32_t eid[4];
@@ -62,6 +63,7 @@ __global__ __launch_bounds__(256) void k_count(GraphDev G, const ReqDev* __restr
     for (int i = 0; i < 4; ++i) {
       const int64_t pos = base + i * 256 + tid;
       k[i] = 0;
+      ek[i] = -1;
       bk[i] = -1;
       eid[i] = 0;
       if (pos < n) {
@@ -72,6 +74,7 @@ __global__ __launch_bounds__(256) void k_count(GraphDev G, const ReqDev* __restr
         const int32_t F = r.fanout[H.hop];
         const int32_t d = G.deg[v];
         k[i] = (uint32_t)entry_k(d, F, r.dedup);
+        if (k[i]) ek[i] = bias_kind(r.bias);
         if (!BIN && H.bytes) {
           const int kind = bias_kind(r.bias);
           const int ck = r.bias == CSAW_BIAS_USER ? 1 : 0;
@@ -89,6 +92,15 @@ __global__ __launch_bounds__(256) void k_count(GraphDev G, const ReqDev* __restr
           atomicAdd(&dsum[bk[i]], (unsigned long long)d);
           atomicAdd(&lsum[bk[i]], (uint32_t)ceil_log2_u32((uint32_t)d));
         }
+      }
+    }
+    if (!BIN && H.kind_mask) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t m = (ballot(ek[i] == kUniform) ? 1u << kUniform : 0u) | (ballot(ek[i] == kInt) ? 1u << kInt : 0u) |
+                           (ballot(ek[i] == kF32) ? 1u << kF32 : 0u);
+        const int64_t pos = base + i * 256 + wid * kWave;
+        if (lane == 0 && pos < n) H.kind_mask[pos / kWave] = (uint8_t)m;
       }
     }
     if (!BIN && H.bytes) {
@@ -372,6 +384,10 @@ __global__ __launch_bounds__(256, KEYS == kKeys32 && !REMAP ? 4 : 1) void k_expa
   const int64_t bs = min((int64_t)kWave, max(per, (n + nw - 1) / nw));
   for (int64_t e0 = (blockIdx.x * 4 + wid) * bs; e0 < n; e0 += nw * bs) {
     const int cnt = (int)min(bs, n - e0);
+    if (H.only_kind && H.kind_mask) {  // nothing of this launch's kind among them
+      const int m = H.kind_mask[e0 / kWave] | H.kind_mask[(e0 + cnt - 1) / kWave];
+      if (!((m >> KIND) & 1)) continue;
+    }
     if constexpr (kGroupOk) {
       if (grp) {
         group_expand_batch<KIND, KEYS, REMAP>(G, hv, R, gs2req, H, nullptr, e0, cnt, gs, glds + wid * kGroupStride,
@@ -873,7 +889,7 @@ int launch_fill(const LaunchCfg& L, uint32_t* p, uint32_t v, int64_t n) {
 int launch_expand_plain(const LaunchCfg& L, int kind, const GraphDev& G, const csaw_graph_view& hv, const ReqDev* R,
                         const int32_t* gs2req, const HopDev& H, int64_t max_entries, int gs, bool remap) {
   int64_t nwg = (max_entries + 3) / 4;
-  int grid = (int)std::max<int64_t>(1, std::min<int64_t>(nwg, grid_of(L, L.expand_per_cu)));
+  int grid = (int)std::max<int64_t>(1, std::min<int64_t>(nwg, grid_of(L, L.frontier_per_cu)));
   if (L.grid_override > 0) grid = L.grid_override;
   // the CDF cache (and its index) is in the view: plain sampling with cdf_cache
   const bool idx = G.cdf_idx || G.int_idx32[0] || G.int_idx32[1] || G.int_idx[0] || G.int_idx[1];

@@ -42,7 +42,8 @@ struct LaunchCfg {
   hipStream_t stream = nullptr;
   int num_cu = 256;
   int count_per_cu = 8;
-  int expand_per_cu = 8;   // WAVE / plain / copy workgroups per CU
+  int expand_per_cu = 8;   // WAVE / copy workgroups per CU
+  int frontier_per_cu = 8; // workgroups per CU of the whole-hop kernels
   int thread_per_cu = 4;   // THREAD workgroups per CU
   int block_per_cu = 2;    // BLOCK workgroups per CU
   int grid_override = 0;

@@ -423,3 +423,25 @@ def test_mdrw_frontier_sizes(C, O, g14, fs):
         so, do, oo = O.mdrw(og, seeds, S, fs, D, request=D)
         src, dst, offs = C.mdrw(g, seeds, S, fs, D, request=D)
         assert np.array_equal(offs, oo) and np.array_equal(src, so) and np.array_equal(dst, do), (S, D)
+
+
+@pytest.mark.parametrize("cdf_cache", [True, False])
+@pytest.mark.parametrize("sizes", [(1500, 2100, 1777, 1301), (7, 129, 1, 63), (64, 1, 640, 65)])
+def test_batched_frontier_order(C, O, g14, cdf_cache, sizes):
+    """Batched hops in frontier order, one kernel per bias kind: hops above and
+    below the binning threshold, kinds that meet inside a 64-entry batch,
+    replacement and region remap beside the default, graph replays."""
+    g, og, *_ = g14
+    specs, want = [], []
+    for i, (n, bias, dedup) in enumerate(zip(sizes, (0, 1, 2, 3), (1, 2, 0, 1))):
+        fan = [[25, 10], [12, 3], [15, 10, 2], [33, 2]][i]
+        s = {"seeds": g.seeds(n, request=i), "fanouts": fan, "bias": bias, "dedup": dedup, "request": i}
+        specs.append(s)
+        want.append(O.sample(og, s["seeds"], fan, bias=bias if bias != 3 else O.BIAS_USER, dedup=dedup, request=i))
+    for kw in ({}, {"use_graph": True}, {"serial_expand": True}, {"sched": C.SCHED_MLP, "mlp": C.Mlp(2)}, {"timing": True}):
+        p = C.Plan(g, specs, mode=C.MODE_BATCHED, cdf_cache=cdf_cache, **kw)
+        for _ in range(3):
+            p.run()
+            for r in range(4):
+                same(p.result(r), want[r], f"request {r} {kw} cache {cdf_cache}")
+        p.close()
