@@ -257,6 +257,11 @@ __device__ __forceinline__ uint64_t readlane_u64(uint64_t v, int l) {
   return ((uint64_t)hi << 32) | lo;
 }
 
+__device__ __forceinline__ uint64_t readfirst_u64(uint64_t v) {
+  return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32)) << 32) |
+         (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+}
+
 // Inclusive wave64 scans on DPP: four row_shr steps (1, 2, 4, 8) give every
 // lane the prefix within its row of 16 lanes; row_bcast:15 then adds row
 // r's last lane to row r+1 (rows 1 and 3), and row_bcast:31 adds lane 31 to

@@ -357,13 +357,14 @@ __global__ void k_fill_u32(uint32_t* __restrict__ p, uint32_t v, int64_t n) {
 // the CDF cache and its 16-ary index (searched through the index).  KEYS:
 // kKeys32 when no integer cache of the view is 64-bit (the 64-bit searches
 // compiled out of the group path).
+constexpr int64_t kWideHopEntries = 16384;
 // REMAP: the hop's requests of this kind use the region-remap mode.
 // The group-only builds are held to 128 registers, four waves per SIMD: their
 // waves wait for memory most of the time (FP32 {15, 10, 5} from 30,011 seeds:
 // 645 us at three waves, 565 us at four).
 template <int KIND, bool IDX, int KEYS, bool REMAP = false>
 __global__ __launch_bounds__(256, KEYS == kKeys32 && !REMAP ? 4 : 1) void k_expand_plain(GraphDev G, csaw_graph_view hv, const ReqDev* __restrict__ R,
-                                                      const int32_t* __restrict__ gs2req, HopDev H, int gs) {
+                                                      const int32_t* __restrict__ gs2req, HopDev H, int hop_gs) {
   constexpr bool kGroupOk = KIND != kInt || IDX;  // no per-entry CDF build needed
   constexpr bool kGroupLds = KIND == kF32 || (KIND == kInt && IDX);  // small cached CDFs staged in LDS
   // (32-bit-key builds are always given a group size: the whole-wave path and
@@ -376,6 +377,12 @@ __global__ __launch_bounds__(256, KEYS == kKeys32 && !REMAP ? 4 : 1) void k_expa
   const int64_t n = *H.n_ptr;
   const int wid = threadIdx.x / kWave;
   const int64_t nw = (int64_t)gridDim.x * 4;
+  // A small hop gives each entry a whole wave: what it waits for are the few
+  // slots with many redraws, and 64 attempts a round end those sooner.  (Uniform
+  // draws collide too rarely for that: groups throughout.)  Region remap of 8,191
+  // seeds on RMAT-22: 813 us in groups, 681 us; FP32 {10, 10} from 10,000 on
+  // RMAT-20 150 and 140 us; from 30,011 seeds on no difference.
+  const int gs = hop_gs > 0 && KIND != kUniform && n <= kWideHopEntries ? kWave : hop_gs;
   // batch size adapts to the frontier: one entry (one group round) per wave
   // when it is small (all waves busy), up to 64 entries per metadata round
   // when it is large

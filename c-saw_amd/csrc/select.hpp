@@ -285,15 +285,17 @@ __device__ __forceinline__ float shfl_abs_f(float v, int src) { return __int_as_
 // Slots of one entry on the gs lanes from gbase (gmask; lane gl of them holds
 // slot gl, F <= gs), all of which follow the same path.  draw(j, a): the float
 // of slot j's attempt a; pick(r): the index r picks; p(i): the normalised CDF.
-// Returns the lane's index (-1 for gl >= F).
+// Returns the lane's index (-1 for gl >= F); with defer, kDeferred on every lane
+// when a slot has nothing after its first attempt and one batch.
 // Bound: the latency of the longest sequences (degrees just above the fanout
 // with most of the weight on taken neighbours: a thousand attempts).  Only the
 // bounds chain from attempt to attempt, two divisions long; draws, picks and
 // their checks do not, so a batch of attempts runs them lane by lane around it.
 // 8,191 seeds of fanouts {10, 10} under degree bias on RMAT-22: 7.3 ms with a
 // wave per entry and every lane on the same attempt, 1.1 ms here.
+constexpr int32_t kDeferred = -2;
 template <class Draw, class Pick, class Norm>
-__device__ __forceinline__ int32_t remap_resolve(int F, int32_t d, int gs, int gl, int gbase, uint64_t gmask,
+__device__ __forceinline__ int32_t remap_resolve(int F, int32_t d, int gs, int gl, int gbase, uint64_t gmask, bool defer,
                                                  const Draw& draw, const Pick& pick, const Norm& p) {
   const float r0 = gl < F ? draw(gl, 0) : 0.0f;
   const int32_t cand = gl < F ? pick(r0) : -1;
@@ -353,6 +355,7 @@ __device__ __forceinline__ int32_t remap_resolve(int F, int32_t d, int gs, int g
       if (free2) chosen = shfl_abs(i2, __builtin_ctzll(free2));
       else if (free) chosen = shfl_abs(i, __builtin_ctzll(free));
       else last = shfl_abs(i2, gbase + nb - 1);
+      if (defer && a0 > 0 && chosen < 0) return kDeferred;
     }
     if (chosen < 0) {
       for (int q = 0; q < d; q += gs) {
@@ -396,7 +399,7 @@ __device__ __forceinline__ int32_t remap_pick(const Picker& pk, float r) {
 
 __device__ int32_t wave_select_remap(const Entry& en, const Picker& pk) {
   return remap_resolve(
-      en.F, en.d, kWave, lane_id(), 0, ~0ull, [&](int j, int a) { return philox_u24(draw(en, j, a)); },
+      en.F, en.d, kWave, lane_id(), 0, ~0ull, false, [&](int j, int a) { return philox_u24(draw(en, j, a)); },
       [&](float r) { return remap_pick(pk, r); }, [&](int32_t i) { return remap_p(pk, i); });
 }
 
@@ -641,7 +644,8 @@ __device__ __forceinline__ GEntry fetch_gentry(const int4* p) {
 // and four.
 // pick(j, a, valid): slot j's attempt a; lanes with valid == false take part.
 // spec: attempts a slot draws at first (the group's size where draws cost no
-// memory reads).
+// memory reads).  defer: return kDeferred on every lane, with nothing chosen, when
+// a slot is left without a free index after those and a round of the whole group.
 //
 // A slot whose draw repeats no earlier draw is final at once.  A pending slot's
 // draw is held by an earlier slot whatever that one's own fate (a slot only
@@ -661,7 +665,7 @@ constexpr int kSpecDraws = 3;
 constexpr int kTakenMaskCap = 128;  // degrees whose taken set fits four words
 template <class Pick>
 __device__ __forceinline__ int32_t resolve_slots(int F, int32_t d, int gs, int gl, int gbase, uint64_t gmask, int32_t* cl,
-                                                 uint32_t* bits, int32_t cand, int spec, const Pick& pick) {
+                                                 uint32_t* bits, int32_t cand, int spec, bool defer, const Pick& pick) {
   const bool act = gl < F;
   // duplicate check: the group's draws read back four at a time (one broadcast
   // ds_read_b128 per four slots)
@@ -749,6 +753,10 @@ __device__ __forceinline__ int32_t resolve_slots(int F, int32_t d, int gs, int g
         c = shfl_abs(ci, __builtin_ctzll(fm));
         break;
       }
+      if (defer) {
+        wave_fence();
+        return kDeferred;
+      }
       if (kReselect - 1 - a0 < gs) last = shfl_abs(ci, gbase + kReselect - 1 - a0);
     }
     for (int q = 0; c < 0; q += gs) {  // (k = min(F, d) slots: some index is free)
@@ -789,7 +797,7 @@ __device__ __forceinline__ int32_t gpick_small(const GEntry& en, const uint32_t*
 // not settle and totals out of its range take the search over p_i.
 template <int KIND>
 __device__ __forceinline__ int32_t group_select_remap(const GraphDev& G, const GEntry& en, int gs, int gl, int gbase,
-                                                      uint64_t gmask, uint32_t* lc, bool small) {
+                                                      uint64_t gmask, uint32_t* lc, bool small, bool defer) {
   const int32_t d = en.d;
   const uint32_t mode = (en.flags >> 4) & 15u;
   const bool user = (en.flags >> 1) & 1u;
@@ -838,7 +846,7 @@ __device__ __forceinline__ int32_t group_select_remap(const GraphDev& G, const G
     return lo < d ? lo : d - 1;
   };
   return remap_resolve(
-      en.F, d, gs, gl, gbase, gmask, [&](int j, int a) { return philox_u24(gdraw(en, j, a)); }, pick, p);
+      en.F, d, gs, gl, gbase, gmask, defer, [&](int j, int a) { return philox_u24(gdraw(en, j, a)); }, pick, p);
 }
 
 // lc: the group's LDS slot of cap words (null: no small path)
@@ -846,7 +854,7 @@ __device__ __forceinline__ int32_t group_select_remap(const GraphDev& G, const G
 // the group is lanes gbase .. gbase + gs - 1 (gmask)
 template <int KIND, int KEYS, bool REMAP>
 __device__ int32_t group_select(const GraphDev& G, const GEntry& en, int gs, int gl, int gbase, uint64_t gmask,
-                                uint32_t* lc, int cap, int32_t* cl, uint32_t* bits) {
+                                uint32_t* lc, int cap, int32_t* cl, uint32_t* bits, bool defer) {
   const int F = en.F;
   const int32_t d = en.d;
   const bool act = gl < F;
@@ -854,7 +862,7 @@ __device__ int32_t group_select(const GraphDev& G, const GEntry& en, int gs, int
   const bool small = KIND != kUniform && lc && d <= cap &&
                      (mode == kPickInt32Idx || mode == kPickF32 || mode == kPickF32Idx);
   if constexpr (REMAP)
-    if (en.flags & 4u) return group_select_remap<KIND>(G, en, gs, gl, gbase, gmask, lc, small);
+    if (en.flags & 4u) return group_select_remap<KIND>(G, en, gs, gl, gbase, gmask, lc, small, defer);
   if (small) {
     const uint32_t* C = KIND == kF32 ? reinterpret_cast<const uint32_t*>(G.cdf)
                                      : ((en.flags >> 1) & 1u ? G.int_cdf32[1] : G.int_cdf32[0]);
@@ -870,7 +878,7 @@ __device__ int32_t group_select(const GraphDev& G, const GEntry& en, int gs, int
   int32_t cand = pick(gl, 0, act);
   if (!act) cand = -1;
   if (!(en.flags & 1u)) return cand;
-  return resolve_slots(F, d, gs, gl, gbase, gmask, cl, bits, cand, small || KIND == kUniform ? gs : kSpecDraws, pick);
+  return resolve_slots(F, d, gs, gl, gbase, gmask, cl, bits, cand, small || KIND == kUniform ? gs : kSpecDraws, defer, pick);
 }
 
 // Expands `count` (<= 64) entries, all with F <= gs, in groups of gs lanes
@@ -883,8 +891,9 @@ constexpr int kGroupLdsWords = (kWave / kGroupMin) * kGroupSmallCap;
 // round4(gs) <= 64 + 3 * NG <= 112 for gs >= 4 (the idle remainder lanes never
 // select, so their slot pointer is never dereferenced)
 constexpr int kCandSlotWords = 128;
-// a batch's entries, the candidate slots, four words of taken set per group
-constexpr int kGroupBaseWords = kWave * 16 + kCandSlotWords + 4 * (kWave / kGroupMin);
+// a batch's entries, the candidate slots, four words of taken set per group, the
+// deferred entries
+constexpr int kGroupBaseWords = kWave * 16 + kCandSlotWords + 4 * (kWave / kGroupMin) + 4;
 constexpr int kGroupWords = kGroupBaseWords + kGroupLdsWords;
 
 // REMAP: entries of region-remap requests may be among them (32-bit keys only).
@@ -894,18 +903,10 @@ __device__ void group_expand_batch(const GraphDev& G, const csaw_graph_view& hv,
                                    const int32_t* __restrict__ order, int64_t first, int count, int gs, uint32_t* lds,
                                    bool small) {
   static_assert(!REMAP || KEYS == kKeys32, "region remap in groups searches 32-bit keys");
-  const int NG = kWave / gs;
   const int lane = lane_id();
-  const int gi = lane / gs;  // group; gi == NG: the idle remainder lanes
-  const int gl = lane - gi * gs, gbase = gi * gs;
-  const int cap = kGroupLdsWords / NG;  // LDS slot words per group
+  const int cap0 = kGroupLdsWords / (kWave / gs);  // LDS slot words per group
   int4* ents = reinterpret_cast<int4*>(lds);
-  // candidate slots of the duplicate check: each group's gs words rounded up to
-  // four (16-byte aligned); the idle remainder lanes' slot follows the groups'
-  int32_t* gcl = reinterpret_cast<int32_t*>(lds + kWave * 16) + gi * ((gs + 3) & ~3);
-  uint32_t* gbits = lds + kWave * 16 + kCandSlotWords + 4 * min(gi, NG - 1);
-  uint32_t* lc = small && gi < NG ? lds + kGroupBaseWords + gi * cap : nullptr;
-  const uint64_t gmask = gs >= kWave ? ~0ull : (((1ull << gs) - 1ull) << gbase);
+  uint32_t* hard = lds + kGroupBaseWords - 4;  // bits of the deferred entries
   GEntry mine;
   mine.d = 0;
   mine.F = 0;
@@ -923,11 +924,11 @@ __device__ void group_expand_batch(const GraphDev& G, const csaw_graph_view& hv,
     const uint32_t mode = (mine.flags >> 4) & 15u;
     if (KIND == kF32 && mode == kPickF32Idx)
       warm = *reinterpret_cast<const uint32_t*>(
-          mine.d <= cap ? G.cdf + mine.o : cdf_index_first_block<float>(G.cdf, G.cdf_idx, G.E, mine.o, mine.d));
+          mine.d <= cap0 ? G.cdf + mine.o : cdf_index_first_block<float>(G.cdf, G.cdf_idx, G.E, mine.o, mine.d));
     if (KIND == kInt && mode == kPickInt32Idx) {
       const bool user = (mine.flags >> 1) & 1u;
       const uint32_t* C = user ? G.int_cdf32[1] : G.int_cdf32[0];
-      warm = mine.d <= cap
+      warm = mine.d <= cap0
                  ? C[mine.o]
                  : *cdf_index_first_block<uint32_t>(C, user ? G.int_idx32[1] : G.int_idx32[0], G.E, mine.o, mine.d);
     }
@@ -966,34 +967,68 @@ __device__ void group_expand_batch(const GraphDev& G, const csaw_graph_view& hv,
   wave_fence();  // the previous batch's rounds have read theirs
   if (selects) store_gentry(ents + 4 * __popcll(sm & ((1ull << lane) - 1ull)), mine);
   wave_fence();
+  if (lane < 2) hard[lane] = 0u;
+  wave_fence();
   // Software pipeline: a round's neighbour load is consumed (written out) only
   // after the next round's selection, so its latency overlaps that round's
   // searches instead of adding to them.
   bool have = false;
   int32_t pv = 0, pg = 0, pnb = 0;
   int64_t pp = 0;
-  for (int e0 = 0; e0 < nsel; e0 += NG) {
-    const int e = gi < NG ? e0 + gi : nsel;
-    const int4* ep = ents + 4 * (e < nsel ? e : 0);
-    int32_t idx = -1;
-    if (e < nsel) {
-      const GEntry en = fetch_gentry(ep);
-      const int32_t res = group_select<KIND, KEYS, REMAP>(G, en, gs, gl, gbase, gmask, lc, cap, gcl, gbits);
-      idx = gl < en.F ? res : -1;
+  // The groups first; then the entries they deferred, a wave each: a slot that
+  // needs hundreds of redraws (a degree just above the fanout, the weight on
+  // neighbours already taken) would hold the other groups of its round, and
+  // takes 64 attempts a round this way.  Degree bias with the CDF cache, fanouts
+  // {15, 10, 5} from 12,000 seeds on RMAT-22: 638 -> 434 us; region remap of
+  // 8,191 seeds 1,274 -> 812 us.  Not for uniform draws, whose redraws are few
+  // and even (their region remap 132 us without, 161 us with).
+  constexpr int kPhases = KIND == kUniform ? 1 : 2;
+  uint64_t left = 0;
+  for (int phase = 0; phase < kPhases; ++phase) {
+    const int w = phase ? kWave : gs;  // lanes per entry
+    const int NG = kWave / w;
+    const int gi = lane / w;  // group; gi == NG: the idle remainder lanes
+    const int gl = lane - gi * w, gbase = gi * w;
+    const int cap = kGroupLdsWords / NG;
+    // candidate slots of the duplicate check: each group's w words rounded up to
+    // four (16-byte aligned); the idle remainder lanes' slot follows the groups'
+    int32_t* gcl = reinterpret_cast<int32_t*>(lds + kWave * 16) + gi * ((w + 3) & ~3);
+    uint32_t* gbits = lds + kWave * 16 + kCandSlotWords + 4 * min(gi, NG - 1);
+    uint32_t* lc = small && gi < NG ? lds + kGroupBaseWords + gi * cap : nullptr;
+    const uint64_t gmask = w >= kWave ? ~0ull : (((1ull << w) - 1ull) << gbase);
+    if (phase) left = readfirst_u64(*reinterpret_cast<const uint64_t*>(hard));
+    const int n = phase ? __popcll(left) : nsel;
+    for (int e0 = 0; e0 < n; e0 += NG) {
+      int e = gi < NG ? e0 + gi : nsel;
+      if (phase) {
+        e = __builtin_ctzll(left);
+        left &= left - 1ull;
+      }
+      const int4* ep = ents + 4 * (e < nsel ? e : 0);
+      int32_t idx = -1;
+      if (e < nsel) {
+        const GEntry en = fetch_gentry(ep);
+        const int32_t res =
+            group_select<KIND, KEYS, REMAP>(G, en, w, gl, gbase, gmask, lc, cap, gcl, gbits,
+                                           kPhases == 2 && phase == 0 && w < kWave);
+        idx = gl < en.F ? res : -1;
+        if (kPhases == 2 && res == kDeferred && gl == 0) atomicOr(&hard[e >> 5], 1u << (e & 31));
+      }
+      if (have) {
+        H.src[pp] = pv;
+        H.dst[pp] = pnb;
+        H.smp[pp] = pg;
+      }
+      have = idx >= 0;
+      if (have) {
+        const int4 a = ep[0], b = ep[1];  // read again rather than held over the selection
+        pv = a.x;
+        pg = a.y;
+        pp = pack_i64(b.z, b.w) + gl;
+        pnb = Update(&hv, G.adj[pack_i64(a.z, a.w) + idx], pv);
+      }
     }
-    if (have) {
-      H.src[pp] = pv;
-      H.dst[pp] = pnb;
-      H.smp[pp] = pg;
-    }
-    have = idx >= 0;
-    if (have) {
-      const int4 a = ep[0], b = ep[1];  // read again rather than held over the selection
-      pv = a.x;
-      pg = a.y;
-      pp = pack_i64(b.z, b.w) + gl;
-      pnb = Update(&hv, G.adj[pack_i64(a.z, a.w) + idx], pv);
-    }
+    wave_fence();
   }
   if (have) {
     H.src[pp] = pv;
