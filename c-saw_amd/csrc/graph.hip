@@ -625,6 +625,7 @@ csaw_graph_view csaw_graph::hook_view() const {
 
 static void graph_free(csaw_graph* g) {
   if (!g) return;
+  g->work->close();
   (void)hipFree(g->off);
   (void)hipFree(g->adj);
   (void)hipFree(g->deg);

@@ -1,9 +1,51 @@
 // Device-resident CSR graph (replaces gpu_graph, non-stream/gpu_graph.cuh:10-65,
 // and the host loader graph<>, non-stream/graph.hpp:4-111).
 #pragma once
+#include <memory>
+#include <mutex>
 #include <vector>
 
 #include "common.hpp"
+
+namespace csaw {
+// The streams and events one plan uses at a time.
+struct PlanStreams {
+  static constexpr int kSide = 3;
+  hipStream_t main = nullptr, side[kSide] = {};
+  hipEvent_t begin = nullptr, end = nullptr;  // of a synchronised run
+  hipEvent_t fork = nullptr, join[kSide] = {};
+  int create(bool with_side);
+  void destroy();
+};
+
+// Workspaces and streams of destroyed plans, kept for the next plan on the same
+// graph (a call of the sampler makes a plan and destroys it).  At most kHeldBytes
+// in blocks of at most kBlockBytes and kHeldStreams stream sets; what the graph
+// still holds when it is destroyed goes back to the device, and an allocation
+// that fails gives everything back and tries again.  The owner of a block waits
+// for its work before give(); take() and give() may be called from any thread.
+struct Workspace {
+  static constexpr size_t kHeldBytes = 256u << 20, kBlockBytes = 128u << 20, kHeldStreams = 8;
+  struct Block {
+    void* p = nullptr;
+    size_t bytes = 0;
+  };
+  int take(size_t bytes, Block* b);
+  void give(Block b);
+  int take_streams(bool with_side, PlanStreams* s);
+  void give_streams(PlanStreams s);
+  void close();  // the graph is gone: blocks given from now on are freed
+  ~Workspace() { close(); }
+
+ private:
+  std::mutex mu;
+  std::vector<Block> blocks;
+  std::vector<PlanStreams> streams;
+  size_t held = 0;
+  bool closed = false;
+  void trim();
+};
+}  // namespace csaw
 
 struct csaw_graph {
   int64_t V = 0, E = 0, max_deg = 0;
@@ -35,6 +77,8 @@ struct csaw_graph {
   // (environment CSAW_INT_CDF_KEYS=64 at graph creation; covers the 64-bit
   // search paths on graphs whose totals are small)
   bool wide_int_cdf = false;
+  // shared with the plans, which may outlive the graph
+  std::shared_ptr<csaw::Workspace> work = std::make_shared<csaw::Workspace>();
 
   csaw::GraphDev view(bool use_cache = false) const;
   csaw_graph_view hook_view() const;

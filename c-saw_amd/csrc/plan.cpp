@@ -12,6 +12,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include <numeric>
 #include <vector>
 
@@ -57,6 +58,10 @@ EventTimer::~EventTimer() {
   }
 }
 
+// csaw_sample packs results of at most this many words (64 MB) for one copy; the
+// time of larger ones is the copy's own
+constexpr int64_t kStageWords = 16 << 20;
+
 static int64_t ub_mul(int64_t a, int64_t b) {
   if (a == 0 || b == 0) return 0;
   if (a > (int64_t)1 << 40 || b > (int64_t)1 << 40 || a > ((int64_t)1 << 62) / b) return (int64_t)1 << 62;
@@ -81,41 +86,124 @@ static int validate_request(const csaw_graph* g, const csaw_request& r) {
   return CSAW_OK;
 }
 
+namespace csaw {
+
+int PlanStreams::create(bool with_side) {
+  if (!main) {
+    CSAW_HIP(hipStreamCreateWithFlags(&main, hipStreamNonBlocking));
+    CSAW_HIP(hipEventCreate(&begin));
+    CSAW_HIP(hipEventCreate(&end));
+  }
+  if (with_side && !join[kSide - 1]) {
+    if (!fork) CSAW_HIP(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
+    for (int i = 0; i < kSide; ++i) {
+      if (!side[i]) CSAW_HIP(hipStreamCreateWithFlags(&side[i], hipStreamNonBlocking));
+      if (!join[i]) CSAW_HIP(hipEventCreateWithFlags(&join[i], hipEventDisableTiming));
+    }
+  }
+  return CSAW_OK;
+}
+
+void PlanStreams::destroy() {
+  for (hipEvent_t e : {begin, end, fork, join[0], join[1], join[2]})
+    if (e) (void)hipEventDestroy(e);
+  for (hipStream_t x : {main, side[0], side[1], side[2]})
+    if (x) (void)hipStreamDestroy(x);
+  *this = PlanStreams();
+}
+
+int Workspace::take(size_t bytes, Block* b) {
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    size_t best = blocks.size();
+    for (size_t i = 0; i < blocks.size(); ++i)
+      if (blocks[i].bytes >= bytes && blocks[i].bytes <= 4 * bytes + (1u << 20) &&
+          (best == blocks.size() || blocks[i].bytes < blocks[best].bytes))
+        best = i;
+    if (best < blocks.size()) {
+      *b = blocks[best];
+      held -= b->bytes;
+      blocks.erase(blocks.begin() + best);
+      return CSAW_OK;
+    }
+  }
+  b->bytes = (bytes + 65535) & ~(size_t)65535;
+  if (hipMalloc(&b->p, b->bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    trim();
+    CSAW_HIP(hipMalloc(&b->p, b->bytes));
+  }
+  return CSAW_OK;
+}
+
+void Workspace::give(Block b) {
+  if (!b.p) return;
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    if (!closed && b.bytes <= kBlockBytes && held + b.bytes <= kHeldBytes) {
+      blocks.push_back(b);
+      held += b.bytes;
+      return;
+    }
+  }
+  (void)hipFree(b.p);
+}
+
+int Workspace::take_streams(bool with_side, PlanStreams* s) {
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    if (!streams.empty()) {
+      *s = streams.back();
+      streams.pop_back();
+    }
+  }
+  return s->create(with_side);
+}
+
+void Workspace::give_streams(PlanStreams s) {
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    if (!closed && streams.size() < kHeldStreams && s.main) {
+      streams.push_back(s);
+      return;
+    }
+  }
+  s.destroy();
+}
+
+void Workspace::trim() {
+  std::vector<Block> out;
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    out.swap(blocks);
+    held = 0;
+  }
+  for (Block& b : out) (void)hipFree(b.p);
+}
+
+void Workspace::close() {
+  trim();
+  std::vector<PlanStreams> out;
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    closed = true;
+    out.swap(streams);
+  }
+  for (PlanStreams& s : out) s.destroy();
+}
+
+}  // namespace csaw
+
 static void plan_free(csaw_plan* p) {
   if (!p) return;
-  for (auto& u : p->units) {
-    (void)hipFree(u.d_req);
-    (void)hipFree(u.d_gs2req);
-    (void)hipFree(u.d_fv0);
-    (void)hipFree(u.d_fs0);
-    (void)hipFree(u.d_fo0);
-    for (auto* q : u.d_eo) (void)hipFree(q);
-    for (auto* q : u.d_src) (void)hipFree(q);
-    for (auto* q : u.d_dst) (void)hipFree(q);
-    for (auto* q : u.d_smp) (void)hipFree(q);
-  }
-  (void)hipFree(p->local_excl);
-  (void)hipFree(p->order);
-  (void)hipFree(p->kind_mask);
-  (void)hipFree(p->blk_excl);
-  (void)hipFree(p->grp_excl);
-  (void)hipFree(p->chunks);
-  (void)hipFree(p->counters);
-  (void)hipFree(p->queues);
-  (void)hipFree(p->totals);
-  (void)hipFree(p->chosen);
-  (void)hipFree(p->log);
-  (void)hipFree(p->d_mlp);
-  (void)hipFree(p->bytes_acc);
+  // work that a call has not waited for may still use the workspace, on a stream
+  // of the caller's
+  if (p->busy) (void)hipDeviceSynchronize();
   if (p->gexec) (void)hipGraphExecDestroy(p->gexec);
-  if (p->own_stream && p->stream) (void)hipStreamDestroy(p->stream);
-  for (int i = 0; i < csaw_plan::kSide; ++i) {
-    if (p->side[i]) (void)hipStreamDestroy(p->side[i]);
-    if (p->join[i]) (void)hipEventDestroy(p->join[i]);
+  if (p->work) {
+    p->work->give(p->slab);
+    p->work->give_streams(p->st);
   }
-  if (p->fork) (void)hipEventDestroy(p->fork);
-  if (p->begin) (void)hipEventDestroy(p->begin);
-  if (p->end) (void)hipEventDestroy(p->end);
   delete p;
 }
 
@@ -175,45 +263,112 @@ static int build_unit(csaw_plan* p, Unit& u) {
       return CSAW_ERR_CAPACITY;
     }
   }
-  // device buffers
-  const int64_t G = u.G;
-  CSAW_HIP(hipMalloc(&u.d_req, sizeof(ReqDev) * std::max<size_t>(rd.size(), 1)));
-  if (!rd.empty()) CSAW_HIP(hipMemcpy(u.d_req, rd.data(), sizeof(ReqDev) * rd.size(), hipMemcpyHostToDevice));
-  std::vector<int32_t> gs2req(G), fv0(G), fs0(G);
-  std::vector<int64_t> fo0(G + 1);
-  for (size_t i = 0; i < u.reqs.size(); ++i) {
-    const csaw_request& r = p->reqs[u.reqs[i]];
-    const std::vector<int32_t>& sd = p->seeds[u.reqs[i]];
-    for (int32_t s = 0; s < r.samples; ++s) {
-      const int64_t g = u.gbase[i] + s;
-      gs2req[g] = (int32_t)i;
-      fv0[g] = sd[s];
-      fs0[g] = (int32_t)g;
+  u.d_eo.assign(u.depth_max, nullptr);
+  u.d_src.assign(u.depth_max, nullptr);
+  u.d_dst.assign(u.depth_max, nullptr);
+  u.d_smp.assign(u.depth_max, nullptr);
+  u.rd = std::move(rd);
+  return CSAW_OK;
+}
+
+// Carves a plan's arrays from one block: a first pass with base null sizes it.
+struct Carver {
+  char* base = nullptr;
+  size_t at = 0;
+  template <typename T>
+  void part(T** p, int64_t count) {
+    if (base) *p = reinterpret_cast<T*>(base + at);
+    at += (std::max<int64_t>(count, 1) * sizeof(T) + 255) & ~(size_t)255;
+  }
+};
+
+struct PlanSizes {
+  int64_t nmax = 1, depth = 1, bin_max = 0, staging = 0;
+  bool several = false, mlp = false;
+};
+
+// What the host fills in comes first (`filled` bytes).
+static void plan_layout(csaw_plan* p, const PlanSizes& z, Carver& c, size_t* filled) {
+  const size_t state = kCtrBytes + kBoundsBytes * p->reqs.size();
+  c.part(&p->counters, state / sizeof(uint32_t));
+  if (c.base) p->bounds = reinterpret_cast<int64_t*>(reinterpret_cast<char*>(p->counters) + kCtrBytes);
+  c.part(&p->bytes_acc, kNumKernKinds);
+  for (auto& u : p->units) {
+    c.part(&u.d_req, (int64_t)u.rd.size());
+    c.part(&u.d_fv0, u.G);
+  }
+  *filled = c.at;
+  for (auto& u : p->units) {
+    c.part(&u.d_gs2req, u.G);
+    c.part(&u.d_fs0, u.G);
+    c.part(&u.d_fo0, u.G + 1);
+  }
+  for (auto& u : p->units)
+    for (int h = 0; h < u.depth_max; ++h) {
+      c.part(&u.d_eo[h], u.G + 1);
+      c.part(&u.d_src[h], u.cap[h]);
+      c.part(&u.d_dst[h], u.cap[h]);
+      c.part(&u.d_smp[h], u.cap[h]);
+    }
+  const int64_t nblk = (z.nmax + kBlockEntries - 1) / kBlockEntries;
+  c.part(&p->local_excl, z.nmax);
+  c.part(&p->blk_excl, nblk);
+  c.part(&p->grp_excl, (nblk + 1023) / 1024);
+  c.part(&p->totals, z.depth);
+  if (z.several) c.part(&p->kind_mask, (z.nmax + kWave - 1) / kWave);
+  if (z.bin_max > 0) {
+    const int64_t bblk = (z.bin_max + kBlockEntries - 1) / kBlockEntries;
+    const int64_t waves = (int64_t)p->L.num_cu * p->L.expand_per_cu * 4;
+    p->chunk_cap = (uint32_t)std::min<int64_t>(bblk * kChunksPerBlock + waves, 0xFFFFFFF0LL);
+    p->queue_cap = p->chunk_cap;
+    c.part(&p->order, bblk * kBlockEntries);
+    c.part(&p->chunks, p->chunk_cap);
+    c.part(&p->queues, (int64_t)kNumQueues * p->queue_cap);
+    c.part(&p->chosen, p->chunk_cap);
+    if (p->opts.log_chunks) c.part(&p->log, p->chunk_cap);
+  }
+  if (z.mlp) c.part(&p->d_mlp, kMlpParams);
+  if (z.staging > 0) c.part(&p->staging, z.staging);
+}
+
+namespace csaw {
+// The first frontier besides its vertices: sample g at position g, of the last
+// request whose first sample is not above g (and has samples).
+__global__ void k_first_frontier(const ReqDev* __restrict__ R, int n_req, int64_t G, int32_t* __restrict__ gs2req,
+                                 int32_t* __restrict__ fs, int64_t* __restrict__ fo) {
+  for (int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; g <= G; g += (int64_t)gridDim.x * blockDim.x) {
+    fo[g] = g;
+    if (g == G) continue;
+    int lo = 0, hi = n_req;  // last request with gbase <= g
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (R[mid].gbase <= g) lo = mid; else hi = mid;
+    }
+    gs2req[g] = lo;
+    fs[g] = (int32_t)g;
+  }
+}
+}  // namespace csaw
+
+// Requests and seeds, one copy in the block's own layout; the rest of the first
+// frontier is written on the device.
+static int upload_inputs(csaw_plan* p, const csaw_request* reqs, size_t filled) {
+  std::vector<char> host(filled, 0);  // (zeroes: the counters, the bounds, the byte counts)
+  auto at = [&](const void* dev) {
+    return host.data() + (reinterpret_cast<const char*>(dev) - static_cast<char*>(p->slab.p));
+  };
+  for (auto& u : p->units) {
+    if (!u.rd.empty()) memcpy(at(u.d_req), u.rd.data(), sizeof(ReqDev) * u.rd.size());
+    for (size_t i = 0; i < u.reqs.size(); ++i) {
+      const csaw_request& r = reqs[u.reqs[i]];
+      if (r.samples > 0) memcpy(at(u.d_fv0) + sizeof(int32_t) * u.gbase[i], r.seeds, sizeof(int32_t) * r.samples);
     }
   }
-  std::iota(fo0.begin(), fo0.end(), (int64_t)0);
-  CSAW_HIP(hipMalloc(&u.d_gs2req, sizeof(int32_t) * std::max<int64_t>(G, 1)));
-  CSAW_HIP(hipMalloc(&u.d_fv0, sizeof(int32_t) * std::max<int64_t>(G, 1)));
-  CSAW_HIP(hipMalloc(&u.d_fs0, sizeof(int32_t) * std::max<int64_t>(G, 1)));
-  CSAW_HIP(hipMalloc(&u.d_fo0, sizeof(int64_t) * (G + 1)));
-  if (G > 0) {
-    CSAW_HIP(hipMemcpy(u.d_gs2req, gs2req.data(), sizeof(int32_t) * G, hipMemcpyHostToDevice));
-    CSAW_HIP(hipMemcpy(u.d_fv0, fv0.data(), sizeof(int32_t) * G, hipMemcpyHostToDevice));
-    CSAW_HIP(hipMemcpy(u.d_fs0, fs0.data(), sizeof(int32_t) * G, hipMemcpyHostToDevice));
-  }
-  CSAW_HIP(hipMemcpy(u.d_fo0, fo0.data(), sizeof(int64_t) * (G + 1), hipMemcpyHostToDevice));
-  for (int h = 0; h < u.depth_max; ++h) {
-    int64_t* eo;
-    int32_t *s, *d, *m;
-    CSAW_HIP(hipMalloc(&eo, sizeof(int64_t) * (G + 1)));
-    u.d_eo.push_back(eo);
-    const int64_t c = std::max<int64_t>(u.cap[h], 1);
-    CSAW_HIP(hipMalloc(&s, sizeof(int32_t) * c));
-    u.d_src.push_back(s);
-    CSAW_HIP(hipMalloc(&d, sizeof(int32_t) * c));
-    u.d_dst.push_back(d);
-    CSAW_HIP(hipMalloc(&m, sizeof(int32_t) * c));
-    u.d_smp.push_back(m);
+  CSAW_HIP(hipMemcpy(p->slab.p, host.data(), filled, hipMemcpyHostToDevice));
+  for (auto& u : p->units) {
+    const int grid = (int)std::min<int64_t>(u.G / 256 + 1, (int64_t)p->L.num_cu * 8);
+    k_first_frontier<<<grid, 256, 0, p->stream>>>(u.d_req, (int)u.rd.size(), u.G, u.d_gs2req, u.d_fs0, u.d_fo0);
+    CSAW_LAUNCH_CHECK();
   }
   return CSAW_OK;
 }
@@ -308,22 +463,22 @@ static int run_unit(csaw_plan* p, Unit& u, hipStream_t st, TimingHook* th) {
       E.log = p->opts.log_chunks ? p->log : nullptr;
       E.int_cache = p->opts.cdf_cache != 0;
       E.remap = u.remap ? 1 : 0;
-      if (p->side[0]) {
+      if (p->fan) {
         // the hop's expansion kernels (one per variant queue) run side by
         // side on four streams, so one kernel's last chunks overlap the
         // others' work; all join before the next hop (with timing on, each
         // kernel's events are recorded on the stream it runs on, so the
         // times are those of this concurrent schedule)
-        hipStream_t ss[1 + csaw_plan::kSide] = {st};
-        CSAW_HIP(hipEventRecord(p->fork, st));
-        for (int i = 0; i < csaw_plan::kSide; ++i) {
-          CSAW_HIP(hipStreamWaitEvent(p->side[i], p->fork, 0));
-          ss[1 + i] = p->side[i];
+        hipStream_t ss[1 + PlanStreams::kSide] = {st};
+        CSAW_HIP(hipEventRecord(p->st.fork, st));
+        for (int i = 0; i < PlanStreams::kSide; ++i) {
+          CSAW_HIP(hipStreamWaitEvent(p->st.side[i], p->st.fork, 0));
+          ss[1 + i] = p->st.side[i];
         }
-        CSAW_TRY(launch_expand_chunks(L, G, hv, u.d_req, u.d_gs2req, H, E, u.kinds, th, ss, 1 + csaw_plan::kSide));
-        for (int i = 0; i < csaw_plan::kSide; ++i) {
-          CSAW_HIP(hipEventRecord(p->join[i], p->side[i]));
-          CSAW_HIP(hipStreamWaitEvent(st, p->join[i], 0));
+        CSAW_TRY(launch_expand_chunks(L, G, hv, u.d_req, u.d_gs2req, H, E, u.kinds, th, ss, 1 + PlanStreams::kSide));
+        for (int i = 0; i < PlanStreams::kSide; ++i) {
+          CSAW_HIP(hipEventRecord(p->st.join[i], p->st.side[i]));
+          CSAW_HIP(hipStreamWaitEvent(st, p->st.join[i], 0));
         }
       } else {
         CSAW_TRY(launch_expand_chunks(L, G, hv, u.d_req, u.d_gs2req, H, E, u.kinds, th));
@@ -340,10 +495,10 @@ static int run_unit(csaw_plan* p, Unit& u, hipStream_t st, TimingHook* th) {
       // one kind's last waves overlap the others' work
       int nk = 0;
       for (int k = 0; k < 3; ++k) nk += u.kinds[k] ? 1 : 0;
-      const bool fan = nk > 1 && p->side[0];
+      const bool fan = nk > 1 && p->fan;
       if (fan) {
-        CSAW_HIP(hipEventRecord(p->fork, st));
-        for (int i = 0; i + 1 < nk; ++i) CSAW_HIP(hipStreamWaitEvent(p->side[i], p->fork, 0));
+        CSAW_HIP(hipEventRecord(p->st.fork, st));
+        for (int i = 0; i + 1 < nk; ++i) CSAW_HIP(hipStreamWaitEvent(p->st.side[i], p->st.fork, 0));
       }
       int next = 0;
       // integer and FP32 kinds first: their chains are the long ones
@@ -362,13 +517,13 @@ static int run_unit(csaw_plan* p, Unit& u, hipStream_t st, TimingHook* th) {
         const int gs = group_size_for(fmax, L.group_min);
         H.only_kind = nk > 1 ? 1 + kind : 0;
         LaunchCfg K = L;
-        if (fan && next > 0) K.stream = p->side[next - 1];
+        if (fan && next > 0) K.stream = p->st.side[next - 1];
         if (th) th->begin(kKernPlain, K.stream);
         CSAW_TRY(launch_expand_plain(K, kind, G, hv, u.d_req, u.d_gs2req, H, u.nmax[h], gs, remap));
         if (th) th->end(kKernPlain, K.stream);
         if (fan && next > 0) {
-          CSAW_HIP(hipEventRecord(p->join[next - 1], K.stream));
-          CSAW_HIP(hipStreamWaitEvent(st, p->join[next - 1], 0));
+          CSAW_HIP(hipEventRecord(p->st.join[next - 1], K.stream));
+          CSAW_HIP(hipStreamWaitEvent(st, p->st.join[next - 1], 0));
         }
         ++next;
       }
@@ -392,8 +547,9 @@ static int run_unit(csaw_plan* p, Unit& u, hipStream_t st, TimingHook* th) {
   return CSAW_OK;
 }
 
-extern "C" int csaw_plan_create(csaw_graph* g, const csaw_request* reqs, int32_t n_req, const csaw_plan_opts* opts,
-                                csaw_plan** out) {
+// stage: leave room for csaw_sample's packed result
+static int plan_create(csaw_graph* g, const csaw_request* reqs, int32_t n_req, const csaw_plan_opts* opts, bool stage,
+                       csaw_plan** out) {
   if (!g || !out || n_req < 0 || (n_req > 0 && !reqs)) return CSAW_ERR_INVALID_ARG;
   *out = nullptr;
   csaw_plan_opts o;
@@ -412,6 +568,7 @@ extern "C" int csaw_plan_create(csaw_graph* g, const csaw_request* reqs, int32_t
   }
   csaw_plan* p = new csaw_plan();
   p->g = g;
+  p->work = g->work;
   p->opts = o;
   p->L.num_cu = g->num_cu;
   if (o.tuning) apply_tuning(p->L, o.tuning);
@@ -430,7 +587,6 @@ extern "C" int csaw_plan_create(csaw_graph* g, const csaw_request* reqs, int32_t
         CSAW_TRY(graph_prepare_vertex_records(g, reqs[i].bias));
       }
       p->reqs.push_back(reqs[i]);
-      p->seeds.emplace_back(reqs[i].seeds, reqs[i].seeds + reqs[i].samples);
       p->reqs.back().seeds = nullptr;
     }
     if (o.mode == CSAW_MODE_BATCHED) {
@@ -442,67 +598,48 @@ extern "C" int csaw_plan_create(csaw_graph* g, const csaw_request* reqs, int32_t
         p->units.back().reqs.push_back(i);
       }
     }
-    int64_t nmax = 1, depth = 1, bin_max = 0;
-    bool several = false;
+    PlanSizes z;
     for (auto& u : p->units) {
       CSAW_TRY(build_unit(p, u));
       for (int64_t v : u.nmax) {
-        nmax = std::max(nmax, v);
+        z.nmax = std::max(z.nmax, v);
         u.bin.push_back(plan_bins_hop(p, u, v));
-        if (u.bin.back()) bin_max = std::max(bin_max, v);
+        if (u.bin.back()) z.bin_max = std::max(z.bin_max, v);
       }
-      several |= u.kinds[0] + u.kinds[1] + u.kinds[2] > 1;
-      depth = std::max<int64_t>(depth, u.depth_max);
+      z.several |= u.kinds[0] + u.kinds[1] + u.kinds[2] > 1;
+      z.depth = std::max<int64_t>(z.depth, u.depth_max);
     }
     p->req_unit.assign(n_req, {-1, -1});
     for (size_t ui = 0; ui < p->units.size(); ++ui)
       for (size_t k = 0; k < p->units[ui].reqs.size(); ++k) p->req_unit[p->units[ui].reqs[k]] = {(int)ui, (int)k};
-    const int64_t nblk = (nmax + kBlockEntries - 1) / kBlockEntries;
-    const int64_t ngrp = (nblk + 1023) / 1024;
-    CSAW_HIP(hipMalloc(&p->local_excl, sizeof(uint32_t) * nmax));
-    CSAW_HIP(hipMalloc(&p->blk_excl, sizeof(uint32_t) * nblk));
-    CSAW_HIP(hipMalloc(&p->grp_excl, sizeof(uint64_t) * ngrp));
-    const size_t state = kCtrBytes + kBoundsBytes * (size_t)n_req;
-    CSAW_HIP(hipMalloc(&p->counters, state));
-    CSAW_HIP(hipMemset(p->counters, 0, state));
-    p->bounds = reinterpret_cast<int64_t*>(reinterpret_cast<char*>(p->counters) + kCtrBytes);
-    p->h_state.assign(state / sizeof(uint32_t), 0u);
-    CSAW_HIP(hipEventCreate(&p->begin));
-    CSAW_HIP(hipEventCreate(&p->end));
-    CSAW_HIP(hipMalloc(&p->totals, sizeof(int64_t) * depth));
-    CSAW_HIP(hipMalloc(&p->bytes_acc, sizeof(unsigned long long) * kNumKernKinds));
-    CSAW_HIP(hipMemset(p->bytes_acc, 0, sizeof(unsigned long long) * kNumKernKinds));
-    if (several) CSAW_HIP(hipMalloc(&p->kind_mask, (nmax + kWave - 1) / kWave));
-    if (bin_max > 0) {
-      const int64_t bblk = (bin_max + kBlockEntries - 1) / kBlockEntries;
-      CSAW_HIP(hipMalloc(&p->order, sizeof(int32_t) * bblk * kBlockEntries));
-      const int64_t waves = (int64_t)p->L.num_cu * p->L.expand_per_cu * 4;
-      p->chunk_cap = (uint32_t)std::min<int64_t>(bblk * kChunksPerBlock + waves, 0xFFFFFFF0LL);
-      CSAW_HIP(hipMalloc(&p->chunks, sizeof(Chunk) * p->chunk_cap));
-      p->queue_cap = p->chunk_cap;
-      CSAW_HIP(hipMalloc(&p->queues, sizeof(uint32_t) * (int64_t)kNumQueues * p->queue_cap));
-      CSAW_HIP(hipMalloc(&p->chosen, p->chunk_cap));
-      if (o.log_chunks) CSAW_HIP(hipMalloc(&p->log, sizeof(ChunkLog) * p->chunk_cap));
+    z.mlp = o.mode == CSAW_MODE_BATCHED && o.sched == CSAW_SCHED_MLP;
+    if (z.mlp && !o.mlp) {
+      set_last_error("CSAW_SCHED_MLP needs a trained csaw_mlp");
+      return CSAW_ERR_INVALID_ARG;
     }
-    if (o.mode == CSAW_MODE_BATCHED) {
-      if (o.sched == CSAW_SCHED_MLP) {
-        if (!o.mlp) {
-          set_last_error("CSAW_SCHED_MLP needs a trained csaw_mlp");
-          return CSAW_ERR_INVALID_ARG;
-        }
-        CSAW_HIP(hipMalloc(&p->d_mlp, sizeof(uint16_t) * kMlpParams));
-        CSAW_TRY(mlp_upload_bf16(o.mlp, p->d_mlp));
-      }
+    if (stage) {
+      // the one request's offsets and edges, if they are worth packing
+      int64_t words = 2 * (int64_t)reqs[0].depth * ((int64_t)reqs[0].samples + 1);
+      for (int64_t c : p->units[0].cap) words += 3 * c;
+      if (words <= kStageWords) z.staging = words;
     }
-    CSAW_HIP(hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking));
-    p->own_stream = true;
-    if (o.mode == CSAW_MODE_BATCHED && !o.serial_expand) {
-      CSAW_HIP(hipEventCreateWithFlags(&p->fork, hipEventDisableTiming));
-      for (int i = 0; i < csaw_plan::kSide; ++i) {
-        CSAW_HIP(hipStreamCreateWithFlags(&p->side[i], hipStreamNonBlocking));
-        CSAW_HIP(hipEventCreateWithFlags(&p->join[i], hipEventDisableTiming));
-      }
-    }
+    size_t filled = 0;
+    Carver size;
+    plan_layout(p, z, size, &filled);
+    CSAW_TRY(p->work->take(size.at, &p->slab));
+    Carver c;
+    c.base = static_cast<char*>(p->slab.p);
+    plan_layout(p, z, c, &filled);
+    p->h_state.assign((kCtrBytes + kBoundsBytes * (size_t)n_req) / sizeof(uint32_t), 0u);
+    if (z.mlp) CSAW_TRY(mlp_upload_bf16(o.mlp, p->d_mlp));
+    CSAW_TRY(p->work->take_streams(o.mode == CSAW_MODE_BATCHED && !o.serial_expand, &p->st));
+    p->stream = p->st.main;
+    p->fan = o.mode == CSAW_MODE_BATCHED && !o.serial_expand;
+    p->busy = true;
+    CSAW_TRY(upload_inputs(p, reqs, filled));
+    // (csaw_sample runs on the same stream and waits there)
+    if (!stage) CSAW_HIP(hipStreamSynchronize(p->stream));
+    p->busy = false;
     p->timer.enabled = o.timing != 0;
     return CSAW_OK;
   };
@@ -515,15 +652,22 @@ extern "C" int csaw_plan_create(csaw_graph* g, const csaw_request* reqs, int32_t
   return CSAW_OK;
 }
 
+extern "C" int csaw_plan_create(csaw_graph* g, const csaw_request* reqs, int32_t n_req, const csaw_plan_opts* opts,
+                                csaw_plan** out) {
+  return plan_create(g, reqs, n_req, opts, false, out);
+}
+
 extern "C" int csaw_plan_run(csaw_plan* p, void* stream, int sync) {
   if (!p) return CSAW_ERR_INVALID_ARG;
   hipStream_t st = stream ? (hipStream_t)stream : p->stream;
   p->hop_logs.clear();
   p->pending_log_hops.clear();
   p->bounds_known = false;
+  const bool was_busy = p->busy;  // (by work on another stream, perhaps)
+  p->busy = true;
   TimingHook* th = p->timer.enabled ? &p->timer : nullptr;
   const bool wait = sync || th;
-  if (wait) CSAW_HIP(hipEventRecord(p->begin, st));
+  if (wait) CSAW_HIP(hipEventRecord(p->st.begin, st));
   if (th) {
     LaunchCfg L = p->L;
     L.stream = st;
@@ -559,12 +703,13 @@ extern "C" int csaw_plan_run(csaw_plan* p, void* stream, int sync) {
     }
   }
   if (wait) {
-    CSAW_HIP(hipEventRecord(p->end, st));
+    CSAW_HIP(hipEventRecord(p->st.end, st));
     CSAW_HIP(hipMemcpyAsync(p->h_state.data(), p->counters, sizeof(uint32_t) * p->h_state.size(), hipMemcpyDeviceToHost,
                             st));
     CSAW_HIP(hipStreamSynchronize(st));
+    p->busy = was_busy;
     float ms = 0.f;
-    CSAW_HIP(hipEventElapsedTime(&ms, p->begin, p->end));
+    CSAW_HIP(hipEventElapsedTime(&ms, p->st.begin, p->st.end));
     p->last_ms = ms;
     if (th) {
       p->timer.collect();
@@ -642,15 +787,12 @@ extern "C" int csaw_plan_copy(const csaw_plan* p, int32_t req, int32_t* src, int
 
 // csaw_plan_copy into device buffers, on the device (for callers that keep
 // the edge lists on the GPU, e.g. as framework tensors).
-extern "C" int csaw_plan_copy_device(const csaw_plan* p, int32_t req, int32_t* src, int32_t* dst, int32_t* sample,
-                                     int64_t* hop_offsets, void* stream, int sync) {
-  if (!p) return CSAW_ERR_INVALID_ARG;
-  std::vector<int64_t> lo, hi;
-  CSAW_TRY(request_bounds(p, req, lo, hi));
+static int copy_edges_device(const csaw_plan* p, int32_t req, const std::vector<int64_t>& lo,
+                             const std::vector<int64_t>& hi, int32_t* src, int32_t* dst, int32_t* sample,
+                             int64_t* hop_offsets, hipStream_t st) {
   const auto [ui, k] = p->req_unit[req];
   const Unit& u = p->units[ui];
   const csaw_request& r = p->reqs[req];
-  hipStream_t st = stream ? (hipStream_t)stream : p->stream;
   CopyArgs A;
   memset(&A, 0, sizeof(A));
   int64_t at = 0;
@@ -671,7 +813,17 @@ extern "C" int csaw_plan_copy_device(const csaw_plan* p, int32_t req, int32_t* s
   A.rows = (int64_t)r.samples + 1;
   A.depth = r.depth;
   A.sub = (int32_t)u.gbase[k];
-  CSAW_TRY(launch_copy_edges(st, A));
+  return launch_copy_edges(st, A);
+}
+
+extern "C" int csaw_plan_copy_device(const csaw_plan* p, int32_t req, int32_t* src, int32_t* dst, int32_t* sample,
+                                     int64_t* hop_offsets, void* stream, int sync) {
+  if (!p) return CSAW_ERR_INVALID_ARG;
+  std::vector<int64_t> lo, hi;
+  CSAW_TRY(request_bounds(p, req, lo, hi));
+  hipStream_t st = stream ? (hipStream_t)stream : p->stream;
+  if (!sync) p->busy = true;
+  CSAW_TRY(copy_edges_device(p, req, lo, hi, src, dst, sample, hop_offsets, st));
   if (sync) CSAW_HIP(hipStreamSynchronize(st));
   return CSAW_OK;
 }
@@ -762,11 +914,32 @@ extern "C" int csaw_plan_destroy(csaw_plan* p) {
 }
 
 // ------------------------------------------------------------ csaw_sample
+// One block of offsets (hop_off), then src, dst and sample columns of n edges.
 struct csaw_edges {
   int32_t depth = 0, samples = 0;
-  std::vector<int32_t> src, dst, smp;
-  std::vector<int64_t> hop_off;
+  int64_t n = 0, n_off = 0;
+  std::unique_ptr<int64_t[]> block;
+  void alloc(int64_t edges, int64_t offsets) {
+    n = edges;
+    n_off = offsets;
+    block.reset(new int64_t[n_off + (3 * n + 1) / 2 + 1]);
+  }
+  int64_t* hop_off() const { return block.get(); }
+  int32_t* col(int c) const { return reinterpret_cast<int32_t*>(block.get() + n_off) + c * n; }
 };
+
+// The request's offsets and columns packed on the device as csaw_edges holds
+// them, then one copy to the host (a copy per hop and column, each its own round
+// trip, took 0.12 ms of a small call).
+static int copy_staged(const csaw_plan* p, const std::vector<int64_t>& lo, const std::vector<int64_t>& hi, csaw_edges* e) {
+  int64_t* off = reinterpret_cast<int64_t*>(p->staging);
+  int32_t* col = reinterpret_cast<int32_t*>(off + e->n_off);
+  CSAW_TRY(copy_edges_device(p, 0, lo, hi, col, col + e->n, col + 2 * e->n, off, p->stream));
+  CSAW_HIP(hipMemcpyAsync(e->block.get(), p->staging, sizeof(int64_t) * e->n_off + 3 * sizeof(int32_t) * e->n,
+                          hipMemcpyDeviceToHost, p->stream));
+  CSAW_HIP(hipStreamSynchronize(p->stream));
+  return CSAW_OK;
+}
 
 extern "C" int csaw_sample(csaw_graph* g, const csaw_params* prm, const int32_t* seeds, csaw_edges** out,
                            csaw_stats* stats) {
@@ -776,26 +949,22 @@ extern "C" int csaw_sample(csaw_graph* g, const csaw_params* prm, const int32_t*
     // FrontierSize > 1 runs the multi-dimensional random walk, as Sampler()
     // dispatches check_layer (main.cu:285-287); the result is one layer.
     if (prm->samples < 0 || prm->depth < 0 || (prm->samples > 0 && !seeds)) return CSAW_ERR_INVALID_ARG;
+    const size_t cap = std::max<size_t>((size_t)prm->samples * prm->depth, 1);
+    std::vector<int32_t> src(cap), dst(cap);
+    std::vector<int64_t> off((size_t)prm->samples + 1);
+    csaw_stats st;
+    CSAW_TRY(csaw_mdrw(g, prm->seed, prm->request_id, prm->samples, prm->frontier_size, prm->depth, seeds, src.data(),
+                       dst.data(), off.data(), &st));
     csaw_edges* e = new csaw_edges();
     e->depth = 1;
     e->samples = prm->samples;
-    const size_t cap = std::max<size_t>((size_t)prm->samples * prm->depth, 1);
-    e->src.resize(cap);
-    e->dst.resize(cap);
-    e->hop_off.resize((size_t)prm->samples + 1);
-    csaw_stats st;
-    int rc = csaw_mdrw(g, prm->seed, prm->request_id, prm->samples, prm->frontier_size, prm->depth, seeds,
-                       e->src.data(), e->dst.data(), e->hop_off.data(), &st);
-    if (rc != CSAW_OK) {
-      delete e;
-      return rc;
+    e->alloc(off[prm->samples], prm->samples + 1);
+    memcpy(e->hop_off(), off.data(), sizeof(int64_t) * off.size());
+    if (e->n > 0) {
+      memcpy(e->col(0), src.data(), sizeof(int32_t) * e->n);
+      memcpy(e->col(1), dst.data(), sizeof(int32_t) * e->n);
     }
-    const int64_t n = e->hop_off[prm->samples];
-    e->src.resize(n);
-    e->dst.resize(n);
-    e->smp.resize(n);
-    for (int32_t s = 0; s < prm->samples; ++s)
-      for (int64_t i = e->hop_off[s]; i < e->hop_off[s + 1]; ++i) e->smp[i] = s;
+    for (int32_t s = 0; s < prm->samples; ++s) std::fill(e->col(2) + off[s], e->col(2) + off[s + 1], s);
     if (stats) *stats = st;
     *out = e;
     return CSAW_OK;
@@ -825,26 +994,26 @@ extern "C" int csaw_sample(csaw_graph* g, const csaw_params* prm, const int32_t*
     o.tuning = &t;
   }
   csaw_plan* p = nullptr;
-  CSAW_TRY(csaw_plan_create(g, &r, 1, &o, &p));
+  CSAW_TRY(plan_create(g, &r, 1, &o, true, &p));
   int st = csaw_plan_run(p, nullptr, 1);
   csaw_edges* e = nullptr;
   if (st == CSAW_OK) {
     e = new csaw_edges();
     e->depth = r.depth;
     e->samples = r.samples;
-    int64_t n = 0;
-    st = csaw_plan_request_info(p, 0, &n);
+    std::vector<int64_t> lo, hi;
+    st = request_bounds(p, 0, lo, hi);
     if (st == CSAW_OK) {
-      e->src.resize(n);
-      e->dst.resize(n);
-      e->smp.resize(n);
-      e->hop_off.resize((size_t)r.depth * (r.samples + 1));
-      st = csaw_plan_copy(p, 0, e->src.data(), e->dst.data(), e->smp.data(), e->hop_off.data());
-    }
-    if (st == CSAW_OK && stats) {
-      memset(stats, 0, sizeof(*stats));
-      stats->edges = n;
-      stats->kernel_ms = p->last_ms;
+      int64_t n = 0;
+      for (int32_t h = 0; h < r.depth; ++h) n += hi[h] - lo[h];
+      e->alloc(n, (int64_t)r.depth * ((int64_t)r.samples + 1));
+      st = p->staging ? copy_staged(p, lo, hi, e)
+                      : csaw_plan_copy(p, 0, e->col(0), e->col(1), e->col(2), e->hop_off());
+      if (st == CSAW_OK && stats) {
+        memset(stats, 0, sizeof(*stats));
+        stats->edges = n;
+        stats->kernel_ms = p->last_ms;
+      }
     }
   }
   csaw_plan_destroy(p);
@@ -858,7 +1027,7 @@ extern "C" int csaw_sample(csaw_graph* g, const csaw_params* prm, const int32_t*
 
 extern "C" int csaw_edges_info(const csaw_edges* e, int64_t* n_edges, int32_t* depth, int32_t* samples) {
   if (!e) return CSAW_ERR_INVALID_ARG;
-  if (n_edges) *n_edges = (int64_t)e->src.size();
+  if (n_edges) *n_edges = e->n;
   if (depth) *depth = e->depth;
   if (samples) *samples = e->samples;
   return CSAW_OK;
@@ -866,10 +1035,10 @@ extern "C" int csaw_edges_info(const csaw_edges* e, int64_t* n_edges, int32_t* d
 
 extern "C" int csaw_edges_copy(const csaw_edges* e, int32_t* src, int32_t* dst, int32_t* sample, int64_t* hop_offsets) {
   if (!e) return CSAW_ERR_INVALID_ARG;
-  if (src && !e->src.empty()) memcpy(src, e->src.data(), sizeof(int32_t) * e->src.size());
-  if (dst && !e->dst.empty()) memcpy(dst, e->dst.data(), sizeof(int32_t) * e->dst.size());
-  if (sample && !e->smp.empty()) memcpy(sample, e->smp.data(), sizeof(int32_t) * e->smp.size());
-  if (hop_offsets && !e->hop_off.empty()) memcpy(hop_offsets, e->hop_off.data(), sizeof(int64_t) * e->hop_off.size());
+  int32_t* out[3] = {src, dst, sample};
+  for (int c = 0; c < 3; ++c)
+    if (out[c] && e->n > 0) memcpy(out[c], e->col(c), sizeof(int32_t) * e->n);
+  if (hop_offsets && e->n_off > 0) memcpy(hop_offsets, e->hop_off(), sizeof(int64_t) * e->n_off);
   return CSAW_OK;
 }
 
@@ -881,10 +1050,13 @@ extern "C" int csaw_edges_from_host(int32_t depth, int32_t samples, int64_t n, c
   csaw_edges* e = new csaw_edges();
   e->depth = depth;
   e->samples = samples;
-  e->src.assign(src, src + n);
-  e->dst.assign(dst, dst + n);
-  e->smp.assign(smp, smp + n);
-  if (hop_off) e->hop_off.assign(hop_off, hop_off + (size_t)depth * (samples + 1));
+  e->alloc(n, hop_off ? (int64_t)depth * (samples + 1) : 0);
+  if (n > 0) {
+    memcpy(e->col(0), src, sizeof(int32_t) * n);
+    memcpy(e->col(1), dst, sizeof(int32_t) * n);
+    memcpy(e->col(2), smp, sizeof(int32_t) * n);
+  }
+  if (e->n_off > 0) memcpy(e->hop_off(), hop_off, sizeof(int64_t) * e->n_off);
   *out = e;
   return CSAW_OK;
 }

@@ -48,6 +48,7 @@ struct Unit {
   std::vector<int64_t> cap;     // per hop: edge capacity
   std::vector<int64_t> nmax;    // per hop: frontier entries upper bound
   std::vector<char> bin;        // per hop: binned into chunks (plan_bins_hop)
+  std::vector<ReqDev> rd;       // the requests as the device sees them
   ReqDev* d_req = nullptr;
   int32_t* d_gs2req = nullptr;
   int32_t* d_fv0 = nullptr;
@@ -74,7 +75,6 @@ int mlp_upload_bf16(const csaw_mlp* m, uint16_t* dst);
 struct csaw_plan {
   csaw_graph* g = nullptr;
   std::vector<csaw_request> reqs;
-  std::vector<std::vector<int32_t>> seeds;
   std::vector<std::pair<int, int>> req_unit;  // (unit, index in unit)
   csaw_plan_opts opts;
   std::vector<csaw::Unit> units;
@@ -85,6 +85,12 @@ struct csaw_plan {
   uint64_t* grp_excl = nullptr;
   csaw::Chunk* chunks = nullptr;
   uint32_t chunk_cap = 0;
+  // every device array below and the units' (one allocation), its work waited for
+  // by the calls themselves unless busy
+  std::shared_ptr<csaw::Workspace> work;
+  csaw::Workspace::Block slab;
+  mutable bool busy = false;
+  int32_t* staging = nullptr;         // csaw_sample: the result, packed for one copy
   // counter block, then the requests' edge bounds (kCtrBytes + n_req *
   // kBoundsBytes): one copy into h_state after a synchronised run brings the
   // overflow flag and every request's place to the host
@@ -100,18 +106,13 @@ struct csaw_plan {
   uint16_t* d_mlp = nullptr;
   unsigned long long* bytes_acc = nullptr;  // algorithmic bytes per kernel kind (timing runs)
   csaw::LaunchCfg L;
+  csaw::PlanStreams st;   // main stream; batched: side streams the expansion
+                          // kernels of a hop fan out to, joined before the next hop
   hipStream_t stream = nullptr;
-  bool own_stream = false;
+  bool fan = false;       // this plan uses the side streams
   hipGraphExec_t gexec = nullptr;
   hipStream_t graph_stream = nullptr;
-  // batched mode: side streams the expansion kernels of a hop fan out to
-  // (joined back before the next hop), fork / join events
-  static constexpr int kSide = 3;
-  hipStream_t side[kSide] = {};
-  hipEvent_t fork = nullptr;
-  hipEvent_t join[kSide] = {};
   csaw::EventTimer timer;
-  hipEvent_t begin = nullptr, end = nullptr;  // of a synchronised run
   double last_ms = 0.0;
   int64_t runs = 0;
   std::vector<csaw::HopLog> hop_logs;
