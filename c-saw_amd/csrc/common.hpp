@@ -77,6 +77,13 @@ struct GraphDev {
   const int32_t* hub_vid;       // sorted ids of vertices with degree > kHubMin
   const int64_t* hub_pool;      // pool offset per hub (n_hubs + 1)
   const uint64_t* hub_cdf[2];   // [DEGREE, USER]: inclusive uint64 CDFs of hubs
+  // the DEGREE hub CDFs as uint32 with their 16-ary index (hub_entries of them),
+  // and no vertex of degree <= kHubMin can total 2^32 either: integer CDFs are
+  // built and searched with 32-bit keys (null: some total may not fit)
+  const uint32_t* hub_cdf32;
+  const uint32_t* hub_idx32;
+  int64_t hub_entries;
+  int32_t build32;
   const uint64_t* int_cdf[2];   // full per-entry CDF cache (null when not used)
   const float* cdf_idx;         // 16-ary search index over cdf (null when not used)
   const uint64_t* int_idx[2];   // 16-ary search indexes over int_cdf

@@ -311,6 +311,8 @@ static int ensure_hub_list(csaw_graph* g) {
   return CSAW_OK;
 }
 
+static int narrow_hubs(csaw_graph* g);
+
 int graph_prepare_bias(csaw_graph* g, int32_t bias) {
   if (bias == CSAW_BIAS_WEIGHT) {
     if (!g->w) {
@@ -340,11 +342,15 @@ int graph_prepare_bias(csaw_graph* g, int32_t bias) {
   if (bias != CSAW_BIAS_DEGREE && bias != CSAW_BIAS_USER) return CSAW_OK;
   const int kind = bias == CSAW_BIAS_DEGREE ? 0 : 1;
   CSAW_TRY(ensure_hub_list(g));
+  // degree totals up to kHubMin neighbours fit 32 bits (hubs are looked at below)
+  const bool fits = kind == 0 && !g->wide_int_cdf && g->max_deg * (int64_t)kHubMin < ((int64_t)1 << 32);
+  if (fits && g->n_hubs == 0) g->build32 = true;
   if (g->hub_cdf[kind] || g->n_hubs == 0) return CSAW_OK;
   std::vector<int64_t> pool(g->n_hubs + 1);
   CSAW_HIP(hipMemcpy(pool.data(), g->hub_pool, sizeof(int64_t) * pool.size(), hipMemcpyDeviceToHost));
   CSAW_HIP(hipMalloc(&g->hub_cdf[kind], sizeof(uint64_t) * g->hub_entries));
   CSAW_TRY(hub_cdf_build(g->view(), g->hook_view(), kind, pool, g->hub_cdf[kind], g->stream, g->num_cu));
+  if (fits) CSAW_TRY(narrow_hubs(g));
   CSAW_HIP(hipStreamSynchronize(g->stream));
   return CSAW_OK;
 }
@@ -530,6 +536,33 @@ static int build_index(const T* C, int64_t E, T** out, hipStream_t stream, int n
   return CSAW_OK;
 }
 
+// The DEGREE hub CDFs as uint32, padded and indexed like the CDF cache, when
+// their totals fit (duplicate neighbours can total more than E).
+static int narrow_hubs(csaw_graph* g) {
+  const int64_t n = g->hub_entries, npad = pad16(n);
+  unsigned long long* d_max = nullptr;
+  CSAW_HIP(hipMalloc(&d_max, sizeof(unsigned long long)));
+  unsigned long long mx = 0;
+  auto body = [&]() -> int {
+    CSAW_HIP(hipMemsetAsync(d_max, 0, sizeof(unsigned long long), g->stream));
+    k_max_u64<<<grid_for(n, 256, g->num_cu), 256, 0, g->stream>>>(g->hub_cdf[0], n, d_max);
+    CSAW_LAUNCH_CHECK();
+    CSAW_HIP(hipMemcpyAsync(&mx, d_max, sizeof(mx), hipMemcpyDeviceToHost, g->stream));
+    CSAW_HIP(hipStreamSynchronize(g->stream));
+    if (mx >= (1ull << 32)) return CSAW_OK;
+    CSAW_HIP(hipMalloc(&g->hub_cdf32, sizeof(uint32_t) * npad));
+    CSAW_HIP(hipMemsetAsync(g->hub_cdf32, 0, sizeof(uint32_t) * npad, g->stream));
+    k_narrow_u32<<<grid_for(n, 256, g->num_cu), 256, 0, g->stream>>>(g->hub_cdf[0], n, g->hub_cdf32);
+    CSAW_LAUNCH_CHECK();
+    CSAW_TRY(build_index<uint32_t>(g->hub_cdf32, n, &g->hub_idx32, g->stream, g->num_cu));
+    g->build32 = true;
+    return CSAW_OK;
+  };
+  const int st = body();
+  (void)hipFree(d_max);
+  return st;
+}
+
 template <typename T>
 __global__ void k_vertex_records(const int64_t* __restrict__ off, const T* __restrict__ C, int64_t V,
                                  VertexRecord* __restrict__ out) {
@@ -595,6 +628,10 @@ csaw::GraphDev csaw_graph::view(bool use_cache) const {
   G.hub_pool = hub_pool;
   G.hub_cdf[0] = hub_cdf[0];
   G.hub_cdf[1] = hub_cdf[1];
+  G.hub_cdf32 = hub_cdf32;
+  G.hub_idx32 = hub_idx32;
+  G.hub_entries = hub_entries;
+  G.build32 = build32 ? 1 : 0;
   G.int_cdf[0] = use_cache ? int_cdf[0] : nullptr;
   G.int_cdf[1] = use_cache ? int_cdf[1] : nullptr;
   // an integer cache is searched through its index: both or neither
@@ -635,6 +672,8 @@ static void graph_free(csaw_graph* g) {
   (void)hipFree(g->hub_pool);
   (void)hipFree(g->hub_cdf[0]);
   (void)hipFree(g->hub_cdf[1]);
+  (void)hipFree(g->hub_cdf32);
+  (void)hipFree(g->hub_idx32);
   (void)hipFree(g->int_cdf[0]);
   (void)hipFree(g->int_cdf[1]);
   (void)hipFree(g->int_idx[0]);

@@ -59,6 +59,9 @@ struct csaw_graph {
   int32_t* hub_vid = nullptr;
   int64_t* hub_pool = nullptr;  // n_hubs+1 pool offsets
   uint64_t* hub_cdf[2] = {nullptr, nullptr};  // [DEGREE, USER]
+  uint32_t* hub_cdf32 = nullptr;              // DEGREE, when every total fits
+  uint32_t* hub_idx32 = nullptr;
+  bool build32 = false;                       // see GraphDev
   uint64_t* int_cdf[2] = {nullptr, nullptr};  // full per-entry CDF cache [DEGREE, USER]
   // 16-ary search indexes over cdf and int_cdf (CDF arrays padded to 16)
   float* cdf_idx = nullptr;

@@ -411,13 +411,18 @@ static HopDev make_hop(csaw_plan* p, Unit& u, int h) {
 // several XCDs, which cost more than the variants gained wherever no entry has a
 // CDF to build: 256 mixed requests over RMAT-22 take 22.7 ms binned, 17.3 ms in
 // frontier order, 8 of 64 to 1,024 seeds 0.89 and 0.41.  Binning stays for integer
-// biases without a 32-bit CDF cache (the workgroup variants share the builds),
-// and for what asks for chunks: forced and random variants, chunk logs.
+// biases whose CDFs neither a 32-bit cache holds nor a group's wave builds (the
+// workgroup variants share those builds), and for what asks for chunks: forced and random variants, chunk logs.
 static bool plan_bins_hop(const csaw_plan* p, const Unit& u, int64_t nmax) {
   if (p->opts.mode != CSAW_MODE_BATCHED) return false;
   if (p->opts.log_chunks || (p->opts.sched != CSAW_SCHED_HEURISTIC && p->opts.sched != CSAW_SCHED_MLP)) return true;
   if (nmax <= kSmallHopEntries) return false;
-  return u.kinds[kInt] && !(p->opts.cdf_cache && !p->g->int_cdf[0] && !p->g->int_cdf[1]);
+  if (!u.kinds[kInt]) return false;
+  if (p->opts.cdf_cache) return p->g->int_cdf[0] || p->g->int_cdf[1];
+  if (!p->g->build32 || u.remap) return true;
+  for (int ri : u.reqs)
+    if (p->reqs[ri].bias == CSAW_BIAS_USER) return true;
+  return false;
 }
 
 static int run_unit(csaw_plan* p, Unit& u, hipStream_t st, TimingHook* th) {
@@ -506,10 +511,11 @@ static int run_unit(csaw_plan* p, Unit& u, hipStream_t st, TimingHook* th) {
         if (!u.kinds[kind]) continue;
         // sub-wave group size from the largest fanout of the kind's requests
         int fmax = 0;
-        bool remap = false;
+        bool remap = false, user = false;
         for (int ri : u.reqs) {
           const csaw_request& r = p->reqs[ri];
           if (r.depth > h && bias_kind(r.bias) == kind) {
+            user |= r.bias == CSAW_BIAS_USER;
             fmax = std::max(fmax, r.fanouts[h]);
             remap |= r.dedup == 2;
           }
@@ -519,7 +525,7 @@ static int run_unit(csaw_plan* p, Unit& u, hipStream_t st, TimingHook* th) {
         LaunchCfg K = L;
         if (fan && next > 0) K.stream = p->st.side[next - 1];
         if (th) th->begin(kKernPlain, K.stream);
-        CSAW_TRY(launch_expand_plain(K, kind, G, hv, u.d_req, u.d_gs2req, H, u.nmax[h], gs, remap));
+        CSAW_TRY(launch_expand_plain(K, kind, G, hv, u.d_req, u.d_gs2req, H, u.nmax[h], gs, remap, user));
         if (th) th->end(kKernPlain, K.stream);
         if (fan && next > 0) {
           CSAW_HIP(hipEventRecord(p->st.join[next - 1], K.stream));

@@ -357,16 +357,16 @@ __global__ void k_fill_u32(uint32_t* __restrict__ p, uint32_t v, int64_t n) {
 // the CDF cache and its 16-ary index (searched through the index).  KEYS:
 // kKeys32 when no integer cache of the view is 64-bit (the 64-bit searches
 // compiled out of the group path).
-constexpr int64_t kWideHopEntries = 16384;
+constexpr int64_t kWideHopEntries = 131072;  // entries times the groups a wave would hold
 // REMAP: the hop's requests of this kind use the region-remap mode.
 // The group-only builds are held to 128 registers, four waves per SIMD: their
 // waves wait for memory most of the time (FP32 {15, 10, 5} from 30,011 seeds:
 // 645 us at three waves, 565 us at four).
-template <int KIND, bool IDX, int KEYS, bool REMAP = false>
+template <int KIND, bool IDX, int KEYS, bool REMAP = false, bool BUILD = false>
 __global__ __launch_bounds__(256, KEYS == kKeys32 && !REMAP ? 4 : 1) void k_expand_plain(GraphDev G, csaw_graph_view hv, const ReqDev* __restrict__ R,
                                                       const int32_t* __restrict__ gs2req, HopDev H, int hop_gs) {
-  constexpr bool kGroupOk = KIND != kInt || IDX;  // no per-entry CDF build needed
-  constexpr bool kGroupLds = KIND == kF32 || (KIND == kInt && IDX);  // small cached CDFs staged in LDS
+  constexpr bool kGroupOk = KIND != kInt || IDX || BUILD;  // no per-entry CDF build needed, or built by the batch
+  constexpr bool kGroupLds = KIND == kF32 || (KIND == kInt && (IDX || BUILD));  // small cached CDFs staged in LDS
   // (32-bit-key builds are always given a group size: the whole-wave path and
   // its 40 KB of LDS per workgroup are left out)
   constexpr bool kGroupOnly = kGroupOk && KEYS == kKeys32;
@@ -377,12 +377,13 @@ __global__ __launch_bounds__(256, KEYS == kKeys32 && !REMAP ? 4 : 1) void k_expa
   const int64_t n = *H.n_ptr;
   const int wid = threadIdx.x / kWave;
   const int64_t nw = (int64_t)gridDim.x * 4;
-  // A small hop gives each entry a whole wave: what it waits for are the few
-  // slots with many redraws, and 64 attempts a round end those sooner.  (Uniform
-  // draws collide too rarely for that: groups throughout.)  Region remap of 8,191
-  // seeds on RMAT-22: 813 us in groups, 681 us; FP32 {10, 10} from 10,000 on
-  // RMAT-20 150 and 140 us; from 30,011 seeds on no difference.
-  const int gs = hop_gs > 0 && KIND != kUniform && n <= kWideHopEntries ? kWave : hop_gs;
+  // A hop that leaves the groups few entries each gives every entry a whole wave:
+  // what it waits for are the few slots with many redraws, and 64 attempts a round
+  // end those sooner.  (Uniform draws collide too rarely for that: groups
+  // throughout.)  On RMAT-22, groups and whole waves: region remap of 8,191 seeds
+  // {10, 10} 813 and 681 us, degree bias {25, 10} from 40,000 with the CDF cache
+  // 608 and 543 us, without 870 and 794; beyond the line the groups are level.
+  const int gs = hop_gs > 0 && KIND != kUniform && n * (kWave / hop_gs) <= kWideHopEntries ? kWave : hop_gs;
   // batch size adapts to the frontier: one entry (one group round) per wave
   // when it is small (all waves busy), up to 64 entries per metadata round
   // when it is large
@@ -397,8 +398,8 @@ __global__ __launch_bounds__(256, KEYS == kKeys32 && !REMAP ? 4 : 1) void k_expa
     }
     if constexpr (kGroupOk) {
       if (grp) {
-        group_expand_batch<KIND, KEYS, REMAP>(G, hv, R, gs2req, H, nullptr, e0, cnt, gs, glds + wid * kGroupStride,
-                                              kGroupLds);
+        group_expand_batch<KIND, KEYS, REMAP, BUILD>(G, hv, R, gs2req, H, nullptr, e0, cnt, gs,
+                                                     glds + wid * kGroupStride, kGroupLds);
         continue;
       }
     }
@@ -893,14 +894,25 @@ int launch_fill(const LaunchCfg& L, uint32_t* p, uint32_t v, int64_t n) {
   return CSAW_OK;
 }
 
-int launch_expand_plain(const LaunchCfg& L, int kind, const GraphDev& G, const csaw_graph_view& hv, const ReqDev* R,
-                        const int32_t* gs2req, const HopDev& H, int64_t max_entries, int gs, bool remap) {
+int launch_expand_plain(const LaunchCfg& L, int kind, const GraphDev& graph, const csaw_graph_view& hv, const ReqDev* R,
+                        const int32_t* gs2req, const HopDev& H, int64_t max_entries, int gs, bool remap, bool user) {
+  GraphDev G = graph;
   int64_t nwg = (max_entries + 3) / 4;
   int grid = (int)std::max<int64_t>(1, std::min<int64_t>(nwg, grid_of(L, L.frontier_per_cu)));
   if (L.grid_override > 0) grid = L.grid_override;
   // the CDF cache (and its index) is in the view: plain sampling with cdf_cache
   const bool idx = G.cdf_idx || G.int_idx32[0] || G.int_idx32[1] || G.int_idx[0] || G.int_idx[1];
   const bool wide = G.int_cdf[0] || G.int_cdf[1];  // a 64-bit integer cache in the view
+  // degree bias with CDFs built by the batch: the hubs' array in the cache's
+  // place.  A hop of whole waves gains nothing from it (a wave per entry builds as
+  // fast: 8,192 seeds {25, 10} on RMAT-20 229 us so, 252 us through the batch).
+  const bool build = kind == kInt && !idx && !wide && !remap && !user && G.build32 &&
+                     max_entries * (kWave / gs) > kWideHopEntries;
+  if (build) {
+    G.int_cdf32[0] = G.hub_cdf32;
+    G.int_idx32[0] = G.hub_idx32;
+    G.E = G.hub_entries;
+  }
   auto go = [&](auto kern, int group) { kern<<<grid, 256, 0, L.stream>>>(G, hv, R, gs2req, H, group); };
   if (kind == kUniform) {
     if (remap) go(k_expand_plain<kUniform, false, kKeys32, true>, gs);
@@ -910,6 +922,7 @@ int launch_expand_plain(const LaunchCfg& L, int kind, const GraphDev& G, const c
     if (idx && !wide && remap) go(k_expand_plain<kInt, true, kKeys32, true>, gs);
     else if (idx && !wide) go(k_expand_plain<kInt, true, kKeys32>, gs);
     else if (idx) go(k_expand_plain<kInt, true, kKeysAny>, remap ? 0 : gs);
+    else if (build) go(k_expand_plain<kInt, false, kKeys32, false, true>, gs);
     else go(k_expand_plain<kInt, false, kKeysAny>, 0);
   } else if (remap) {
     if (idx) go(k_expand_plain<kF32, true, kKeys32, true>, gs);

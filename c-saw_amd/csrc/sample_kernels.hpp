@@ -108,8 +108,10 @@ int launch_copy_edges(hipStream_t st, const CopyArgs& A);
 int launch_fill(const LaunchCfg& L, uint32_t* p, uint32_t v, int64_t n);
 int launch_digest(hipStream_t st, int num_cu, const int32_t* src, const int32_t* dst, const int32_t* smp, int64_t lo,
                   int64_t hi, int64_t pos0, int64_t gbase, unsigned long long* out);
+// user: some request of an integer kind uses the user hooks
 int launch_expand_plain(const LaunchCfg& L, int kind, const GraphDev& G, const csaw_graph_view& hv, const ReqDev* R,
-                        const int32_t* gs2req, const HopDev& H, int64_t max_entries, int gs, bool remap);
+                        const int32_t* gs2req, const HopDev& H, int64_t max_entries, int gs, bool remap,
+                        bool user);
 int launch_choose(const LaunchCfg& L, const ChooseArgs& A, const HopDev& H, int64_t max_chunks);
 int launch_expand_list(const LaunchCfg& L, int kind, const GraphDev& G, const csaw_graph_view& hv, const ReqDev* R,
                        const int32_t* gs2req, const HopDev& H, const int32_t* list, int64_t n);

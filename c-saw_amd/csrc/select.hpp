@@ -583,8 +583,10 @@ __device__ __forceinline__ U4 gdraw(const GEntry& en, int j, int a) {
 // which frees their registers).
 enum GroupKeys { kKeysAny = 0, kKeys32 = 1 };
 
+// co: where the entry's CDF starts in the array searched (its offset, unless the
+// array holds the hubs only)
 template <int KIND, int KEYS = kKeysAny>
-__device__ __forceinline__ int32_t gpick(const GraphDev& G, const GEntry& en, const U4& r) {
+__device__ __forceinline__ int32_t gpick(const GraphDev& G, const GEntry& en, int64_t co, const U4& r) {
   const uint32_t mode = (en.flags >> 4) & 15u;
   const uint64_t t = philox_t64(r);
   if (KIND == kUniform || mode == kPickUniform) return (int32_t)mulhi64_32(t, (uint32_t)en.d);
@@ -596,7 +598,7 @@ __device__ __forceinline__ int32_t gpick(const GraphDev& G, const GEntry& en, co
   const bool user = (en.flags >> 1) & 1u;
   if (KEYS == kKeys32 || mode == kPickInt32Idx)  // uint32 cache: T < 2^32
     return cdf_index_search<uint32_t>(user ? G.int_cdf32[1] : G.int_cdf32[0], user ? G.int_idx32[1] : G.int_idx32[0],
-                                      G.E, en.o, en.d, (uint32_t)mulhi64_32(t, (uint32_t)en.T));
+                                      G.E, co, en.d, (uint32_t)mulhi64_32(t, (uint32_t)en.T));
   const uint64_t x = mulhi64(t, en.T);
   const uint64_t* C = user ? G.int_cdf[1] : G.int_cdf[0];
   if (mode == kPickIntIdx)
@@ -780,13 +782,14 @@ __device__ __forceinline__ int32_t resolve_slots(int F, int32_t d, int gs, int g
 // 170 for fanout 10, 256 for 16 and 512 for 32 lanes.
 constexpr int kGroupSmallCap = 64;  // slot words at the smallest group size
 
+// base: added to integer targets (a CDF that runs on from the one before it)
 template <int KIND>
-__device__ __forceinline__ int32_t gpick_small(const GEntry& en, const uint32_t* lc, const U4& r) {
+__device__ __forceinline__ int32_t gpick_small(const GEntry& en, const uint32_t* lc, uint32_t base, const U4& r) {
   if constexpr (KIND == kF32) {
     const float x = __fmul_rn(philox_u24(r), __uint_as_float((uint32_t)en.T));
     return (int32_t)upper_bound_dev<float>(reinterpret_cast<const float*>(lc), en.d, x);
   } else {
-    const uint32_t x = (uint32_t)mulhi64_32(philox_t64(r), (uint32_t)en.T);  // uint32 cache: T < 2^32
+    const uint32_t x = (uint32_t)mulhi64_32(philox_t64(r), (uint32_t)en.T) + base;  // T < 2^32
     return (int32_t)upper_bound_dev<uint32_t>(lc, en.d, x);
   }
 }
@@ -852,18 +855,35 @@ __device__ __forceinline__ int32_t group_select_remap(const GraphDev& G, const G
 // lc: the group's LDS slot of cap words (null: no small path)
 // gs: group size (4 .. 32, or 64), a run-time value so one build serves all;
 // the group is lanes gbase .. gbase + gs - 1 (gmask)
-template <int KIND, int KEYS, bool REMAP>
-__device__ int32_t group_select(const GraphDev& G, const GEntry& en, int gs, int gl, int gbase, uint64_t gmask,
+// BUILD: lc is the wave's run of built CDFs, the entry's place in it (or its
+// CDF's place among the hubs') the upper half of T.
+template <int KIND, int KEYS, bool REMAP, bool BUILD>
+__device__ int32_t group_select(const GraphDev& G, GEntry en, int gs, int gl, int gbase, uint64_t gmask,
                                 uint32_t* lc, int cap, int32_t* cl, uint32_t* bits, bool defer) {
   const int F = en.F;
   const int32_t d = en.d;
   const bool act = gl < F;
   const uint32_t mode = (en.flags >> 4) & 15u;
-  const bool small = KIND != kUniform && lc && d <= cap &&
-                     (mode == kPickInt32Idx || mode == kPickF32 || mode == kPickF32Idx);
+  bool small = KIND != kUniform && lc && d <= cap &&
+               (mode == kPickInt32Idx || mode == kPickF32 || mode == kPickF32Idx);
   if constexpr (REMAP)
     if (en.flags & 4u) return group_select_remap<KIND>(G, en, gs, gl, gbase, gmask, lc, small, defer);
-  if (small) {
+  uint32_t base = 0;
+  int64_t co = en.o;
+  if constexpr (BUILD) {
+    const uint32_t at = (uint32_t)(en.T >> 32);
+    co = at;
+    small = mode == kPickLds;
+    if (small) {
+      lc += at;
+      base = at ? lc[-1] : 0u;
+      en.T = lc[d - 1] - base;
+      if (en.T == 0) {  // all-zero biases: uniform
+        small = false;
+        en.flags &= ~0xF0u;
+      }
+    }
+  } else if (small) {
     const uint32_t* C = KIND == kF32 ? reinterpret_cast<const uint32_t*>(G.cdf)
                                      : ((en.flags >> 1) & 1u ? G.int_cdf32[1] : G.int_cdf32[0]);
     for (int i = gl; i < d; i += gs) lc[i] = C[en.o + i];
@@ -872,8 +892,10 @@ __device__ int32_t group_select(const GraphDev& G, const GEntry& en, int gs, int
   // one draw (slot j, attempt a); only `valid` lanes' results are used
   auto pick = [&](int j, int a, bool valid) -> int32_t {
     if (!valid) return 0;
-    if (small) return gpick_small<KIND>(en, lc, gdraw(en, j, a));
-    return gpick<KIND, KEYS>(G, en, gdraw(en, j, a));
+    if (small) return gpick_small<KIND>(en, lc, base, gdraw(en, j, a));
+    if (BUILD && ((en.flags >> 4) & 15u) == kPickUniform)
+      return (int32_t)mulhi64_32(philox_t64(gdraw(en, j, a)), (uint32_t)d);
+    return gpick<KIND, KEYS>(G, en, co, gdraw(en, j, a));
   };
   int32_t cand = pick(gl, 0, act);
   if (!act) cand = -1;
@@ -896,8 +918,67 @@ constexpr int kCandSlotWords = 128;
 constexpr int kGroupBaseWords = kWave * 16 + kCandSlotWords + 4 * (kWave / kGroupMin) + 4;
 constexpr int kGroupWords = kGroupBaseWords + kGroupLdsWords;
 
+// Degree CDFs of the entries from rank `done` on, as many as fit the wave's
+// kGroupLdsWords words, built one after another by the whole wave: lane s of a
+// row takes element s of their lists laid end to end (its entry found by a
+// binary search over the running degrees), and one running scan of the biases
+// serves them all, an entry's CDF being what the run adds from its start on.
+// Returns how many entries of the batch are ready: the built ones, and those
+// that need no build among them.
+// Bound: the lists' loads and the degree gathers; a wave per entry built them
+// one after another, 64 lanes on lists of 20 and a binary search over 64-bit keys
+// for the hubs: 40,000 seeds of fanouts {25, 10} on RMAT-22 969 us a run with that,
+// 797 us with this.
+__device__ __forceinline__ int build_degree_cdfs(const GraphDev& G, int4* ents, int done, int nsel, uint32_t* run) {
+  const int lane = lane_id();
+  const int r = done + lane;
+  uint32_t dd = 0;
+  int64_t o = 0;
+  if (r < nsel) {
+    const int4 a = ents[4 * r], b = ents[4 * r + 1];
+    o = pack_i64(a.z, a.w);
+    if ((((uint32_t)ents[4 * r + 2].w >> 4) & 15u) == kPickLds) dd = (uint32_t)b.x;
+  }
+  const uint32_t incl = wave_incl_scan_u32(dd);
+  const int ready = __popcll(ballot(r < nsel && incl <= (uint32_t)kGroupLdsWords));
+  const uint32_t total = readlane_u(incl, ready - 1);
+  if (lane < ready && dd) ents[4 * r + 3].w = (int)(incl - dd);
+  constexpr int kRows = 4;
+  uint32_t acc = 0;
+  for (uint32_t s0 = 0; s0 < total; s0 += kRows * kWave) {
+    int32_t u[kRows];
+    uint32_t w[kRows];
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) {
+      const uint32_t s = s0 + k * kWave + lane;
+      int L = 0;  // first lane whose running degree exceeds s
+#pragma unroll
+      for (int b = 32; b >= 1; b >>= 1)
+        if (shfl_abs_u(incl, L + b - 1) <= s) L += b;
+      L = L < kWave ? L : kWave - 1;
+      const uint32_t start = shfl_abs_u(incl, L) - shfl_abs_u(dd, L);
+      const int64_t ol = (int64_t)shfl_abs_u64((uint64_t)o, L);
+      u[k] = s < total ? G.adj[ol + (int64_t)(s - start)] : -1;
+    }
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) w[k] = u[k] >= 0 ? (uint32_t)G.deg[u[k]] : 0u;
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) {
+      const uint32_t s = s0 + k * kWave + lane;
+      const uint32_t sc = acc + wave_incl_scan_u32(w[k]);
+      if (s < total) run[s] = sc;
+      acc = readlane_u(sc, kWave - 1);
+    }
+  }
+  wave_fence();
+  return ready;
+}
+
 // REMAP: entries of region-remap requests may be among them (32-bit keys only).
-template <int KIND, int KEYS = kKeysAny, bool REMAP = false>
+// BUILD: degree bias without the CDF cache (kInt, 32-bit totals): CDFs of up to
+// kHubMin neighbours are built here, the hubs' are searched in G.int_cdf32[0],
+// an array of the hubs alone.
+template <int KIND, int KEYS = kKeysAny, bool REMAP = false, bool BUILD = false>
 __device__ void group_expand_batch(const GraphDev& G, const csaw_graph_view& hv, const ReqDev* __restrict__ R,
                                    const int32_t* __restrict__ gs2req, const HopDev& H,
                                    const int32_t* __restrict__ order, int64_t first, int count, int gs, uint32_t* lds,
@@ -913,7 +994,17 @@ __device__ void group_expand_batch(const GraphDev& G, const csaw_graph_view& hv,
   uint32_t warm = 0;
   if (lane < count) {
     const Entry en0 = load_entry(G, R, gs2req, H, order ? (int64_t)order[first + lane] : first + lane);
-    mine = make_gentry<KIND>(G, en0);
+    mine = make_gentry<BUILD ? kUniform : KIND>(G, en0);
+    if (BUILD && mine.d > 0 && mine.F > 0 && !(en0.dedup && mine.d <= mine.F)) {
+      if (mine.d <= kHubMin) {
+        mine.flags |= kPickLds << 4;
+      } else {
+        const int64_t at = G.hub_pool[hub_find(G.hub_vid, G.n_hubs, mine.v)];
+        const uint32_t T = G.int_cdf32[0][at + mine.d - 1];
+        mine.T = (uint64_t)T | ((uint64_t)at << 32);
+        if (T) mine.flags |= kPickInt32Idx << 4;
+      }
+    }
     if (H.only_kind && bias_kind(en0.bias) + 1 != H.only_kind) {  // another kind's launch
       mine.d = 0;
       mine.flags &= ~0xF0u;  // no search state, no warm-up load
@@ -925,7 +1016,7 @@ __device__ void group_expand_batch(const GraphDev& G, const csaw_graph_view& hv,
     if (KIND == kF32 && mode == kPickF32Idx)
       warm = *reinterpret_cast<const uint32_t*>(
           mine.d <= cap0 ? G.cdf + mine.o : cdf_index_first_block<float>(G.cdf, G.cdf_idx, G.E, mine.o, mine.d));
-    if (KIND == kInt && mode == kPickInt32Idx) {
+    if (KIND == kInt && !BUILD && mode == kPickInt32Idx) {
       const bool user = (mine.flags >> 1) & 1u;
       const uint32_t* C = user ? G.int_cdf32[1] : G.int_cdf32[0];
       warm = mine.d <= cap0
@@ -967,8 +1058,6 @@ __device__ void group_expand_batch(const GraphDev& G, const csaw_graph_view& hv,
   wave_fence();  // the previous batch's rounds have read theirs
   if (selects) store_gentry(ents + 4 * __popcll(sm & ((1ull << lane) - 1ull)), mine);
   wave_fence();
-  if (lane < 2) hard[lane] = 0u;
-  wave_fence();
   // Software pipeline: a round's neighbour load is consumed (written out) only
   // after the next round's selection, so its latency overlaps that round's
   // searches instead of adding to them.
@@ -984,51 +1073,61 @@ __device__ void group_expand_batch(const GraphDev& G, const csaw_graph_view& hv,
   // and even (their region remap 132 us without, 161 us with).
   constexpr int kPhases = KIND == kUniform ? 1 : 2;
   uint64_t left = 0;
-  for (int phase = 0; phase < kPhases; ++phase) {
-    const int w = phase ? kWave : gs;  // lanes per entry
-    const int NG = kWave / w;
-    const int gi = lane / w;  // group; gi == NG: the idle remainder lanes
-    const int gl = lane - gi * w, gbase = gi * w;
-    const int cap = kGroupLdsWords / NG;
-    // candidate slots of the duplicate check: each group's w words rounded up to
-    // four (16-byte aligned); the idle remainder lanes' slot follows the groups'
-    int32_t* gcl = reinterpret_cast<int32_t*>(lds + kWave * 16) + gi * ((w + 3) & ~3);
-    uint32_t* gbits = lds + kWave * 16 + kCandSlotWords + 4 * min(gi, NG - 1);
-    uint32_t* lc = small && gi < NG ? lds + kGroupBaseWords + gi * cap : nullptr;
-    const uint64_t gmask = w >= kWave ? ~0ull : (((1ull << w) - 1ull) << gbase);
-    if (phase) left = readfirst_u64(*reinterpret_cast<const uint64_t*>(hard));
-    const int n = phase ? __popcll(left) : nsel;
-    for (int e0 = 0; e0 < n; e0 += NG) {
-      int e = gi < NG ? e0 + gi : nsel;
-      if (phase) {
-        e = __builtin_ctzll(left);
-        left &= left - 1ull;
-      }
-      const int4* ep = ents + 4 * (e < nsel ? e : 0);
-      int32_t idx = -1;
-      if (e < nsel) {
-        const GEntry en = fetch_gentry(ep);
-        const int32_t res =
-            group_select<KIND, KEYS, REMAP>(G, en, w, gl, gbase, gmask, lc, cap, gcl, gbits,
-                                           kPhases == 2 && phase == 0 && w < kWave);
-        idx = gl < en.F ? res : -1;
-        if (kPhases == 2 && res == kDeferred && gl == 0) atomicOr(&hard[e >> 5], 1u << (e & 31));
-      }
-      if (have) {
-        H.src[pp] = pv;
-        H.dst[pp] = pnb;
-        H.smp[pp] = pg;
-      }
-      have = idx >= 0;
-      if (have) {
-        const int4 a = ep[0], b = ep[1];  // read again rather than held over the selection
-        pv = a.x;
-        pg = a.y;
-        pp = pack_i64(b.z, b.w) + gl;
-        pnb = Update(&hv, G.adj[pack_i64(a.z, a.w) + idx], pv);
-      }
+  int done = 0;
+  while (done < nsel) {
+    const int ready = BUILD ? build_degree_cdfs(G, ents, done, nsel, lds + kGroupBaseWords) : nsel;
+    const int stop = done + ready;
+    if (kPhases == 2) {
+      if (lane < 2) hard[lane] = 0u;
+      wave_fence();
     }
-    wave_fence();
+    for (int phase = 0; phase < kPhases; ++phase) {
+      const int w = phase ? kWave : gs;  // lanes per entry
+      const int NG = kWave / w;
+      const int gi = lane / w;  // group; gi == NG: the idle remainder lanes
+      const int gl = lane - gi * w, gbase = gi * w;
+      const int cap = kGroupLdsWords / NG;
+      // candidate slots of the duplicate check: each group's w words rounded up to
+      // four (16-byte aligned); the idle remainder lanes' slot follows the groups'
+      int32_t* gcl = reinterpret_cast<int32_t*>(lds + kWave * 16) + gi * ((w + 3) & ~3);
+      uint32_t* gbits = lds + kWave * 16 + kCandSlotWords + 4 * min(gi, NG - 1);
+      uint32_t* lc = BUILD ? lds + kGroupBaseWords : (small && gi < NG ? lds + kGroupBaseWords + gi * cap : nullptr);
+      const uint64_t gmask = w >= kWave ? ~0ull : (((1ull << w) - 1ull) << gbase);
+      if (phase) left = readfirst_u64(*reinterpret_cast<const uint64_t*>(hard));
+      const int n = phase ? __popcll(left) : ready;
+      for (int e0 = 0; e0 < n; e0 += NG) {
+        int e = gi < NG ? done + e0 + gi : stop;
+        if (phase) {
+          e = __builtin_ctzll(left);
+          left &= left - 1ull;
+        }
+        const int4* ep = ents + 4 * (e < stop ? e : done);
+        int32_t idx = -1;
+        if (e < stop) {
+          const GEntry en = fetch_gentry(ep);
+          const int32_t res =
+              group_select<KIND, KEYS, REMAP, BUILD>(G, en, w, gl, gbase, gmask, lc, cap, gcl, gbits,
+                                             kPhases == 2 && phase == 0 && w < kWave);
+          idx = gl < en.F ? res : -1;
+          if (kPhases == 2 && res == kDeferred && gl == 0) atomicOr(&hard[e >> 5], 1u << (e & 31));
+        }
+        if (have) {
+          H.src[pp] = pv;
+          H.dst[pp] = pnb;
+          H.smp[pp] = pg;
+        }
+        have = idx >= 0;
+        if (have) {
+          const int4 a = ep[0], b = ep[1];  // read again rather than held over the selection
+          pv = a.x;
+          pg = a.y;
+          pp = pack_i64(b.z, b.w) + gl;
+          pnb = Update(&hv, G.adj[pack_i64(a.z, a.w) + idx], pv);
+        }
+      }
+      wave_fence();
+    }
+    done = stop;
   }
   if (have) {
     H.src[pp] = pv;

@@ -445,3 +445,33 @@ def test_batched_frontier_order(C, O, g14, cdf_cache, sizes):
             for r in range(4):
                 same(p.result(r), want[r], f"request {r} {kw} cache {cdf_cache}")
         p.close()
+
+
+@pytest.mark.parametrize("fan", [1, 4, 5, 16, 33, 64])
+def test_degree_cdfs_built_in_groups(C, O, fan):
+    """Degree bias without the CDF cache: degrees around the lanes of a row, the
+    LDS words of a wave's run (entries that end it, fill it and start the next)
+    and the hubs beyond; directed lists with zero-degree neighbours (all-zero
+    biases, zero runs); a repeated neighbour."""
+    rng = np.random.default_rng(fan)
+    degs = [1, 2, 3, 63, 64, 65, 127, 255, 256, 257, 400, 511, 512, 513, 640, 1023, 1024, 1025, 1026, 3000]
+    V = 6000
+    lists = [np.sort(rng.choice(V, d, replace=False)) for d in degs]
+    lists.append(np.arange(3000, 3100))              # neighbours without out-edges
+    lists.append(np.repeat(np.arange(5), 9))         # repeated neighbours
+    lists += [np.sort(rng.choice(V, rng.integers(0, 40) if i < 2900 else 0, replace=False))
+              for i in range(V - len(lists))]
+    off = np.concatenate([[0], np.cumsum([len(x) for x in lists])]).astype(np.int64)
+    adj = np.concatenate(lists).astype(np.int32)
+    g = C.Graph.from_csr(off, adj)
+    og = O.OracleGraph(off, adj)
+    for n in (40, 700, 17000):
+        seeds = rng.integers(0, len(degs) + 2 if n < 1000 else V, n).astype(np.int32)
+        for dedup in (1, 0):
+            want = O.sample(og, seeds, [fan, 3], bias=O.BIAS_DEGREE, dedup=dedup)
+            same(C.sample(g, seeds, [fan, 3], bias=C.BIAS_DEGREE, dedup=dedup), want, f"plain {n} {dedup}")
+            p = C.Plan(g, [{"seeds": seeds, "fanouts": [fan, 3], "bias": C.BIAS_DEGREE, "dedup": dedup, "request": 0}],
+                       mode=C.MODE_BATCHED)
+            p.run()
+            same(p.result(0), want, f"batched {n} {dedup}")
+            p.close()
