@@ -313,6 +313,7 @@ static void plan_layout(csaw_plan* p, const PlanSizes& z, Carver& c, size_t* fil
   const int64_t nblk = (z.nmax + kBlockEntries - 1) / kBlockEntries;
   c.part(&p->local_excl, z.nmax);
   c.part(&p->blk_excl, nblk);
+  c.part(&p->blk_scan, std::min<int64_t>(nblk, 1024));
   c.part(&p->grp_excl, (nblk + 1023) / 1024);
   c.part(&p->totals, z.depth);
   if (z.several) c.part(&p->kind_mask, (z.nmax + kWave - 1) / kWave);
@@ -383,6 +384,7 @@ static HopDev make_hop(csaw_plan* p, Unit& u, int h) {
   H.gb = u.gb[h];
   H.local_excl = p->local_excl;
   H.blk_excl = p->blk_excl;
+  H.blk_scan = p->blk_scan;
   H.grp_excl = p->grp_excl;
   H.order = p->order;
   H.chunks = p->chunks;

@@ -82,6 +82,7 @@ struct csaw_plan {
   int32_t* order = nullptr;
   uint8_t* kind_mask = nullptr;  // whole-hop kernels of several kinds (HopDev)
   uint32_t* blk_excl = nullptr;
+  uint32_t* blk_scan = nullptr;
   uint64_t* grp_excl = nullptr;
   csaw::Chunk* chunks = nullptr;
   uint32_t chunk_cap = 0;

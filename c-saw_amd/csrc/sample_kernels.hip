@@ -7,6 +7,7 @@
 //   k_scan_blocks   exclusive scan of block sums within groups of 1024 blocks
 //   k_scan_groups   exclusive scan of group sums; hop total
 //   k_offsets       per-sample edge offsets of the hop (= next frontier offsets)
+//   k_scan_offsets  the three in one for hops of at most 1024 blocks
 //   k_choose        variant per chunk (heuristic / forced / random / MLP),
 //                   appended to per-variant queues with wave-aggregated atomics
 //   k_expand<V,K>   persistent: pulls chunks of its queue and expands them
@@ -245,14 +246,9 @@ __global__ __launch_bounds__(256) void k_scan_groups(HopDev H, int64_t* __restri
 
 // per-sample edge offsets for samples [0, gb] of this hop, and the bounds of
 // the requests active in it (the offsets at their first and past their last
-// sample)
-__global__ void k_offsets(HopDev H, const ReqDev* __restrict__ R, const int64_t* __restrict__ total) {
-  const int64_t n = *H.n_ptr;
-  auto offset = [&](int64_t g) -> int64_t {
-    const int64_t x = H.fo[g];
-    return x >= n ? *total
-                  : (int64_t)H.grp_excl[x >> kGroupShift] + H.blk_excl[x >> kBlockShift] + H.local_excl[x];
-  };
+// sample).  offset(g): the edges before sample g's frontier.
+template <class Offset>
+__device__ __forceinline__ void write_offsets(const HopDev& H, const ReqDev* __restrict__ R, const Offset& offset) {
   const int64_t t0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
   for (int64_t g = t0; g <= H.gb; g += step) H.eo[g] = offset(g);
   if (!H.bounds) return;
@@ -261,6 +257,56 @@ __global__ void k_offsets(HopDev H, const ReqDev* __restrict__ R, const int64_t*
     if (r.depth > H.hop)
       H.bounds[((int64_t)r.slot * CSAW_MAX_HOPS + H.hop) * 2 + (i & 1)] = offset(r.gbase + (i & 1 ? r.samples : 0));
   }
+}
+
+__global__ void k_offsets(HopDev H, const ReqDev* __restrict__ R, const int64_t* __restrict__ total) {
+  const int64_t n = *H.n_ptr;
+  write_offsets(H, R, [&](int64_t g) -> int64_t {
+    const int64_t x = H.fo[g];
+    return x >= n ? *total
+                  : (int64_t)H.grp_excl[x >> kGroupShift] + H.blk_excl[x >> kBlockShift] + H.local_excl[x];
+  });
+}
+
+// Both scans and the offsets of a hop of at most one group (1,048,576 entries)
+// in one launch: every workgroup scans the block sums in LDS, the first writes
+// them out for the expansion.  Such hops are bound by the launches between
+// their kernels (with three launches a hop 3,000 seeds
+// {15, 10, 5} by weight took 212 us, with one 196; 1,000 seeds {2, 2} 76 and 70).
+__global__ __launch_bounds__(256) void k_scan_offsets(HopDev H, const ReqDev* __restrict__ R, int64_t* __restrict__ total) {
+  __shared__ uint32_t wsum[4];
+  __shared__ uint32_t pre_s[1024];
+  const int64_t n = *H.n_ptr;
+  const int nblk = (int)((n + kBlockEntries - 1) >> kBlockShift);
+  const int tid = threadIdx.x, lane = lane_id(), wid = tid / kWave;
+  uint32_t x[4], s = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int b = tid * 4 + i;
+    x[i] = b < nblk ? H.blk_excl[b] : 0u;
+    s += x[i];
+  }
+  const uint32_t incl = wave_incl_scan_u32(s);
+  if (lane == kWave - 1) wsum[wid] = incl;
+  __syncthreads();
+  uint32_t pre = incl - s;
+  for (int w = 0; w < wid; ++w) pre += wsum[w];
+  const uint32_t all = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    pre_s[tid * 4 + i] = pre;
+    if (blockIdx.x == 0 && tid * 4 + i < nblk) H.blk_scan[tid * 4 + i] = pre;
+    pre += x[i];
+  }
+  if (blockIdx.x == 0 && tid == 0) {
+    if (nblk > 0) H.grp_excl[0] = 0;
+    *total = (int64_t)all;
+  }
+  __syncthreads();
+  write_offsets(H, R, [&](int64_t g) -> int64_t {
+    const int64_t e = H.fo[g];
+    return e >= n ? (int64_t)all : (int64_t)pre_s[e >> kBlockShift] + H.local_excl[e];
+  });
 }
 
 // ---------------------------------------------------------------- copy-out
@@ -871,16 +917,22 @@ int launch_bin_list(const LaunchCfg& L, const GraphDev& G, const ReqDev* R, cons
   return CSAW_OK;
 }
 
-int launch_scans(const LaunchCfg& L, const HopDev& H, const ReqDev* R, int64_t* total, int64_t max_entries) {
+int launch_scans(const LaunchCfg& L, HopDev& H, const ReqDev* R, int64_t* total, int64_t max_entries) {
   int64_t nb = (max_entries + kBlockEntries - 1) / kBlockEntries;
   int64_t ng = (nb + 1023) / 1024;
+  int64_t gs = std::max<int64_t>(H.gb + 1, H.bounds ? 2 * (int64_t)H.n_req : 0);
+  int g2 = (int)std::max<int64_t>(1, std::min<int64_t>((gs + 255) / 256, grid_of(L, 8)));
+  if (ng <= 1) {
+    k_scan_offsets<<<std::min(g2, L.num_cu), 256, 0, L.stream>>>(H, R, total);
+    CSAW_LAUNCH_CHECK();
+    H.blk_excl = H.blk_scan;
+    return CSAW_OK;
+  }
   int grid = (int)std::max<int64_t>(1, std::min<int64_t>(ng, grid_of(L, 4)));
   k_scan_blocks<<<grid, 256, 0, L.stream>>>(H);
   CSAW_LAUNCH_CHECK();
   k_scan_groups<<<1, 256, 0, L.stream>>>(H, total);
   CSAW_LAUNCH_CHECK();
-  int64_t gs = std::max<int64_t>(H.gb + 1, H.bounds ? 2 * (int64_t)H.n_req : 0);
-  int g2 = (int)std::max<int64_t>(1, std::min<int64_t>((gs + 255) / 256, grid_of(L, 8)));
   k_offsets<<<g2, 256, 0, L.stream>>>(H, R, total);
   CSAW_LAUNCH_CHECK();
   return CSAW_OK;

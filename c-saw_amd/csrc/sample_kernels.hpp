@@ -89,7 +89,8 @@ int launch_count(const LaunchCfg& L, const GraphDev& G, const ReqDev* R, const i
 // Bins the n entries list[0 .. n) into chunks (H.order by list position).
 int launch_bin_list(const LaunchCfg& L, const GraphDev& G, const ReqDev* R, const int32_t* gs2req, const HopDev& H,
                     const int32_t* list, int64_t n);
-int launch_scans(const LaunchCfg& L, const HopDev& H, const ReqDev* R, int64_t* total, int64_t max_entries);
+// Places the hop's edges; afterwards H.blk_excl is the scanned one.
+int launch_scans(const LaunchCfg& L, HopDev& H, const ReqDev* R, int64_t* total, int64_t max_entries);
 // One request's hops (k_copy_edges): hop h's edges are [lo[h], lo[h] + n[h])
 // of its columns col[0 .. 2][h] (src, dst, sample) and go to out[c] + at[h];
 // eo[h] are its rows = samples + 1 offsets, written to hop_offsets[h * rows ..]

@@ -586,13 +586,14 @@ extern "C" int csaw_stream_sample_opts(csaw_host_graph* hg, const csaw_request* 
       CSAW_TRY(B.alloc(&d_smp[h], cap[h]));
     }
     const int64_t nblk = (mx + kBlockEntries - 1) / kBlockEntries;
-    uint32_t *d_local, *d_blk, *d_cnt, *d_poff, *d_cursor;
+    uint32_t *d_local, *d_blk, *d_blk_scan, *d_cnt, *d_poff, *d_cursor;
     uint64_t* d_grp;
     int64_t* d_tot;
     uint8_t* d_pid;
     int32_t *d_list, *d_vb;
     CSAW_TRY(B.alloc(&d_local, mx));
     CSAW_TRY(B.alloc(&d_blk, nblk));
+    CSAW_TRY(B.alloc(&d_blk_scan, std::min<int64_t>(nblk, 1024)));
     CSAW_TRY(B.alloc(&d_grp, (nblk + 1023) / 1024));
     CSAW_TRY(B.alloc(&d_tot, std::max(r.depth, 1)));
     CSAW_TRY(B.alloc(&d_pid, mx));
@@ -669,6 +670,7 @@ extern "C" int csaw_stream_sample_opts(csaw_host_graph* hg, const csaw_request* 
       H.gb = S;
       H.local_excl = d_local;
       H.blk_excl = d_blk;
+      H.blk_scan = d_blk_scan;
       H.grp_excl = d_grp;
       H.src = d_src[h];
       H.dst = d_dst[h];

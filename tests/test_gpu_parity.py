@@ -475,3 +475,24 @@ def test_degree_cdfs_built_in_groups(C, O, fan):
             p.run()
             same(p.result(0), want, f"batched {n} {dedup}")
             p.close()
+
+
+@pytest.mark.parametrize("n", [1, 1023, 1024, 1025, 65536, (1 << 20) - 1, 1 << 20, (1 << 20) + 1])
+def test_offsets_of_one_group_and_more(C, O, g14, n):
+    """Edge placement around a block of 1024 entries and around the 1024 blocks
+    that one launch scans; plain and batched (request bounds), a capture's
+    replays."""
+    g, og, *_ = g14
+    sizes = [n - n // 3, n // 3] if n > 2 else [n]
+    specs, want = [], []
+    for i, k in enumerate(sizes):
+        s = {"seeds": g.seeds(k, request=i), "fanouts": [1, 1], "bias": 0, "dedup": 1, "request": i}
+        specs.append(s)
+        want.append(O.sample(og, s["seeds"], s["fanouts"], bias=O.BIAS_UNIFORM, request=i))
+    for kw in ({"mode": C.MODE_PLAIN}, {"mode": C.MODE_BATCHED}, {"mode": C.MODE_BATCHED, "use_graph": True}):
+        p = C.Plan(g, specs, **kw)
+        for _ in range(3):
+            p.run()
+            for i, w in enumerate(want):
+                same(p.result(i), w, f"{n} {kw} request {i}")
+        p.close()
