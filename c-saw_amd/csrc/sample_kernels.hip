@@ -455,7 +455,10 @@ __global__ __launch_bounds__(256, KEYS == kKeys32 && !REMAP ? 4 : 1) void k_expa
   }
 }
 
-// one wave per 64 listed entries (the streaming path: entries of one partition)
+// A list of entries (the streaming path: those of one partition), a wave per
+// entry: lists are short, and 64 entries a wave left all but 60 workgroups' worth
+// of the chip idle (4,000 degree-biased entries 400 us, of which a wave's serial
+// chain of 64 entries was nearly all).
 template <int KIND>
 __global__ __launch_bounds__(256) void k_expand_list(GraphDev G, csaw_graph_view hv, const ReqDev* __restrict__ R,
                                                      const int32_t* __restrict__ gs2req, HopDev H,
@@ -475,7 +478,7 @@ __global__ __launch_bounds__(256) void k_expand_list(GraphDev G, csaw_graph_view
 int launch_expand_list(const LaunchCfg& L, int kind, const GraphDev& G, const csaw_graph_view& hv, const ReqDev* R,
                        const int32_t* gs2req, const HopDev& H, const int32_t* list, int64_t n) {
   if (n <= 0) return CSAW_OK;
-  const int64_t nwg = (n + 4 * kWave - 1) / (4 * kWave);
+  const int64_t nwg = (n + 3) / 4;
   const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(nwg, (int64_t)L.num_cu * L.expand_per_cu));
   if (kind == kUniform) k_expand_list<kUniform><<<grid, 256, 0, L.stream>>>(G, hv, R, gs2req, H, list, n);
   else if (kind == kInt) k_expand_list<kInt><<<grid, 256, 0, L.stream>>>(G, hv, R, gs2req, H, list, n);

@@ -205,6 +205,22 @@ __global__ __launch_bounds__(256) void k_part_scatter(HopDev H, const uint8_t* _
 }
 
 constexpr int64_t kChunkedMin = 16384;  // frontier entries below which a partition is not binned
+
+// Whether a partition of cnt frontier entries is binned into chunks with a kernel
+// variant each, or expanded one wave per entry in list order.  Every drawing
+// vertex has its CDF by then, so the variants share no builds, and list order
+// writes a wave's edges next to one another.  Expansion of {15, 10, 5} by degree
+// from 16,384 seeds over 16 partitions of RMAT-22: 17.9 ms binned from 16,384
+// entries on, 9.8 in list order; {10, 10, 5} from 65,536 over 3 (a million entries
+// a partition) 16.0 and 7.7; {25, 10} by user bias from 60,000 over 4 15.6 and
+// 3.4.  So only what asks for chunks gets them: a line set by the caller, forced
+// and random variants, chunk logs.
+static bool partition_bins(const csaw_stream_opts& o, bool batched, int64_t cnt) {
+  if (!batched) return false;
+  if (o.bin_min_entries > 0) return cnt >= o.bin_min_entries;
+  if (!o.log_chunks && (o.sched == CSAW_SCHED_HEURISTIC || o.sched == CSAW_SCHED_MLP)) return false;
+  return cnt >= kChunkedMin;
+}
 constexpr int64_t kPieceBlocks = 1 << 17;  // packed blocks per staged piece (8M entries)
 
 // One wave per block of a staged piece: blocks pb0 + k (k < nb) at bytes
@@ -835,9 +851,7 @@ extern "C" int csaw_stream_sample_opts(csaw_host_graph* hg, const csaw_request* 
           }
           last_use[buf] = ++use_tick;
         }
-        // small partitions are expanded one wave per entry whatever the
-        // schedule: binning and choosing cost more than they save there
-        const bool chunked = batched && (int64_t)cnt[p] >= (o.bin_min_entries > 0 ? o.bin_min_entries : kChunkedMin);
+        const bool chunked = partition_bins(o, batched, (int64_t)cnt[p]);
         hipEvent_t eb0, eb1, ex0, ex1;
         CSAW_TRY(event(&eb0));
         CSAW_TRY(event(&eb1));

@@ -364,8 +364,9 @@ typedef struct csaw_stream_opts {
                         /*  factor x its estimated bus bytes < its slice's  */
                         /*  bytes (0: 2)                                     */
   int32_t bin_min_entries; /* batched: partitions with fewer frontier       */
-                        /*  entries run one wave per entry, unbinned (0:     */
-                        /*  16384; 1: bin every partition)                   */
+                        /*  entries run one wave per entry, unbinned (0: all */
+                        /*  under the heuristic and learned schedules        */
+                        /*  without logs, else 16384; 1: bin every partition)*/
   /* Per-chunk cost-model data (batched mode; each partition's chunks are
    * read back after it expands, so logging runs slower).  Rows as in
    * csaw_plan_chunk_log; keys are hop << 40 | partition << 32 | chunk key. */

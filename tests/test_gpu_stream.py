@@ -248,3 +248,26 @@ def test_stream_packed_multi_piece(C):
                           slice_policy=C.SLICE_COPY)
     same(got, want, "two pieces per slice")
     assert got["stats"].h2d_bytes < got["stats"].h2d_raw_bytes
+
+
+@pytest.mark.parametrize("bias", [0, 1, 3])
+@pytest.mark.parametrize("n", [1, 5, 8191, 8193, 70001])
+def test_stream_list_order(C, graphs, bias, n):
+    """Partitions in list order under the default schedules: fewer entries than
+    waves, around one entry per launched wave and several batches a wave; without
+    a bin line the schedules bin nothing, with logs or forced variants they do."""
+    g, hg, og = graphs
+    seeds = g.seeds(n, request=n)
+    for dedup in (1, 0, 2):
+        want = C.sample(g, seeds, [3, 2], bias=bias, dedup=dedup, request=4)
+        for parts in (1, 3):
+            for kw in (dict(sched=C.SCHED_HEURISTIC), dict(sched=C.SCHED_MLP, mlp=C.Mlp(2))):
+                got = C.stream_sample(hg, seeds, [3, 2], bias=bias, dedup=dedup, request=4, partitions=parts,
+                                      budget_bytes=1 << 30, mode=C.MODE_BATCHED, **kw)
+                same(got, want, f"{n} {dedup} {parts}")
+                assert got["stats"].chunks == 0
+    if n > 16384 and bias != 3:
+        got = C.stream_sample(hg, seeds, [3, 2], bias=bias, dedup=2, request=4, partitions=1, budget_bytes=1 << 30,
+                              mode=C.MODE_BATCHED, sched=C.SCHED_FORCED, variant=1)
+        same(got, want, "forced")
+        assert got["stats"].chunks > 0
