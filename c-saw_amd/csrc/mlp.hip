@@ -129,8 +129,10 @@ __global__ __launch_bounds__(kWave) void k_mlp_rows(const uint16_t* __restrict__
 // Bound: the latency of the first tile (the rows were written by other XCDs)
 // and the 256-deep chain.  For 256 rows: 88 us with a lane's pairs loaded from
 // memory one by one, 26 us with 32 pairs loaded ahead, 15 us from LDS with the
-// tile widths as run-time values, 12 us as constants.
+// tile widths as run-time values, 12.3 us as constants, 10.9 us staged by sixteen
+// waves (one wave a workgroup, four times the workgroups: 28 us).
 constexpr int kParamRows = 128;
+constexpr int kParamThreads = 1024;  // all stage, the first four waves sum
 constexpr int kParamGrid = 25;
 struct ParamOut {
   float *grad, *master;
@@ -142,8 +144,8 @@ template <bool SGD, int WB, int NA, int SA>
 __device__ __forceinline__ void param_tile(int64_t n, const float* __restrict__ B, const float* __restrict__ A, float* tb,
                                            float* ta, int ca, int cb, int p, const ParamOut& O) {
   const int tid = threadIdx.x;
-  constexpr int kQuads = (kParamRows * WB / 4 + kMlpThreads - 1) / kMlpThreads;  // float4s of a B tile per thread
-  constexpr int kSingles = (kParamRows * NA + kMlpThreads - 1) / kMlpThreads;
+  constexpr int kQuads = (kParamRows * WB / 4 + kParamThreads - 1) / kParamThreads;  // float4s of a B tile per thread
+  constexpr int kSingles = (kParamRows * NA + kParamThreads - 1) / kParamThreads;
   float4 qb[kQuads];
   float qa[kSingles > 0 ? kSingles : 1];
   // quads past the last row end inside the array's padding (256 bytes)
@@ -152,26 +154,27 @@ __device__ __forceinline__ void param_tile(int64_t n, const float* __restrict__ 
     const float4* src = reinterpret_cast<const float4*>(B + s0 * WB);
 #pragma unroll
     for (int k = 0; k < kQuads; ++k)
-      if (k * kMlpThreads + tid < (rows * WB + 3) / 4) qb[k] = src[k * kMlpThreads + tid];
+      if (k * kParamThreads + tid < (rows * WB + 3) / 4) qb[k] = src[k * kParamThreads + tid];
     if constexpr (NA > 0) {
       const float* asrc = A + s0 * SA;
 #pragma unroll
       for (int k = 0; k < kSingles; ++k) {
-        const int i = k * kMlpThreads + tid;
+        const int i = k * kParamThreads + tid;
         if (i < rows * NA) qa[k] = asrc[(i / NA) * SA + i % NA];
       }
     }
   };
   float acc = 0.f;
   load(0);
+  const float old = SGD && p >= 0 ? O.master[p] : 0.f;  // not after the chain
   for (int64_t s0 = 0; s0 < n; s0 += kParamRows) {
     const int rows = (int)(n - s0 < kParamRows ? n - s0 : kParamRows);
 #pragma unroll
     for (int k = 0; k < kQuads; ++k)
-      if (k * kMlpThreads + tid < (rows * WB + 3) / 4) reinterpret_cast<float4*>(tb)[k * kMlpThreads + tid] = qb[k];
+      if (k * kParamThreads + tid < (rows * WB + 3) / 4) reinterpret_cast<float4*>(tb)[k * kParamThreads + tid] = qb[k];
 #pragma unroll
     for (int k = 0; k < kSingles; ++k)
-      if (k * kMlpThreads + tid < rows * NA) ta[k * kMlpThreads + tid] = qa[k];
+      if (k * kParamThreads + tid < rows * NA) ta[k * kParamThreads + tid] = qa[k];
     __syncthreads();
     if (s0 + kParamRows < n) load(s0 + kParamRows);
     if (p >= 0) {
@@ -188,7 +191,7 @@ __device__ __forceinline__ void param_tile(int64_t n, const float* __restrict__ 
   }
   if (p < 0) return;
   if (SGD) {
-    const float v = O.master[p] - O.lr * acc;
+    const float v = old - O.lr * acc;
     O.master[p] = v;
     O.wb[p] = f32_to_bf16(v);
   } else {
@@ -197,7 +200,7 @@ __device__ __forceinline__ void param_tile(int64_t n, const float* __restrict__ 
 }
 
 template <bool SGD>
-__global__ __launch_bounds__(kMlpThreads) void k_mlp_params(int64_t n, const float* __restrict__ Xb,
+__global__ __launch_bounds__(kParamThreads) void k_mlp_params(int64_t n, const float* __restrict__ Xb,
                                                             const float* __restrict__ H1, const float* __restrict__ H2,
                                                             const float* __restrict__ dY, const float* __restrict__ dH1,
                                                             const float* __restrict__ dH2, ParamOut O) {
@@ -206,12 +209,15 @@ __global__ __launch_bounds__(kMlpThreads) void k_mlp_params(int64_t n, const flo
   const int b = blockIdx.x, lane = lane_id(), wid = threadIdx.x / kWave;
   const int bias_p = wid == 0 ? lane : -1;
   if (b < 16) {  // W2, rows 4b .. 4b + 3
-    param_tile<SGD, kMlpHid, 4, kMlpHid>(n, H1, dH2 + 4 * b, tb, ta, wid, lane, kMlpW2 + (4 * b + wid) * kMlpHid + lane, O);
+    param_tile<SGD, kMlpHid, 4, kMlpHid>(n, H1, dH2 + 4 * b, tb, ta, wid, lane,
+                                         wid < 4 ? kMlpW2 + (4 * b + wid) * kMlpHid + lane : -1, O);
   } else if (b < 20) {  // W1, sixteen rows
     const int a0 = 16 * (b - 16), ca = 4 * wid + lane / kMlpIn, cb = lane % kMlpIn;
-    param_tile<SGD, kMlpIn, 16, kMlpHid>(n, Xb, dH1 + a0, tb, ta, ca, cb, kMlpW1 + (a0 + ca) * kMlpIn + cb, O);
+    param_tile<SGD, kMlpIn, 16, kMlpHid>(n, Xb, dH1 + a0, tb, ta, ca, cb,
+                                         wid < 4 ? kMlpW1 + (a0 + ca) * kMlpIn + cb : -1, O);
   } else if (b == 20) {  // W3, rows 0 .. 3
-    param_tile<SGD, kMlpHid, 4, kMlpOut>(n, H2, dY, tb, ta, wid, lane, kMlpW3 + wid * kMlpHid + lane, O);
+    param_tile<SGD, kMlpHid, 4, kMlpOut>(n, H2, dY, tb, ta, wid, lane,
+                                         wid < 4 ? kMlpW3 + wid * kMlpHid + lane : -1, O);
   } else if (b == 21) {  // W3, row 4
     param_tile<SGD, kMlpHid, 1, kMlpOut>(n, H2, dY + 4, tb, ta, 0, lane, wid == 0 ? kMlpW3 + 4 * kMlpHid + lane : -1, O);
   } else if (b < 24) {  // b1, b2
@@ -412,7 +418,7 @@ extern "C" int csaw_mlp_grad(csaw_mlp* m, const float* X, const float* T, const 
   CSAW_HIP(hipMemcpy(w.M, M, sizeof(float) * n * kMlpOut, hipMemcpyHostToDevice));
   const double cnt = mask_count(M, n);
   CSAW_TRY(mlp_rows_loss(m, w, nullptr, n, cnt > 0 ? (float)(1.0 / cnt) : 0.f, true));
-  k_mlp_params<false><<<kParamGrid, kMlpThreads, 0, m->stream>>>(n, w.Xb, w.H1, w.H2, w.dY, w.dH1, w.dH2,
+  k_mlp_params<false><<<kParamGrid, kParamThreads, 0, m->stream>>>(n, w.Xb, w.H1, w.H2, w.dY, w.dH1, w.dH2,
                                                                  ParamOut{w.grad, nullptr, nullptr, 0.f});
   CSAW_LAUNCH_CHECK();
   CSAW_TRY(mlp_sum_loss(m, w, n));
@@ -450,7 +456,7 @@ extern "C" int csaw_mlp_train(csaw_mlp* m, const float* X, const float* T, const
         for (int j = 0; j < kMlpOut; ++j) cnt += M[(int64_t)perm[b + s] * kMlpOut + j] != 0.f ? 1.0 : 0.0;
       if (cnt == 0) continue;
       CSAW_TRY(mlp_rows_loss(m, w, w.idx + b, cnt_rows, (float)(1.0 / cnt), true));
-      k_mlp_params<true><<<kParamGrid, kMlpThreads, 0, m->stream>>>(cnt_rows, w.Xb, w.H1, w.H2, w.dY, w.dH1, w.dH2,
+      k_mlp_params<true><<<kParamGrid, kParamThreads, 0, m->stream>>>(cnt_rows, w.Xb, w.H1, w.H2, w.dY, w.dH1, w.dH2,
                                                                     ParamOut{nullptr, m->d_master, m->d_w, lr});
       CSAW_LAUNCH_CHECK();
     }

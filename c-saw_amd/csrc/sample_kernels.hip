@@ -427,8 +427,8 @@ __global__ __launch_bounds__(256, KEYS == kKeys32 && !REMAP ? 4 : 1) void k_expa
   // what it waits for are the few slots with many redraws, and 64 attempts a round
   // end those sooner.  (Uniform draws collide too rarely for that: groups
   // throughout.)  On RMAT-22, groups and whole waves: region remap of 8,191 seeds
-  // {10, 10} 813 and 681 us, degree bias {25, 10} from 40,000 with the CDF cache
-  // 608 and 543 us, without 870 and 794; beyond the line the groups are level.
+  // {10, 10} 542 and 469 us, degree bias {25, 10} from 40,000 with the CDF cache
+  // 609 and 534 us, without 854 and 735; beyond the line the groups are level.
   const int gs = hop_gs > 0 && KIND != kUniform && n * (kWave / hop_gs) <= kWideHopEntries ? kWave : hop_gs;
   // batch size adapts to the frontier: one entry (one group round) per wave
   // when it is small (all waves busy), up to 64 entries per metadata round
