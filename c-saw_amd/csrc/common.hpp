@@ -127,7 +127,7 @@ struct HopDev {
   int32_t gb;           // first inactive global sample
   uint32_t* local_excl; // per entry
   uint32_t* blk_excl;   // per block of 1024 entries
-  uint32_t* blk_scan;   // where a one-group hop's scan of them goes (launch_scans)
+  uint32_t* blk_scan;   // where a one-group hop's scan of them goes (launch_scans), or null
   uint64_t* grp_excl;   // per group of 1024 blocks
   int32_t* order;       // bucket-sorted entry ids (per block region)
   Chunk* chunks;

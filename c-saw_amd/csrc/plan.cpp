@@ -1,14 +1,16 @@
 // Sampling plans: the host side of Sampler() (non-stream/main.cu:196-308),
 // re-designed around reusable device buffers.
 //
-// A plan owns every buffer a run needs (allocated once at creation, sized by
-// the per-request upper bound S * F_0 * ... * F_h per hop), so csaw_plan_run
-// allocates nothing and its launch sequence can be captured in a hipGraph.
+// A plan holds every buffer a run needs in one block (sized at creation by the
+// per-request upper bound S * F_0 * ... * F_h per hop, taken from the graph's
+// pool), so csaw_plan_run allocates nothing and its launch sequence can be
+// captured in a hipGraph.
 // PLAIN mode executes one request after another (one unit per request, a
 // wave per frontier entry, synchronising after each request like a call of
 // the reference's Sampler()); BATCHED mode puts all requests into one unit:
-// one launch sequence per hop over the concatenated frontiers, with degree
-// binning and a per-chunk kernel-variant choice.
+// one launch sequence per hop over the concatenated frontiers: a kernel per bias
+// kind in frontier order, or degree binning and a kernel variant per chunk
+// (plan_bins_hop).
 #include <algorithm>
 #include <cmath>
 #include <cstring>

@@ -16,11 +16,10 @@
 //    array instead of a pass over the neighbour list per frontier entry;
 //  - output positions come from the same global prefix sums as the
 //    in-memory run, so the edge list is bit-identical to it.
-// In batched mode each partition's entries are binned into chunks by degree
-// class and every chunk runs the kernel variant the schedule picks (the
-// fixed heuristic, a forced variant, a random one or the learned cost
-// model), exactly as in the in-memory batched run; in plain mode one wave
-// expands each listed entry.
+// One wave expands each listed entry of a partition; where chunks are asked for
+// (partition_bins) its entries are binned into chunks by degree class and every
+// chunk runs the kernel variant the schedule picks (the fixed heuristic, a
+// forced variant, a random one or the learned cost model).
 // Every device allocation is charged against budget_bytes.
 #include <algorithm>
 #include <cmath>
@@ -602,14 +601,13 @@ extern "C" int csaw_stream_sample_opts(csaw_host_graph* hg, const csaw_request* 
       CSAW_TRY(B.alloc(&d_smp[h], cap[h]));
     }
     const int64_t nblk = (mx + kBlockEntries - 1) / kBlockEntries;
-    uint32_t *d_local, *d_blk, *d_blk_scan, *d_cnt, *d_poff, *d_cursor;
+    uint32_t *d_local, *d_blk, *d_cnt, *d_poff, *d_cursor;
     uint64_t* d_grp;
     int64_t* d_tot;
     uint8_t* d_pid;
     int32_t *d_list, *d_vb;
     CSAW_TRY(B.alloc(&d_local, mx));
     CSAW_TRY(B.alloc(&d_blk, nblk));
-    CSAW_TRY(B.alloc(&d_blk_scan, std::min<int64_t>(nblk, 1024)));
     CSAW_TRY(B.alloc(&d_grp, (nblk + 1023) / 1024));
     CSAW_TRY(B.alloc(&d_tot, std::max(r.depth, 1)));
     CSAW_TRY(B.alloc(&d_pid, mx));
@@ -686,7 +684,6 @@ extern "C" int csaw_stream_sample_opts(csaw_host_graph* hg, const csaw_request* 
       H.gb = S;
       H.local_excl = d_local;
       H.blk_excl = d_blk;
-      H.blk_scan = d_blk_scan;
       H.grp_excl = d_grp;
       H.src = d_src[h];
       H.dst = d_dst[h];

@@ -349,10 +349,10 @@ typedef enum csaw_slice_policy {
 
 /* How each partition's frontier entries are expanded. */
 typedef struct csaw_stream_opts {
-  int32_t mode;         /* CSAW_MODE_BATCHED: entries binned into chunks by  */
-                        /*  degree class and each chunk run by the variant  */
-                        /*  `sched` picks; CSAW_MODE_PLAIN: one wave per     */
-                        /*  listed entry                                     */
+  int32_t mode;         /* CSAW_MODE_BATCHED: partitions of bin_min_entries  */
+                        /*  and more are binned into chunks by degree class, */
+                        /*  each run by the variant `sched` picks; the rest, */
+                        /*  and CSAW_MODE_PLAIN: one wave per listed entry   */
   int32_t sched;        /* csaw_sched                                        */
   int32_t variant;      /* forced variant                                    */
   uint64_t explore_key; /* key of CSAW_SCHED_RANDOM                          */
