@@ -521,14 +521,12 @@ __global__ void k_index_level(const T* __restrict__ C, int64_t E, int sh, int64_
 }
 
 template <typename T>
-static int build_index(const T* C, int64_t E, T** out, hipStream_t stream, int num_cu) {
-  const int64_t tot = cdf_index_size(E);
-  CSAW_HIP(hipMalloc(out, sizeof(T) * (tot > 0 ? tot : 16)));
+static int build_index(const T* C, int64_t E, T* out, hipStream_t stream, int num_cu) {
   int64_t at = 0;
   for (int l = 1; l <= cdf_index_levels(E); ++l) {
     const int sh = 4 * l;
     const int64_t n = (E + ((int64_t)1 << sh) - 1) >> sh, npad = cdf_index_level_size(E, l);
-    k_index_level<T><<<grid_for(npad, 256, num_cu), 256, 0, stream>>>(C, E, sh, n, npad, *out + at);
+    k_index_level<T><<<grid_for(npad, 256, num_cu), 256, 0, stream>>>(C, E, sh, n, npad, out + at);
     CSAW_LAUNCH_CHECK();
     at += npad;
   }
@@ -536,12 +534,25 @@ static int build_index(const T* C, int64_t E, T** out, hipStream_t stream, int n
   return CSAW_OK;
 }
 
+template <typename T>
+static int build_index(const T* C, int64_t E, T** out, hipStream_t stream, int num_cu) {
+  CSAW_HIP(hipMalloc(out, sizeof(T) * std::max<int64_t>(cdf_index_size(E), 16)));
+  return build_index(C, E, *out, stream, num_cu);
+}
+
 // The DEGREE hub CDFs as uint32, padded and indexed like the CDF cache, when
-// their totals fit (duplicate neighbours can total more than E).
+// their totals fit (duplicate neighbours can total more than E) and there is
+// room for them; without them every entry keeps to the uint64 hubs.
 static int narrow_hubs(csaw_graph* g) {
   const int64_t n = g->hub_entries, npad = pad16(n);
+  auto room = [](auto** p, int64_t count) -> bool {
+    if (hipMalloc((void**)p, sizeof(**p) * count) == hipSuccess) return true;
+    (void)hipGetLastError();
+    *p = nullptr;
+    return false;
+  };
   unsigned long long* d_max = nullptr;
-  CSAW_HIP(hipMalloc(&d_max, sizeof(unsigned long long)));
+  if (!room(&d_max, 1)) return CSAW_OK;
   unsigned long long mx = 0;
   auto body = [&]() -> int {
     CSAW_HIP(hipMemsetAsync(d_max, 0, sizeof(unsigned long long), g->stream));
@@ -550,11 +561,17 @@ static int narrow_hubs(csaw_graph* g) {
     CSAW_HIP(hipMemcpyAsync(&mx, d_max, sizeof(mx), hipMemcpyDeviceToHost, g->stream));
     CSAW_HIP(hipStreamSynchronize(g->stream));
     if (mx >= (1ull << 32)) return CSAW_OK;
-    CSAW_HIP(hipMalloc(&g->hub_cdf32, sizeof(uint32_t) * npad));
+    if (!room(&g->hub_cdf32, npad)) return CSAW_OK;
     CSAW_HIP(hipMemsetAsync(g->hub_cdf32, 0, sizeof(uint32_t) * npad, g->stream));
     k_narrow_u32<<<grid_for(n, 256, g->num_cu), 256, 0, g->stream>>>(g->hub_cdf[0], n, g->hub_cdf32);
     CSAW_LAUNCH_CHECK();
-    CSAW_TRY(build_index<uint32_t>(g->hub_cdf32, n, &g->hub_idx32, g->stream, g->num_cu));
+    if (!room(&g->hub_idx32, std::max<int64_t>(cdf_index_size(n), 16))) {
+      CSAW_HIP(hipStreamSynchronize(g->stream));
+      (void)hipFree(g->hub_cdf32);
+      g->hub_cdf32 = nullptr;
+      return CSAW_OK;
+    }
+    CSAW_TRY(build_index<uint32_t>(g->hub_cdf32, n, g->hub_idx32, g->stream, g->num_cu));
     g->build32 = true;
     return CSAW_OK;
   };
