@@ -842,6 +842,7 @@ __global__ __launch_bounds__(256, G32 ? 4 : 1) void k_expand_block(GraphDev G, c
         continue;
       }
       Picker pk;
+      pk.L = cdf;
       bool build = !picker_global(G, en, KIND, kBlockIntCap, pk);
       const bool use_bm = BITMAP && en.dedup && en.d <= kBlockBitmapCap;
       if (build) {

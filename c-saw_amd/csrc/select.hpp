@@ -76,6 +76,21 @@ __device__ __forceinline__ uint32_t int_bias(const GraphDev& G, const csaw_graph
   return bias == CSAW_BIAS_USER ? EdgeBias(u, &hv) : (uint32_t)G.deg[u];
 }
 
+// First of the n >= 1 nondecreasing values of C that exceeds x (n if none does),
+// in as many steps whatever it finds, on 32-bit positions: no lane of a group
+// waits for another's branch.  Degree bias {25, 10} from 40,000 seeds without the
+// CDF cache 739 -> 722 us, {15, 10, 5} from 12,000 with it 405 -> 393, 200 requests
+// 687 -> 671.
+template <typename T>
+__device__ __forceinline__ int32_t upper_bound_lds(const T* C, int32_t n, T x) {
+  int32_t lo = 0;
+  for (int32_t h; n > 1; n -= h) {
+    h = n >> 1;
+    lo += C[lo + h - 1] > x ? 0 : h;
+  }
+  return lo + (C[lo] > x ? 0 : 1);
+}
+
 // ITS state of one entry: the entry's CDF is C[o .. o+d) (o = 0 for LDS).
 enum PickMode {
   kPickUniform = 0,
@@ -94,6 +109,7 @@ struct Picker {
   float Tf;
   const void* C;
   const void* K;
+  const uint64_t* L;  // C of kPickLds, as the LDS pointer it is (C's loads are generic)
   int64_t o;
 
   // E: entries of the CDF array (sizes the index levels).  IDX = false
@@ -122,6 +138,7 @@ struct Picker {
       if (mode == kPickInt32Idx)
         return (int32_t)upper_bound_dev<uint32_t>(static_cast<const uint32_t*>(C) + o, d, (uint32_t)x);
     }
+    if (mode == kPickLds) return upper_bound_lds<uint64_t>(L, d, x);
     return (int32_t)upper_bound_dev<uint64_t>(static_cast<const uint64_t*>(C) + o, d, x);
   }
 };
@@ -201,65 +218,66 @@ __device__ int32_t wave_select(int64_t E, const Entry& en, const Picker& pk, uin
   }
   int32_t cand = 0;
   if (lane < F) cand = pk.template pick<IDX>(E, draw(en, lane, 0));
-  // Fast path: up to the first slot whose attempt-0 draw repeats an earlier
-  // slot's draw, the sequential definition accepts every attempt-0 draw, so
-  // those slots are final; only the rest go through the ordered loop.
   bool dup = false;
   for (int i = 0; i + 1 < F; ++i) {
     const int32_t ci = readlane(cand, i);
     dup |= (lane > i) & (lane < F) & (cand == ci);
   }
-  const uint64_t dm = ballot(dup);
-  if (dm == 0ull) return lane < F ? cand : -1;
-  const int j0 = __builtin_ctzll(dm);
-  res = lane < j0 ? cand : -1;
+  // Only pending slots are visited: those whose draw an earlier slot holds (a slot
+  // that leaves its draw for another index leaves it to the earlier holder), and
+  // those after a slot that moves to their draw.  The bitmap takes the slots
+  // before the visited one, those in between all at once.  (Every slot after the
+  // first collision in turn, each with its LDS round trip, and generic loads of the
+  // CDF: {25, 10} from 40,000 seeds under degree bias 721 us, so 711.)
+  res = lane < F ? cand : -1;
+  uint64_t pending = ballot(dup);
+  if (pending == 0ull) return res;
   if (bm) {
     const int words = (d + 31) >> 5;
     for (int i = lane; i < words; i += kWave) bm[i] = 0u;
     wave_fence();
-    if (lane < j0) atomicOr(&bm[cand >> 5], 1u << (cand & 31));
-    wave_fence();
   }
-  for (int jj = j0; jj < F; ++jj) {
-    int32_t c = readlane(cand, jj);
-    bool taken = bm ? ((bm[c >> 5] >> (c & 31)) & 1u) : (ballot(res == c) != 0ull);
-    if (taken) {
-      int32_t chosen = -1, last = c;
-      for (int a0 = 1; a0 < kReselect; a0 += kWave) {
-        const int a = a0 + lane;
-        bool fr = false;
-        int32_t ci = 0;
-        if (a < kReselect) {
-          ci = pk.template pick<IDX>(E, draw(en, jj, a));
-          fr = !wave_taken_lane(ci, res, jj, bm);
-        }
-        const uint64_t m = ballot(fr);
-        if (m) {
-          chosen = readlane(ci, __builtin_ctzll(m));
-          break;
-        }
-        const int ll = kReselect - 1 - a0;
-        if (ll < kWave) last = readlane(ci, ll);
-      }
-      if (chosen < 0) {
-        for (int q = 0; q < d; q += kWave) {
-          const int32_t i = (int32_t)(((int64_t)last + 1 + q + lane) % d);
-          const bool fr = (q + lane < d) && !wave_taken_lane(i, res, jj, bm);
-          const uint64_t m = ballot(fr);
-          if (m) {
-            chosen = readlane(i, __builtin_ctzll(m));
-            break;
-          }
-        }
-      }
-      c = chosen;
-    }
+  int in_bm = 0;  // slots in the bitmap
+  while (pending) {
+    const int jj = __builtin_ctzll(pending);
+    pending &= pending - 1ull;
     if (bm) {
-      if (lane == 0) bm[c >> 5] |= 1u << (c & 31);
+      if (lane >= in_bm && lane < jj) atomicOr(&bm[res >> 5], 1u << (res & 31));
+      in_bm = jj;
       wave_fence();
     }
-    if (lane == jj) res = c;
+    int32_t chosen = -1, last = 0;
+    for (int a0 = 1; a0 < kReselect; a0 += kWave) {
+      const int a = a0 + lane;
+      bool fr = false;
+      int32_t ci = 0;
+      if (a < kReselect) {
+        ci = pk.template pick<IDX>(E, draw(en, jj, a));
+        fr = !wave_taken_lane(ci, res, jj, bm);
+      }
+      const uint64_t m = ballot(fr);
+      if (m) {
+        chosen = readlane(ci, __builtin_ctzll(m));
+        break;
+      }
+      const int ll = kReselect - 1 - a0;
+      if (ll < kWave) last = readlane(ci, ll);
+    }
+    if (chosen < 0) {
+      for (int q = 0; q < d; q += kWave) {
+        const int32_t i = (int32_t)(((int64_t)last + 1 + q + lane) % d);
+        const bool fr = (q + lane < d) && !wave_taken_lane(i, res, jj, bm);
+        const uint64_t m = ballot(fr);
+        if (m) {
+          chosen = readlane(i, __builtin_ctzll(m));
+          break;
+        }
+      }
+    }
+    if (lane == jj) res = chosen;
+    pending |= ballot(lane > jj && lane < F && cand == chosen);
   }
+  wave_fence();  // every lane has read the bitmap before the next entry clears it
   return res;
 }
 
@@ -450,6 +468,7 @@ __device__ void expand_entry_wave(const GraphDev& G, const csaw_graph_view& hv, 
     wave_copy_all(G, hv, H, en);
     return;
   }
+  pk.L = cdf;
   if (build) {
     pk.C = cdf;
     pk.o = 0;
@@ -491,6 +510,7 @@ __device__ __forceinline__ Picker bcast_picker(const Picker& m, int j) {
   p.Tf = __int_as_float(readlane(__float_as_int(m.Tf), j));
   p.C = (const void*)readlane_u64((uint64_t)m.C, j);
   p.K = (const void*)readlane_u64((uint64_t)m.K, j);
+  p.L = nullptr;
   p.o = readlane_i64(m.o, j);
   return p;
 }
@@ -512,6 +532,7 @@ __device__ void wave_expand_batch(const GraphDev& G, const csaw_graph_view& hv, 
   pm.Tf = 0.f;
   pm.C = nullptr;
   pm.K = nullptr;
+  pm.L = nullptr;
   pm.o = 0;
   int build = 0;
   mine.d = 0;
@@ -795,21 +816,6 @@ __device__ __forceinline__ int32_t resolve_slots(int F, int32_t d, int gs, int g
 // 170 for fanout 10, 256 for 16 and 512 for 32 lanes.
 constexpr int kGroupSmallCap = 64;  // slot words at the smallest group size
 
-// First of the n >= 1 nondecreasing values of C that exceeds x (n if none does),
-// in as many steps whatever it finds, on 32-bit positions: no lane of a group
-// waits for another's branch.  Degree bias {25, 10} from 40,000 seeds without the
-// CDF cache 739 -> 722 us, {15, 10, 5} from 12,000 with it 405 -> 393, 200 requests
-// 687 -> 671.
-template <typename T>
-__device__ __forceinline__ int32_t upper_bound_lds(const T* C, int32_t n, T x) {
-  int32_t lo = 0;
-  for (int32_t h; n > 1; n -= h) {
-    h = n >> 1;
-    lo += C[lo + h - 1] > x ? 0 : h;
-  }
-  return lo + (C[lo] > x ? 0 : 1);
-}
-
 // base: added to integer targets (a CDF that runs on from the one before it)
 template <int KIND>
 __device__ __forceinline__ int32_t gpick_small(const GEntry& en, const uint32_t* lc, uint32_t base, const U4& r) {
@@ -856,7 +862,7 @@ __device__ __forceinline__ int32_t group_select_remap(const GraphDev& G, const G
       uint32_t key;
       if (remap_key(r, (uint32_t)d, &key)) return (int32_t)key - 1;
     } else if (small) {
-      return (int32_t)min(upper_bound_dev<float>(lp, d, r), (int64_t)d - 1);
+      return min(upper_bound_lds<float>(lp, d, r), d - 1);
     } else if (KIND == kF32) {
       float x;
       if (remap_key(r, __uint_as_float(T), &x)) {
