@@ -77,8 +77,8 @@ struct GraphDev {
   const int32_t* hub_vid;       // sorted ids of vertices with degree > kHubMin
   const int64_t* hub_pool;      // pool offset per hub (n_hubs + 1)
   const uint64_t* hub_cdf[2];   // [DEGREE, USER]: inclusive uint64 CDFs of hubs
-  // the DEGREE hub CDFs as uint32 with their 16-ary index (hub_entries of them),
-  // and no vertex of degree <= kHubMin can total 2^32 either: integer CDFs are
+  // the DEGREE hub CDFs as uint32 with their 16-ary index (hub_entries < 2^32 of
+  // them), and no vertex of degree <= kHubMin can total 2^32 either: integer CDFs are
   // built and searched with 32-bit keys (null: some total may not fit)
   const uint32_t* hub_cdf32;
   const uint32_t* hub_idx32;

@@ -541,10 +541,12 @@ static int build_index(const T* C, int64_t E, T** out, hipStream_t stream, int n
 }
 
 // The DEGREE hub CDFs as uint32, padded and indexed like the CDF cache, when
-// their totals fit (duplicate neighbours can total more than E) and there is
-// room for them; without them every entry keeps to the uint64 hubs.
+// their totals fit (duplicate neighbours can total more than E), so do the hubs'
+// places among them (the batch build keeps a place beside its total in 64 bits),
+// and there is room for them; without them every entry keeps to the uint64 hubs.
 static int narrow_hubs(csaw_graph* g) {
   const int64_t n = g->hub_entries, npad = pad16(n);
+  if (n > (int64_t)UINT32_MAX) return CSAW_OK;
   auto room = [](auto** p, int64_t count) -> bool {
     if (hipMalloc((void**)p, sizeof(**p) * count) == hipSuccess) return true;
     (void)hipGetLastError();

@@ -1,0 +1,79 @@
+// Checks of the library's host code on the host, over the HIP runtime of
+// fake_hip.hpp: what is asked of the runtime, in which order, and what the
+// library does when a call fails.  One check per run, named by the argument.
+#include "fake_hip.hpp"
+
+#include <cstdlib>
+#include <functional>
+
+#include "../../include/csaw.h"
+
+#define NEED(x)                                                                                 \
+  do {                                                                                          \
+    if (!(x)) {                                                                                 \
+      std::printf("line %d: %s (last error: %s)\n", __LINE__, #x, csaw_last_error());           \
+      std::exit(1);                                                                             \
+    }                                                                                           \
+  } while (0)
+
+// V vertices of degree d each; ids are read by no host code and reserved only
+static csaw_graph* regular_graph(int64_t V, int64_t d) {
+  std::vector<int64_t> off(V + 1);
+  for (int64_t v = 0; v <= V; ++v) off[v] = v * d;
+  const size_t bytes = sizeof(int32_t) * (size_t)off[V] + 1;
+  void* ids = mmap(nullptr, bytes, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+  NEED(ids != MAP_FAILED);
+  csaw_graph* g = nullptr;
+  NEED(csaw_graph_create(off.data(), 1, (const int32_t*)ids, nullptr, V, off[V], &g) == CSAW_OK);
+  munmap(ids, bytes);
+  return g;
+}
+
+static csaw_request request(int32_t samples, std::vector<int32_t> fanouts, int32_t bias, const int32_t* seeds) {
+  csaw_request r;
+  memset(&r, 0, sizeof(r));
+  r.samples = samples;
+  r.depth = (int32_t)fanouts.size();
+  for (size_t h = 0; h < fanouts.size(); ++h) r.fanouts[h] = fanouts[h];
+  r.bias = bias;
+  r.dedup = 1;
+  r.seeds = seeds;
+  return r;
+}
+
+// Degree bias over hubs whose lists hold 2^32 entries and more together: a CDF's
+// place among them does not fit the 32 bits that the batch build keeps of it, so
+// such a graph is searched by the kernels that keep 64.
+static void hub_positions() {
+  const int64_t d = 4097;  // hubs: beyond 1,024 neighbours
+  const int32_t n = 40000;
+  std::vector<int32_t> seeds(n, 0);
+  const csaw_request r = request(n, {25, 10}, CSAW_BIAS_DEGREE, seeds.data());
+  auto batch_built = [&](int64_t V) {
+    csaw_graph* g = regular_graph(V, d);
+    csaw_plan* p = nullptr;
+    NEED(csaw_plan_create(g, &r, 1, nullptr, &p) == CSAW_OK);
+    fake().log.clear();
+    NEED(csaw_plan_run(p, nullptr, 1) == CSAW_OK);
+    NEED(fake().logged("k_expand_plain"));
+    const bool built = fake().logged("k_expand_plainILi1ELb0ELi1ELb0ELb1E");
+    csaw_plan_destroy(p);
+    csaw_graph_destroy(g);
+    return built;
+  };
+  const int64_t fit = ((int64_t(1) << 32) - 1) / d;
+  NEED(batch_built(1000));
+  NEED(batch_built(fit));
+  NEED(!batch_built(fit + 1));
+}
+
+int main(int argc, char** argv) {
+  const std::map<std::string, std::function<void()>> checks = {
+      {"hub_positions", hub_positions},
+  };
+  const auto it = checks.find(argc > 1 ? argv[1] : "");
+  if (it == checks.end()) return 2;
+  it->second();
+  std::printf("ok\n");
+  return 0;
+}
