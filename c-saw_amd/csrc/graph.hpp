@@ -11,6 +11,7 @@ namespace csaw {
 // The streams and events one plan uses at a time.
 struct PlanStreams {
   static constexpr int kSide = 3;
+  int device = -1;
   hipStream_t main = nullptr, side[kSide] = {};
   hipEvent_t begin = nullptr, end = nullptr;  // of a synchronised run
   hipEvent_t fork = nullptr, join[kSide] = {};
@@ -22,13 +23,16 @@ struct PlanStreams {
 // graph (a call of the sampler makes a plan and destroys it).  At most kHeldBytes
 // in blocks of at most kBlockBytes and kHeldStreams stream sets; what the graph
 // still holds when it is destroyed goes back to the device, and an allocation
-// that fails gives everything back and tries again.  The owner of a block waits
-// for its work before give(); take() and give() may be called from any thread.
+// that fails gives everything back and tries again.  What is handed out is of the
+// device that is current then, as a fresh allocation would be.  The owner of a
+// block waits for its work before give(); take() and give() may be called from
+// any thread, whatever device is current there.
 struct Workspace {
   static constexpr size_t kHeldBytes = 256u << 20, kBlockBytes = 128u << 20, kHeldStreams = 8;
   struct Block {
     void* p = nullptr;
     size_t bytes = 0;
+    int device = -1;
   };
   int take(size_t bytes, Block* b);
   void give(Block b);

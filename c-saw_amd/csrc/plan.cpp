@@ -115,11 +115,13 @@ void PlanStreams::destroy() {
 }
 
 int Workspace::take(size_t bytes, Block* b) {
+  int device = 0;
+  CSAW_HIP(hipGetDevice(&device));
   {
     std::lock_guard<std::mutex> lock(mu);
     size_t best = blocks.size();
     for (size_t i = 0; i < blocks.size(); ++i)
-      if (blocks[i].bytes >= bytes && blocks[i].bytes <= 4 * bytes + (1u << 20) &&
+      if (blocks[i].device == device && blocks[i].bytes >= bytes && blocks[i].bytes <= 4 * bytes + (1u << 20) &&
           (best == blocks.size() || blocks[i].bytes < blocks[best].bytes))
         best = i;
     if (best < blocks.size()) {
@@ -130,6 +132,7 @@ int Workspace::take(size_t bytes, Block* b) {
     }
   }
   b->bytes = (bytes + 65535) & ~(size_t)65535;
+  b->device = device;
   if (hipMalloc(&b->p, b->bytes) != hipSuccess) {
     (void)hipGetLastError();
     trim();
@@ -152,13 +155,18 @@ void Workspace::give(Block b) {
 }
 
 int Workspace::take_streams(bool with_side, PlanStreams* s) {
+  int device = 0;
+  CSAW_HIP(hipGetDevice(&device));
   {
     std::lock_guard<std::mutex> lock(mu);
-    if (!streams.empty()) {
-      *s = streams.back();
-      streams.pop_back();
-    }
+    for (size_t i = streams.size(); i-- > 0;)
+      if (streams[i].device == device) {
+        *s = streams[i];
+        streams.erase(streams.begin() + i);
+        break;
+      }
   }
+  s->device = device;
   return s->create(with_side);
 }
 
@@ -196,11 +204,21 @@ void Workspace::close() {
 
 }  // namespace csaw
 
+// Waits for everything on `device`, which need not be the current one.
+static hipError_t wait_for_device(int device) {
+  int cur = device;
+  hipError_t e = hipGetDevice(&cur);
+  if (e == hipSuccess && cur != device) e = hipSetDevice(device);
+  if (e == hipSuccess) e = hipDeviceSynchronize();
+  if (cur != device) (void)hipSetDevice(cur);
+  return e;
+}
+
 static void plan_free(csaw_plan* p) {
   if (!p) return;
   // work that a call has not waited for may still use the workspace, on a stream
   // of the caller's
-  if (p->busy) (void)hipDeviceSynchronize();
+  if (p->busy) (void)wait_for_device(p->slab.device);
   if (p->gexec) (void)hipGraphExecDestroy(p->gexec);
   if (p->work) {
     p->work->give(p->slab);

@@ -67,9 +67,42 @@ static void hub_positions() {
   NEED(!batch_built(fit + 1));
 }
 
+// A plan run but not waited for, destroyed while another device is current: the
+// wait is for the plan's device, and the caller's device stays current.  What the
+// plan held goes to the next plan of its device and to none of another's.
+static void wait_on_own_device() {
+  csaw_graph* g = regular_graph(100, 8);
+  const std::vector<int32_t> seeds(50, 1);
+  const csaw_request r = request(50, {4, 4}, CSAW_BIAS_UNIFORM, seeds.data());
+  csaw_plan_opts o;
+  memset(&o, 0, sizeof(o));
+  o.mode = CSAW_MODE_BATCHED;
+  csaw_plan *p = nullptr, *q = nullptr;
+  NEED(csaw_plan_create(g, &r, 1, &o, &p) == CSAW_OK);
+  NEED(csaw_plan_run(p, nullptr, 0) == CSAW_OK);
+  fake().device = 1;
+  fake().log.clear();
+  csaw_plan_destroy(p);
+  NEED(fake().logged("wait for device 0"));
+  NEED(!fake().logged("wait for device 1"));
+  NEED(fake().device == 1);
+  const size_t before = fake().allocs.size();
+  const uintptr_t handles = fake().handles;
+  NEED(csaw_plan_create(g, &r, 1, &o, &p) == CSAW_OK);  // of device 1
+  NEED(fake().allocs.size() == before + 1 && fake().handles > handles);
+  fake().device = 0;
+  const uintptr_t made = fake().handles;
+  NEED(csaw_plan_create(g, &r, 1, &o, &q) == CSAW_OK);  // of device 0: what p left
+  NEED(fake().allocs.size() == before + 1 && fake().handles == made);
+  csaw_plan_destroy(p);
+  csaw_plan_destroy(q);
+  csaw_graph_destroy(g);
+}
+
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> checks = {
       {"hub_positions", hub_positions},
+      {"wait_on_own_device", wait_on_own_device},
   };
   const auto it = checks.find(argc > 1 ? argv[1] : "");
   if (it == checks.end()) return 2;

@@ -30,3 +30,7 @@ def run(exe, name):
 
 def test_hub_positions_past_32_bits(host_check):
     run(host_check, "hub_positions")
+
+
+def test_unwaited_plan_waits_on_its_own_device(host_check):
+    run(host_check, "wait_on_own_device")
