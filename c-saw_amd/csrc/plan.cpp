@@ -217,12 +217,16 @@ static hipError_t wait_for_device(int device) {
 static void plan_free(csaw_plan* p) {
   if (!p) return;
   // work that a call has not waited for may still use the workspace, on a stream
-  // of the caller's
-  if (p->busy) (void)wait_for_device(p->slab.device);
+  // of the caller's; where that wait fails nothing goes back to the pool
+  const bool idle = !p->busy || wait_for_device(p->slab.device) == hipSuccess;
+  if (!idle) (void)hipGetLastError();
   if (p->gexec) (void)hipGraphExecDestroy(p->gexec);
-  if (p->work) {
+  if (p->work && idle) {
     p->work->give(p->slab);
     p->work->give_streams(p->st);
+  } else {
+    (void)hipFree(p->slab.p);
+    p->st.destroy();
   }
   delete p;
 }

@@ -99,10 +99,35 @@ static void wait_on_own_device() {
   csaw_graph_destroy(g);
 }
 
+// A wait that fails leaves the plan's work where it may be: its memory and
+// streams go to no other plan.
+static void failed_wait() {
+  csaw_graph* g = regular_graph(100, 8);
+  const std::vector<int32_t> seeds(50, 1);
+  const csaw_request r = request(50, {4, 4}, CSAW_BIAS_UNIFORM, seeds.data());
+  csaw_plan_opts o;
+  memset(&o, 0, sizeof(o));
+  o.mode = CSAW_MODE_BATCHED;
+  csaw_plan* p = nullptr;
+  NEED(csaw_plan_create(g, &r, 1, &o, &p) == CSAW_OK);
+  NEED(csaw_plan_run(p, nullptr, 0) == CSAW_OK);
+  fake().fail_in["hipDeviceSynchronize"] = 1;
+  fake().log.clear();
+  csaw_plan_destroy(p);
+  NEED(fake().logged("free on 0"));
+  const size_t before = fake().allocs.size();
+  const uintptr_t handles = fake().handles;
+  NEED(csaw_plan_create(g, &r, 1, &o, &p) == CSAW_OK);
+  NEED(fake().allocs.size() == before + 1 && fake().handles > handles);
+  csaw_plan_destroy(p);
+  csaw_graph_destroy(g);
+}
+
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> checks = {
       {"hub_positions", hub_positions},
       {"wait_on_own_device", wait_on_own_device},
+      {"failed_wait", failed_wait},
   };
   const auto it = checks.find(argc > 1 ? argv[1] : "");
   if (it == checks.end()) return 2;

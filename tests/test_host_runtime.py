@@ -34,3 +34,7 @@ def test_hub_positions_past_32_bits(host_check):
 
 def test_unwaited_plan_waits_on_its_own_device(host_check):
     run(host_check, "wait_on_own_device")
+
+
+def test_nothing_is_pooled_after_a_failed_wait(host_check):
+    run(host_check, "failed_wait")
