@@ -218,7 +218,7 @@ static void plan_free(csaw_plan* p) {
   if (!p) return;
   // work that a call has not waited for may still use the workspace, on a stream
   // of the caller's; where that wait fails nothing goes back to the pool
-  const bool idle = !p->busy || wait_for_device(p->slab.device) == hipSuccess;
+  const bool idle = p->unwaited == 0 || wait_for_device(p->slab.device) == hipSuccess;
   if (!idle) (void)hipGetLastError();
   if (p->gexec) (void)hipGraphExecDestroy(p->gexec);
   if (p->work && idle) {
@@ -663,15 +663,15 @@ static int plan_create(csaw_graph* g, const csaw_request* reqs, int32_t n_req, c
     c.base = static_cast<char*>(p->slab.p);
     plan_layout(p, z, c, &filled);
     p->h_state.assign((kCtrBytes + kBoundsBytes * (size_t)n_req) / sizeof(uint32_t), 0u);
+    InFlight upload(p->unwaited);
     if (z.mlp) CSAW_TRY(mlp_upload_bf16(o.mlp, p->d_mlp));
     CSAW_TRY(p->work->take_streams(o.mode == CSAW_MODE_BATCHED && !o.serial_expand, &p->st));
     p->stream = p->st.main;
     p->fan = o.mode == CSAW_MODE_BATCHED && !o.serial_expand;
-    p->busy = true;
     CSAW_TRY(upload_inputs(p, reqs, filled));
     // (csaw_sample runs on the same stream and waits there)
     if (!stage) CSAW_HIP(hipStreamSynchronize(p->stream));
-    p->busy = false;
+    upload.waited();
     p->timer.enabled = o.timing != 0;
     return CSAW_OK;
   };
@@ -695,8 +695,7 @@ extern "C" int csaw_plan_run(csaw_plan* p, void* stream, int sync) {
   p->hop_logs.clear();
   p->pending_log_hops.clear();
   p->bounds_known = false;
-  const bool was_busy = p->busy;  // (by work on another stream, perhaps)
-  p->busy = true;
+  InFlight run(p->unwaited);
   TimingHook* th = p->timer.enabled ? &p->timer : nullptr;
   const bool wait = sync || th;
   if (wait) CSAW_HIP(hipEventRecord(p->st.begin, st));
@@ -739,7 +738,7 @@ extern "C" int csaw_plan_run(csaw_plan* p, void* stream, int sync) {
     CSAW_HIP(hipMemcpyAsync(p->h_state.data(), p->counters, sizeof(uint32_t) * p->h_state.size(), hipMemcpyDeviceToHost,
                             st));
     CSAW_HIP(hipStreamSynchronize(st));
-    p->busy = was_busy;
+    run.waited();
     float ms = 0.f;
     CSAW_HIP(hipEventElapsedTime(&ms, p->st.begin, p->st.end));
     p->last_ms = ms;
@@ -854,9 +853,12 @@ extern "C" int csaw_plan_copy_device(const csaw_plan* p, int32_t req, int32_t* s
   std::vector<int64_t> lo, hi;
   CSAW_TRY(request_bounds(p, req, lo, hi));
   hipStream_t st = stream ? (hipStream_t)stream : p->stream;
-  if (!sync) p->busy = true;
+  InFlight copy(p->unwaited);
   CSAW_TRY(copy_edges_device(p, req, lo, hi, src, dst, sample, hop_offsets, st));
-  if (sync) CSAW_HIP(hipStreamSynchronize(st));
+  if (sync) {
+    CSAW_HIP(hipStreamSynchronize(st));
+    copy.waited();
+  }
   return CSAW_OK;
 }
 
@@ -867,6 +869,7 @@ extern "C" int csaw_plan_digest(const csaw_plan* p, int32_t req, uint64_t* diges
   const auto [ui, k] = p->req_unit[req];
   const Unit& u = p->units[ui];
   unsigned long long* d;
+  InFlight sum(p->unwaited);
   CSAW_HIP(hipMalloc(&d, sizeof(unsigned long long)));
   CSAW_HIP(hipMemsetAsync(d, 0, sizeof(unsigned long long), p->stream));
   int64_t at = 0;
@@ -879,6 +882,7 @@ extern "C" int csaw_plan_digest(const csaw_plan* p, int32_t req, uint64_t* diges
   if (st == CSAW_OK) {
     CSAW_HIP(hipMemcpyAsync(&v, d, sizeof(v), hipMemcpyDeviceToHost, p->stream));
     CSAW_HIP(hipStreamSynchronize(p->stream));
+    sum.waited();
   }
   (void)hipFree(d);
   *digest = (uint64_t)v ^ ((uint64_t)at * 0x100000001b3ull);
@@ -966,10 +970,12 @@ struct csaw_edges {
 static int copy_staged(const csaw_plan* p, const std::vector<int64_t>& lo, const std::vector<int64_t>& hi, csaw_edges* e) {
   int64_t* off = reinterpret_cast<int64_t*>(p->staging);
   int32_t* col = reinterpret_cast<int32_t*>(off + e->n_off);
+  InFlight copy(p->unwaited);
   CSAW_TRY(copy_edges_device(p, 0, lo, hi, col, col + e->n, col + 2 * e->n, off, p->stream));
   CSAW_HIP(hipMemcpyAsync(e->block.get(), p->staging, sizeof(int64_t) * e->n_off + 3 * sizeof(int32_t) * e->n,
                           hipMemcpyDeviceToHost, p->stream));
   CSAW_HIP(hipStreamSynchronize(p->stream));
+  copy.waited();
   return CSAW_OK;
 }
 

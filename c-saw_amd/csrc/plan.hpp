@@ -1,5 +1,6 @@
 // Host-side plan state (see plan.cpp).
 #pragma once
+#include <atomic>
 #include <utility>
 #include <vector>
 
@@ -70,6 +71,15 @@ void apply_tuning(LaunchCfg& L, const csaw_tuning* t);
 int validate_tuning(const csaw_tuning* t);
 int mlp_upload_bf16(const csaw_mlp* m, uint16_t* dst);
 
+// A call's device work on a plan's arrays, counted from before its first launch
+// until the call has waited for it.  A call that does not wait, or whose launch or
+// wait fails, leaves its count.
+struct InFlight {
+  std::atomic<int>& n;
+  explicit InFlight(std::atomic<int>& count) : n(count) { ++n; }
+  void waited() { --n; }
+};
+
 }  // namespace csaw
 
 struct csaw_plan {
@@ -86,11 +96,10 @@ struct csaw_plan {
   uint64_t* grp_excl = nullptr;
   csaw::Chunk* chunks = nullptr;
   uint32_t chunk_cap = 0;
-  // every device array below and the units' (one allocation), its work waited for
-  // by the calls themselves unless busy
+  // every device array below and the units' (one allocation)
   std::shared_ptr<csaw::Workspace> work;
   csaw::Workspace::Block slab;
-  mutable bool busy = false;
+  mutable std::atomic<int> unwaited{0};  // calls whose work may still use it (InFlight)
   int32_t* staging = nullptr;         // csaw_sample: the result, packed for one copy
   // counter block, then the requests' edge bounds (kCtrBytes + n_req *
   // kBoundsBytes): one copy into h_state after a synchronised run brings the

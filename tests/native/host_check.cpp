@@ -123,11 +123,60 @@ static void failed_wait() {
   csaw_graph_destroy(g);
 }
 
+// Calls that wait for what they launch and fail before they have: the plan is
+// waited for when it goes, before its memory is anyone else's.
+static void failed_copy_out() {
+  csaw_graph* g = regular_graph(100, 8);
+  const std::vector<int32_t> seeds(50, 1);
+  auto waits = [&](const std::function<void()>& destroy) {
+    fake().log.clear();
+    destroy();
+    return fake().logged("wait for device 0");
+  };
+  // csaw_sample: the run waits and brings the bounds home (the first copy), then
+  // the edges are packed and copied (the second)
+  csaw_params prm;
+  memset(&prm, 0, sizeof(prm));
+  prm.samples = 50;
+  prm.frontier_size = 1;
+  prm.neighbor_size = 4;
+  prm.depth = 2;
+  prm.dedup = 1;
+  csaw_edges* e = nullptr;
+  NEED(!waits([&] { NEED(csaw_sample(g, &prm, seeds.data(), &e, nullptr) == CSAW_OK); }));
+  csaw_edges_free(e);
+  NEED(waits([&] {
+    fake().fail_in["hipMemcpyAsync"] = 2;
+    NEED(csaw_sample(g, &prm, seeds.data(), &e, nullptr) != CSAW_OK && !e);
+  }));
+  NEED(waits([&] {
+    fake().fail_in["hipStreamSynchronize"] = 2;
+    NEED(csaw_sample(g, &prm, seeds.data(), &e, nullptr) != CSAW_OK && !e);
+  }));
+  // a plan's copy to device buffers and its digest
+  const csaw_request r = request(50, {4, 4}, CSAW_BIAS_UNIFORM, seeds.data());
+  std::vector<int32_t> out(3000);
+  uint64_t digest = 0;
+  for (int what = 0; what < 3; ++what) {
+    csaw_plan* p = nullptr;
+    NEED(csaw_plan_create(g, &r, 1, nullptr, &p) == CSAW_OK);
+    NEED(csaw_plan_run(p, nullptr, 1) == CSAW_OK);
+    NEED(csaw_plan_copy_device(p, 0, out.data(), nullptr, nullptr, nullptr, nullptr, 1) == CSAW_OK);
+    NEED(csaw_plan_digest(p, 0, &digest) == CSAW_OK);
+    if (what) fake().fail_in["hipStreamSynchronize"] = 1;
+    if (what == 1) NEED(csaw_plan_copy_device(p, 0, out.data(), nullptr, nullptr, nullptr, nullptr, 1) != CSAW_OK);
+    if (what == 2) NEED(csaw_plan_digest(p, 0, &digest) != CSAW_OK);
+    NEED(waits([&] { csaw_plan_destroy(p); }) == (what != 0));
+  }
+  csaw_graph_destroy(g);
+}
+
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> checks = {
       {"hub_positions", hub_positions},
       {"wait_on_own_device", wait_on_own_device},
       {"failed_wait", failed_wait},
+      {"failed_copy_out", failed_copy_out},
   };
   const auto it = checks.find(argc > 1 ? argv[1] : "");
   if (it == checks.end()) return 2;

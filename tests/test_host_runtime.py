@@ -38,3 +38,7 @@ def test_unwaited_plan_waits_on_its_own_device(host_check):
 
 def test_nothing_is_pooled_after_a_failed_wait(host_check):
     run(host_check, "failed_wait")
+
+
+def test_calls_that_fail_before_they_have_waited(host_check):
+    run(host_check, "failed_copy_out")
