@@ -91,12 +91,11 @@ static int validate_request(const csaw_graph* g, const csaw_request& r) {
 namespace csaw {
 
 int PlanStreams::create(bool with_side) {
-  if (!main) {
-    CSAW_HIP(hipStreamCreateWithFlags(&main, hipStreamNonBlocking));
-    CSAW_HIP(hipEventCreate(&begin));
-    CSAW_HIP(hipEventCreate(&end));
-  }
-  if (with_side && !join[kSide - 1]) {
+  // (each by itself: an earlier call may have failed half-way)
+  if (!main) CSAW_HIP(hipStreamCreateWithFlags(&main, hipStreamNonBlocking));
+  if (!begin) CSAW_HIP(hipEventCreate(&begin));
+  if (!end) CSAW_HIP(hipEventCreate(&end));
+  if (with_side) {
     if (!fork) CSAW_HIP(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
     for (int i = 0; i < kSide; ++i) {
       if (!side[i]) CSAW_HIP(hipStreamCreateWithFlags(&side[i], hipStreamNonBlocking));

@@ -171,12 +171,36 @@ static void failed_copy_out() {
   csaw_graph_destroy(g);
 }
 
+// A set of streams and events that could be made in part only: the next plan
+// makes what it lacks.
+static void partial_streams() {
+  const std::vector<int32_t> seeds(50, 1);
+  const csaw_request r = request(50, {4, 4}, CSAW_BIAS_UNIFORM, seeds.data());
+  csaw_plan_opts o;
+  memset(&o, 0, sizeof(o));
+  o.mode = CSAW_MODE_BATCHED;
+  const std::pair<const char*, int> made[] = {
+      {"hipStreamCreateWithFlags", 4}, {"hipEventCreate", 2}, {"hipEventCreateWithFlags", 4}};
+  for (const auto& m : made)
+    for (int k = 1; k <= m.second; ++k) {
+      csaw_graph* g = regular_graph(100, 8);
+      csaw_plan* p = nullptr;
+      fake().fail_in[m.first] = k;
+      NEED(csaw_plan_create(g, &r, 1, &o, &p) != CSAW_OK);
+      NEED(csaw_plan_create(g, &r, 1, &o, &p) == CSAW_OK);
+      NEED(csaw_plan_run(p, nullptr, 1) == CSAW_OK);
+      csaw_plan_destroy(p);
+      csaw_graph_destroy(g);
+    }
+}
+
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> checks = {
       {"hub_positions", hub_positions},
       {"wait_on_own_device", wait_on_own_device},
       {"failed_wait", failed_wait},
       {"failed_copy_out", failed_copy_out},
+      {"partial_streams", partial_streams},
   };
   const auto it = checks.find(argc > 1 ? argv[1] : "");
   if (it == checks.end()) return 2;

@@ -42,3 +42,7 @@ def test_nothing_is_pooled_after_a_failed_wait(host_check):
 
 def test_calls_that_fail_before_they_have_waited(host_check):
     run(host_check, "failed_copy_out")
+
+
+def test_partly_made_streams_are_completed(host_check):
+    run(host_check, "partial_streams")
