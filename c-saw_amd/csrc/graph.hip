@@ -261,10 +261,10 @@ int graph_alloc_common(csaw_graph* g) {
 
 // Degree array + validation.
 static int finish_graph(csaw_graph* g) {
-  CSAW_HIP(hipMalloc(&g->deg, sizeof(int32_t) * (g->V > 0 ? g->V : 1)));
+  CSAW_HIP(device_malloc(&g->deg, sizeof(int32_t) * (g->V > 0 ? g->V : 1)));
   unsigned long long* dmax;
   uint32_t* bad;
-  CSAW_HIP(hipMalloc(&dmax, sizeof(unsigned long long) + sizeof(uint32_t)));
+  CSAW_HIP(device_malloc(&dmax, sizeof(unsigned long long) + sizeof(uint32_t)));
   bad = (uint32_t*)(dmax + 1);
   CSAW_HIP(hipMemsetAsync(dmax, 0, sizeof(unsigned long long) + sizeof(uint32_t), g->stream));
   if (g->V > 0) {
@@ -301,8 +301,8 @@ static int ensure_hub_list(csaw_graph* g) {
       vid.push_back((int32_t)v);
       pool.push_back(pool.back() + deg[v]);
     }
-  CSAW_HIP(hipMalloc(&g->hub_vid, sizeof(int32_t) * (vid.size() + 1)));
-  CSAW_HIP(hipMalloc(&g->hub_pool, sizeof(int64_t) * pool.size()));
+  CSAW_HIP(device_malloc(&g->hub_vid, sizeof(int32_t) * (vid.size() + 1)));
+  CSAW_HIP(device_malloc(&g->hub_pool, sizeof(int64_t) * pool.size()));
   if (!vid.empty())
     CSAW_HIP(hipMemcpy(g->hub_vid, vid.data(), sizeof(int32_t) * vid.size(), hipMemcpyHostToDevice));
   CSAW_HIP(hipMemcpy(g->hub_pool, pool.data(), sizeof(int64_t) * pool.size(), hipMemcpyHostToDevice));
@@ -322,7 +322,7 @@ int graph_prepare_bias(csaw_graph* g, int32_t bias) {
     if (!g->cdf) {
       // padded to 16 entries: the search index reads aligned 16-entry blocks
       const int64_t n = pad16(g->E > 0 ? g->E : 1);
-      CSAW_HIP(hipMalloc(&g->cdf, sizeof(float) * n));
+      CSAW_HIP(device_malloc(&g->cdf, sizeof(float) * n));
       CSAW_HIP(hipMemsetAsync(g->cdf, 0, sizeof(float) * n, g->stream));
       if (g->V > 0) {
         CSAW_TRY(ensure_hub_list(g));
@@ -348,7 +348,7 @@ int graph_prepare_bias(csaw_graph* g, int32_t bias) {
   if (g->hub_cdf[kind] || g->n_hubs == 0) return CSAW_OK;
   std::vector<int64_t> pool(g->n_hubs + 1);
   CSAW_HIP(hipMemcpy(pool.data(), g->hub_pool, sizeof(int64_t) * pool.size(), hipMemcpyDeviceToHost));
-  CSAW_HIP(hipMalloc(&g->hub_cdf[kind], sizeof(uint64_t) * g->hub_entries));
+  CSAW_HIP(device_malloc(&g->hub_cdf[kind], sizeof(uint64_t) * g->hub_entries));
   CSAW_TRY(hub_cdf_build(g->view(), g->hook_view(), kind, pool, g->hub_cdf[kind], g->stream, g->num_cu));
   if (fits) CSAW_TRY(narrow_hubs(g));
   CSAW_HIP(hipStreamSynchronize(g->stream));
@@ -376,10 +376,10 @@ int hub_cdf_build(const GraphDev& G, const csaw_graph_view& hv, int kind, const 
   int32_t *d_seg_hub, *d_seg_idx;
   int64_t* d_seg_first;
   uint64_t* d_seg_tot;
-  CSAW_HIP(hipMalloc(&d_seg_hub, sizeof(int32_t) * n_seg));
-  CSAW_HIP(hipMalloc(&d_seg_idx, sizeof(int32_t) * n_seg));
-  CSAW_HIP(hipMalloc(&d_seg_first, sizeof(int64_t) * seg_first.size()));
-  CSAW_HIP(hipMalloc(&d_seg_tot, sizeof(uint64_t) * n_seg));
+  CSAW_HIP(device_malloc(&d_seg_hub, sizeof(int32_t) * n_seg));
+  CSAW_HIP(device_malloc(&d_seg_idx, sizeof(int32_t) * n_seg));
+  CSAW_HIP(device_malloc(&d_seg_first, sizeof(int64_t) * seg_first.size()));
+  CSAW_HIP(device_malloc(&d_seg_tot, sizeof(uint64_t) * n_seg));
   CSAW_HIP(hipMemcpyAsync(d_seg_hub, seg_hub.data(), sizeof(int32_t) * n_seg, hipMemcpyHostToDevice, stream));
   CSAW_HIP(hipMemcpyAsync(d_seg_idx, seg_idx.data(), sizeof(int32_t) * n_seg, hipMemcpyHostToDevice, stream));
   CSAW_HIP(hipMemcpyAsync(d_seg_first, seg_first.data(), sizeof(int64_t) * seg_first.size(), hipMemcpyHostToDevice,
@@ -468,7 +468,7 @@ int graph_prepare_int_cache(csaw_graph* g, int32_t bias) {
   if (g->int_cdf[kind] || g->int_cdf32[kind]) return CSAW_OK;
   CSAW_TRY(graph_prepare_bias(g, bias));
   const int64_t n = pad16(g->E > 0 ? g->E : 1);
-  CSAW_HIP(hipMalloc(&g->int_cdf[kind], sizeof(uint64_t) * n));
+  CSAW_HIP(device_malloc(&g->int_cdf[kind], sizeof(uint64_t) * n));
   CSAW_HIP(hipMemsetAsync(g->int_cdf[kind], 0, sizeof(uint64_t) * n, g->stream));
   GraphDev G = g->view();
   csaw_graph_view hv = g->hook_view();
@@ -485,7 +485,7 @@ int graph_prepare_int_cache(csaw_graph* g, int32_t bias) {
   // Every per-vertex total below 2^32 (the largest entry is the largest
   // total): keep the cache as uint32, half the bytes per search.
   unsigned long long* d_max = nullptr;
-  CSAW_HIP(hipMalloc(&d_max, sizeof(unsigned long long)));
+  CSAW_HIP(device_malloc(&d_max, sizeof(unsigned long long)));
   CSAW_HIP(hipMemsetAsync(d_max, 0, sizeof(unsigned long long), g->stream));
   if (g->E > 0) {
     k_max_u64<<<grid_for(g->E, 256, g->num_cu), 256, 0, g->stream>>>(g->int_cdf[kind], g->E, d_max);
@@ -496,7 +496,7 @@ int graph_prepare_int_cache(csaw_graph* g, int32_t bias) {
   CSAW_HIP(hipStreamSynchronize(g->stream));
   CSAW_HIP(hipFree(d_max));
   if (mx < (1ull << 32) && !g->wide_int_cdf) {
-    CSAW_HIP(hipMalloc(&g->int_cdf32[kind], sizeof(uint32_t) * n));
+    CSAW_HIP(device_malloc(&g->int_cdf32[kind], sizeof(uint32_t) * n));
     k_narrow_u32<<<grid_for(n, 256, g->num_cu), 256, 0, g->stream>>>(g->int_cdf[kind], n, g->int_cdf32[kind]);
     CSAW_LAUNCH_CHECK();
     CSAW_HIP(hipStreamSynchronize(g->stream));
@@ -536,7 +536,7 @@ static int build_index(const T* C, int64_t E, T* out, hipStream_t stream, int nu
 
 template <typename T>
 static int build_index(const T* C, int64_t E, T** out, hipStream_t stream, int num_cu) {
-  CSAW_HIP(hipMalloc(out, sizeof(T) * std::max<int64_t>(cdf_index_size(E), 16)));
+  CSAW_HIP(device_malloc(out, sizeof(T) * std::max<int64_t>(cdf_index_size(E), 16)));
   return build_index(C, E, *out, stream, num_cu);
 }
 
@@ -548,8 +548,7 @@ static int narrow_hubs(csaw_graph* g) {
   const int64_t n = g->hub_entries, npad = pad16(n);
   if (n > (int64_t)UINT32_MAX) return CSAW_OK;
   auto room = [](auto** p, int64_t count) -> bool {
-    if (hipMalloc((void**)p, sizeof(**p) * count) == hipSuccess) return true;
-    (void)hipGetLastError();
+    if (device_malloc(p, sizeof(**p) * count) == hipSuccess) return true;
     *p = nullptr;
     return false;
   };
@@ -603,7 +602,7 @@ int graph_prepare_vertex_records(csaw_graph* g, int32_t bias) {
   if (k < 0 || g->vrec[k] || g->V == 0) return CSAW_OK;
   if (k == 2 && !g->cdf) return CSAW_OK;
   if (k < 2 && !g->int_cdf32[k]) return CSAW_OK;
-  CSAW_HIP(hipMalloc(&g->vrec[k], sizeof(VertexRecord) * g->V));
+  CSAW_HIP(device_malloc(&g->vrec[k], sizeof(VertexRecord) * g->V));
   const int grid = grid_for(g->V, 256, g->num_cu);
   if (k == 2)
     k_vertex_records<float><<<grid, 256, 0, g->stream>>>(g->off, g->cdf, g->V, g->vrec[k]);
@@ -734,13 +733,13 @@ extern "C" int csaw_graph_create(const void* offsets, int offsets_are_i64, const
   g->V = V;
   g->E = E;
   auto body = [&]() -> int {
-    CSAW_HIP(hipMalloc(&g->off, sizeof(int64_t) * (V + 1)));
-    CSAW_HIP(hipMalloc(&g->adj, sizeof(int32_t) * (E > 0 ? E : 1)));
+    CSAW_HIP(device_malloc(&g->off, sizeof(int64_t) * (V + 1)));
+    CSAW_HIP(device_malloc(&g->adj, sizeof(int32_t) * (E > 0 ? E : 1)));
     if (offsets_are_i64) {
       CSAW_HIP(hipMemcpy(g->off, offsets, sizeof(int64_t) * (V + 1), hipMemcpyHostToDevice));
     } else {
       int32_t* tmp;
-      CSAW_HIP(hipMalloc(&tmp, sizeof(int32_t) * (V + 1)));
+      CSAW_HIP(device_malloc(&tmp, sizeof(int32_t) * (V + 1)));
       CSAW_HIP(hipMemcpy(tmp, offsets, sizeof(int32_t) * (V + 1), hipMemcpyHostToDevice));
       k_widen_offsets<<<grid_for(V + 1, 256, g->num_cu), 256, 0, g->stream>>>(tmp, V + 1, g->off);
       CSAW_LAUNCH_CHECK();
@@ -749,7 +748,7 @@ extern "C" int csaw_graph_create(const void* offsets, int offsets_are_i64, const
     }
     if (E > 0) CSAW_HIP(hipMemcpy(g->adj, indices, sizeof(int32_t) * E, hipMemcpyHostToDevice));
     if (weights) {
-      CSAW_HIP(hipMalloc(&g->w, sizeof(float) * (E > 0 ? E : 1)));
+      CSAW_HIP(device_malloc(&g->w, sizeof(float) * (E > 0 ? E : 1)));
       if (E > 0) CSAW_HIP(hipMemcpy(g->w, weights, sizeof(float) * E, hipMemcpyHostToDevice));
     }
     return finish_graph(g);
@@ -774,8 +773,8 @@ int rmat_generate_device(int scale, int edge_factor, double a, double b, double 
   const int64_t M = (int64_t)edge_factor << scale;
   const size_t n = (size_t)(2 * M);
   uint64_t *k0, *k1;
-  CSAW_HIP(hipMalloc(&k0, sizeof(uint64_t) * n));
-  CSAW_HIP(hipMalloc(&k1, sizeof(uint64_t) * n));
+  CSAW_HIP(device_malloc(&k0, sizeof(uint64_t) * n));
+  CSAW_HIP(device_malloc(&k1, sizeof(uint64_t) * n));
   k_rmat_pairs<<<grid_for(M, 256, num_cu), 256, 0, stream>>>(scale, M, thr32(a), thr32(a + b), thr32(a + b + c),
                                                              (uint32_t)key, (uint32_t)(key >> 32), k0);
   CSAW_LAUNCH_CHECK();
@@ -783,17 +782,17 @@ int rmat_generate_device(int scale, int edge_factor, double a, double b, double 
   size_t tmp_bytes = 0;
   CSAW_HIP(rocprim::radix_sort_keys(nullptr, tmp_bytes, db, n, 0, 2 * scale, stream));
   void* tmp;
-  CSAW_HIP(hipMalloc(&tmp, tmp_bytes));
+  CSAW_HIP(device_malloc(&tmp, tmp_bytes));
   CSAW_HIP(rocprim::radix_sort_keys(tmp, tmp_bytes, db, n, 0, 2 * scale, stream));
   CSAW_HIP(hipStreamSynchronize(stream));
   CSAW_HIP(hipFree(tmp));
   uint64_t* sorted = db.current();
   uint64_t* uniq = db.alternate();
   uint32_t* d_cnt;
-  CSAW_HIP(hipMalloc(&d_cnt, sizeof(uint32_t)));
+  CSAW_HIP(device_malloc(&d_cnt, sizeof(uint32_t)));
   tmp_bytes = 0;
   CSAW_HIP(rocprim::unique(nullptr, tmp_bytes, sorted, uniq, d_cnt, n, rocprim::equal_to<uint64_t>(), stream));
-  CSAW_HIP(hipMalloc(&tmp, tmp_bytes));
+  CSAW_HIP(device_malloc(&tmp, tmp_bytes));
   CSAW_HIP(rocprim::unique(tmp, tmp_bytes, sorted, uniq, d_cnt, n, rocprim::equal_to<uint64_t>(), stream));
   uint32_t cnt = 0;
   CSAW_HIP(hipMemcpyAsync(&cnt, d_cnt, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
@@ -806,8 +805,8 @@ int rmat_generate_device(int scale, int edge_factor, double a, double b, double 
     CSAW_HIP(hipMemcpy(&last, uniq + E - 1, sizeof(uint64_t), hipMemcpyDeviceToHost));
     if (last == ((1ull << (2 * scale)) - 1)) --E;  // self-loop sentinel
   }
-  CSAW_HIP(hipMalloc(d_off, sizeof(int64_t) * (V + 1)));
-  CSAW_HIP(hipMalloc(d_adj, sizeof(int32_t) * (E > 0 ? E : 1)));
+  CSAW_HIP(device_malloc(d_off, sizeof(int64_t) * (V + 1)));
+  CSAW_HIP(device_malloc(d_adj, sizeof(int32_t) * (E > 0 ? E : 1)));
   k_keys_to_csr<<<grid_for(E + 1, 256, num_cu), 256, 0, stream>>>(uniq, E, scale, V, *d_adj, *d_off);
   CSAW_LAUNCH_CHECK();
   CSAW_HIP(hipStreamSynchronize(stream));
@@ -834,7 +833,7 @@ extern "C" int csaw_graph_create_rmat(int scale, int edge_factor, double a, doub
                                   &g->adj));
     const int64_t E = g->E;
     if (with_weights) {
-      CSAW_HIP(hipMalloc(&g->w, sizeof(float) * (E > 0 ? E : 1)));
+      CSAW_HIP(device_malloc(&g->w, sizeof(float) * (E > 0 ? E : 1)));
       if (E > 0) {
         k_weights<<<grid_for(E, 256, g->num_cu), 256, 0, g->stream>>>((uint32_t)key, (uint32_t)(key >> 32), E, g->w);
         CSAW_LAUNCH_CHECK();
@@ -931,7 +930,7 @@ extern "C" int csaw_seeds(const csaw_graph* g, uint64_t key, uint32_t request, i
   if (!g || n < 0 || (n > 0 && !out) || g->V < 1) return CSAW_ERR_INVALID_ARG;
   if (n == 0) return CSAW_OK;
   int32_t* d;
-  CSAW_HIP(hipMalloc(&d, sizeof(int32_t) * n));
+  CSAW_HIP(device_malloc(&d, sizeof(int32_t) * n));
   k_seeds<<<grid_for(n, 256, g->num_cu), 256, 0, g->stream>>>((uint32_t)key, (uint32_t)(key >> 32), request, g->V, n, d);
   CSAW_LAUNCH_CHECK();
   CSAW_HIP(hipMemcpyAsync(out, d, sizeof(int32_t) * n, hipMemcpyDeviceToHost, g->stream));

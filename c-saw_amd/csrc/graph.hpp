@@ -22,8 +22,8 @@ struct PlanStreams {
 // Workspaces and streams of destroyed plans, kept for the next plan on the same
 // graph (a call of the sampler makes a plan and destroys it).  At most kHeldBytes
 // in blocks of at most kBlockBytes and kHeldStreams stream sets; what the graph
-// still holds when it is destroyed goes back to the device, and an allocation
-// that fails gives everything back and tries again.  What is handed out is of the
+// still holds when it is destroyed goes back to the device, and so do the blocks
+// of every graph when an allocation of the library fails (device_malloc).  What is handed out is of the
 // device that is current then, as a fresh allocation would be.  The owner of a
 // block waits for its work before give(); take() and give() may be called from
 // any thread, whatever device is current there.
@@ -39,7 +39,11 @@ struct Workspace {
   int take_streams(bool with_side, PlanStreams* s);
   void give_streams(PlanStreams s);
   void close();  // the graph is gone: blocks given from now on are freed
-  ~Workspace() { close(); }
+  void drain(std::vector<Block>* out);  // takes every held block
+  Workspace();
+  ~Workspace();
+  Workspace(const Workspace&) = delete;
+  Workspace& operator=(const Workspace&) = delete;
 
  private:
   std::mutex mu;
@@ -47,8 +51,15 @@ struct Workspace {
   std::vector<PlanStreams> streams;
   size_t held = 0;
   bool closed = false;
-  void trim();
 };
+
+// hipMalloc that, where there is no room, gives back what the pools hold and
+// tries again: every device allocation of the library.
+hipError_t device_malloc(void** p, size_t bytes);
+template <typename T>
+hipError_t device_malloc(T** p, size_t bytes) {
+  return device_malloc(reinterpret_cast<void**>(p), bytes);
+}
 }  // namespace csaw
 
 struct csaw_graph {

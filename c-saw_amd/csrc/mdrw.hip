@@ -295,10 +295,10 @@ extern "C" int csaw_mdrw(csaw_graph* g, uint64_t seed, uint32_t request_id, int3
     (void)hipFree(d_cnt);
   };
   auto body = [&]() -> int {
-    CSAW_HIP(hipMalloc(&d_seeds, sizeof(int32_t) * std::max<int64_t>(ns, 1)));
-    CSAW_HIP(hipMalloc(&d_src, sizeof(int32_t) * slots));
-    CSAW_HIP(hipMalloc(&d_dst, sizeof(int32_t) * slots));
-    CSAW_HIP(hipMalloc(&d_cnt, sizeof(int32_t) * std::max<int32_t>(samples, 1)));
+    CSAW_HIP(device_malloc(&d_seeds, sizeof(int32_t) * std::max<int64_t>(ns, 1)));
+    CSAW_HIP(device_malloc(&d_src, sizeof(int32_t) * slots));
+    CSAW_HIP(device_malloc(&d_dst, sizeof(int32_t) * slots));
+    CSAW_HIP(device_malloc(&d_cnt, sizeof(int32_t) * std::max<int32_t>(samples, 1)));
     if (ns > 0) CSAW_HIP(hipMemcpy(d_seeds, seeds, sizeof(int32_t) * ns, hipMemcpyHostToDevice));
     hipEvent_t e0, e1;
     CSAW_HIP(hipEventCreate(&e0));

@@ -301,7 +301,7 @@ static int mlp_alloc_work(MlpWork& w, int64_t n_data, int64_t n_batch) {
     } else {
       part(&w.Y, n_data * kMlpOut);
     }
-    if (!w.slab) CSAW_HIP(hipMalloc(&w.slab, at));
+    if (!w.slab) CSAW_HIP(device_malloc(&w.slab, at));
   }
   return CSAW_OK;
 }
@@ -349,8 +349,8 @@ extern "C" int csaw_mlp_create(uint64_t init_key, csaw_mlp** out) {
   auto body = [&]() -> int {
     CSAW_TRY(device_init(&m->num_cu));
     CSAW_HIP(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
-    CSAW_HIP(hipMalloc(&m->d_master, sizeof(float) * kMlpParams));
-    CSAW_HIP(hipMalloc(&m->d_w, sizeof(uint16_t) * kMlpParams));
+    CSAW_HIP(device_malloc(&m->d_master, sizeof(float) * kMlpParams));
+    CSAW_HIP(device_malloc(&m->d_w, sizeof(uint16_t) * kMlpParams));
     return csaw_mlp_set_params(m, m->master.data());
   };
   int st = body();

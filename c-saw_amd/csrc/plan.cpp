@@ -132,11 +132,7 @@ int Workspace::take(size_t bytes, Block* b) {
   }
   b->bytes = (bytes + 65535) & ~(size_t)65535;
   b->device = device;
-  if (hipMalloc(&b->p, b->bytes) != hipSuccess) {
-    (void)hipGetLastError();
-    trim();
-    CSAW_HIP(hipMalloc(&b->p, b->bytes));
-  }
+  CSAW_HIP(device_malloc(&b->p, b->bytes));
   return CSAW_OK;
 }
 
@@ -180,25 +176,69 @@ void Workspace::give_streams(PlanStreams s) {
   s.destroy();
 }
 
-void Workspace::trim() {
-  std::vector<Block> out;
-  {
-    std::lock_guard<std::mutex> lock(mu);
-    out.swap(blocks);
-    held = 0;
-  }
-  for (Block& b : out) (void)hipFree(b.p);
+void Workspace::drain(std::vector<Block>* out) {
+  std::lock_guard<std::mutex> lock(mu);
+  out->insert(out->end(), blocks.begin(), blocks.end());
+  blocks.clear();
+  held = 0;
 }
 
 void Workspace::close() {
-  trim();
-  std::vector<PlanStreams> out;
+  std::vector<Block> out;
+  std::vector<PlanStreams> sets;
+  drain(&out);
   {
     std::lock_guard<std::mutex> lock(mu);
     closed = true;
-    out.swap(streams);
+    sets.swap(streams);
   }
-  for (PlanStreams& s : out) s.destroy();
+  for (Block& b : out) (void)hipFree(b.p);
+  for (PlanStreams& s : sets) s.destroy();
+}
+
+// The pools that exist, for device_malloc.  (Never destroyed: a graph may go
+// after this file's statics.)
+namespace {
+struct Pools {
+  std::mutex mu;
+  std::vector<Workspace*> all;
+};
+Pools& pools() {
+  static Pools* p = new Pools;
+  return *p;
+}
+}  // namespace
+
+Workspace::Workspace() {
+  Pools& P = pools();
+  std::lock_guard<std::mutex> lock(P.mu);
+  P.all.push_back(this);
+}
+
+Workspace::~Workspace() {
+  {
+    Pools& P = pools();
+    std::lock_guard<std::mutex> lock(P.mu);
+    P.all.erase(std::find(P.all.begin(), P.all.end(), this));
+  }
+  close();
+}
+
+hipError_t device_malloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipSuccess) return e;
+  (void)hipGetLastError();
+  std::vector<Workspace::Block> out;
+  {
+    Pools& P = pools();
+    std::lock_guard<std::mutex> lock(P.mu);
+    for (Workspace* w : P.all) w->drain(&out);
+  }
+  if (out.empty()) return e;
+  for (Workspace::Block& b : out) (void)hipFree(b.p);
+  e = hipMalloc(p, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
 }
 
 }  // namespace csaw
@@ -869,7 +909,7 @@ extern "C" int csaw_plan_digest(const csaw_plan* p, int32_t req, uint64_t* diges
   const Unit& u = p->units[ui];
   unsigned long long* d;
   InFlight sum(p->unwaited);
-  CSAW_HIP(hipMalloc(&d, sizeof(unsigned long long)));
+  CSAW_HIP(device_malloc(&d, sizeof(unsigned long long)));
   CSAW_HIP(hipMemsetAsync(d, 0, sizeof(unsigned long long), p->stream));
   int64_t at = 0;
   int st = CSAW_OK;

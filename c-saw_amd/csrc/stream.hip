@@ -260,7 +260,7 @@ struct Budget {
       set_last_error("device budget exceeded: need " + std::to_string(used + bytes) + " of " + std::to_string(limit));
       return CSAW_ERR_BUDGET_TOO_SMALL;
     }
-    CSAW_HIP(hipMalloc((void**)p, bytes));
+    CSAW_HIP(device_malloc((void**)p, bytes));
     ptrs.push_back((void*)*p);
     used += bytes;
     peak = std::max(peak, used);

@@ -211,9 +211,9 @@ extern "C" int csaw_walk_plan_create(csaw_graph* g, int32_t bias, uint64_t seed,
   p->n = n_walkers;
   p->len = len;
   auto body = [&]() -> int {
-    CSAW_HIP(hipMalloc(&p->d_seeds, sizeof(int32_t) * std::max<int64_t>(n_walkers, 1)));
-    CSAW_HIP(hipMalloc(&p->d_W, sizeof(int32_t) * std::max<int64_t>(n_walkers * (len + 1), 1)));
-    CSAW_HIP(hipMalloc(&p->d_steps, 2 * sizeof(unsigned long long)));
+    CSAW_HIP(device_malloc(&p->d_seeds, sizeof(int32_t) * std::max<int64_t>(n_walkers, 1)));
+    CSAW_HIP(device_malloc(&p->d_W, sizeof(int32_t) * std::max<int64_t>(n_walkers * (len + 1), 1)));
+    CSAW_HIP(device_malloc(&p->d_steps, 2 * sizeof(unsigned long long)));
     if (n_walkers > 0)
       CSAW_HIP(hipMemcpy(p->d_seeds, seeds, sizeof(int32_t) * n_walkers, hipMemcpyHostToDevice));
     CSAW_HIP(hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking));

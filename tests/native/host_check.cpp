@@ -194,6 +194,76 @@ static void partial_streams() {
     }
 }
 
+// No allocation of the library fails while a pool holds memory that would do.
+static void pool_makes_room() {
+  csaw_graph* g = regular_graph(2000, 8);
+  csaw_graph* hubs = regular_graph(100, 2000);
+  csaw_host_graph* hg = nullptr;
+  {
+    std::vector<int64_t> off(1001);
+    for (int64_t v = 0; v <= 1000; ++v) off[v] = 8 * v;
+    const std::vector<int32_t> ids(8000, 0);
+    NEED(csaw_host_graph_from_csr(off.data(), ids.data(), 1000, 8000, &hg) == CSAW_OK);
+  }
+  const std::vector<int32_t> seeds(4000, 1);
+  // a block of about 11 MB in the pool of g, and no other memory left than that
+  auto fill = [&] {
+    const csaw_request r = request(4000, {25, 8}, CSAW_BIAS_UNIFORM, seeds.data());
+    csaw_plan* p = nullptr;
+    fake().limit = SIZE_MAX;
+    NEED(csaw_plan_create(g, &r, 1, nullptr, &p) == CSAW_OK);
+    NEED(csaw_plan_run(p, nullptr, 1) == CSAW_OK);
+    csaw_plan_destroy(p);
+    fake().limit = fake().used;
+  };
+  std::vector<int32_t> out(4000 * 8), walks(4000 * 9);
+  std::vector<int64_t> offs(4001);
+  fill();
+  csaw_mlp* m = nullptr;
+  NEED(csaw_mlp_create(1, &m) == CSAW_OK);
+  fill();
+  std::vector<float> X(16, 0.f), Y(16);
+  NEED(csaw_mlp_forward(m, X.data(), 1, Y.data()) == CSAW_OK);
+  fill();
+  NEED(csaw_random_walk(g, CSAW_BIAS_DEGREE, 1, 0, seeds.data(), 4000, 8, walks.data(), nullptr) == CSAW_OK);
+  fill();
+  NEED(csaw_mdrw(g, 1, 0, 2000, 2, 8, seeds.data(), out.data(), out.data(), offs.data(), nullptr) == CSAW_OK);
+  fill();
+  NEED(csaw_seeds(g, 1, 0, 100, out.data()) == CSAW_OK);
+  fill();
+  csaw_graph* other = regular_graph(10, 2);
+  csaw_graph_destroy(other);
+  for (int cache = 0; cache < 2; ++cache) {
+    fill();
+    const csaw_request r = request(10, {5}, CSAW_BIAS_DEGREE, seeds.data());
+    csaw_plan_opts o;
+    memset(&o, 0, sizeof(o));
+    o.cdf_cache = cache;
+    csaw_plan* p = nullptr;
+    NEED(csaw_plan_create(hubs, &r, 1, &o, &p) == CSAW_OK);
+    uint64_t digest = 0;
+    NEED(csaw_plan_run(p, nullptr, 1) == CSAW_OK);
+    fill();
+    NEED(csaw_plan_digest(p, 0, &digest) == CSAW_OK);
+    csaw_plan_destroy(p);
+  }
+  fill();
+  const csaw_request r = request(10, {5}, CSAW_BIAS_UNIFORM, seeds.data());
+  csaw_edges* e = nullptr;
+  csaw_stream_stats st;
+  NEED(csaw_stream_sample(hg, &r, 8 << 20, 2, &e, &st) == CSAW_OK);
+  csaw_edges_free(e);
+  // and one that is too large for the device all the same says so
+  fill();
+  const csaw_request big = request(4000, {64, 64}, CSAW_BIAS_UNIFORM, seeds.data());
+  csaw_plan* p = nullptr;
+  NEED(csaw_plan_create(g, &big, 1, nullptr, &p) == CSAW_ERR_OOM);
+  csaw_mlp_destroy(m);
+  csaw_host_graph_destroy(hg);
+  csaw_graph_destroy(hubs);
+  csaw_graph_destroy(g);
+}
+
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> checks = {
       {"hub_positions", hub_positions},
@@ -201,6 +271,7 @@ int main(int argc, char** argv) {
       {"failed_wait", failed_wait},
       {"failed_copy_out", failed_copy_out},
       {"partial_streams", partial_streams},
+      {"pool_makes_room", pool_makes_room},
   };
   const auto it = checks.find(argc > 1 ? argv[1] : "");
   if (it == checks.end()) return 2;

@@ -46,3 +46,7 @@ def test_calls_that_fail_before_they_have_waited(host_check):
 
 def test_partly_made_streams_are_completed(host_check):
     run(host_check, "partial_streams")
+
+
+def test_pooled_memory_makes_room_for_any_allocation(host_check):
+    run(host_check, "pool_makes_room")
