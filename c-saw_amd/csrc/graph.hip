@@ -311,8 +311,6 @@ static int ensure_hub_list(csaw_graph* g) {
   return CSAW_OK;
 }
 
-static int narrow_hubs(csaw_graph* g);
-
 int graph_prepare_bias(csaw_graph* g, int32_t bias) {
   if (bias == CSAW_BIAS_WEIGHT) {
     if (!g->w) {
@@ -342,15 +340,11 @@ int graph_prepare_bias(csaw_graph* g, int32_t bias) {
   if (bias != CSAW_BIAS_DEGREE && bias != CSAW_BIAS_USER) return CSAW_OK;
   const int kind = bias == CSAW_BIAS_DEGREE ? 0 : 1;
   CSAW_TRY(ensure_hub_list(g));
-  // degree totals up to kHubMin neighbours fit 32 bits (hubs are looked at below)
-  const bool fits = kind == 0 && !g->wide_int_cdf && g->max_deg * (int64_t)kHubMin < ((int64_t)1 << 32);
-  if (fits && g->n_hubs == 0) g->build32 = true;
   if (g->hub_cdf[kind] || g->n_hubs == 0) return CSAW_OK;
   std::vector<int64_t> pool(g->n_hubs + 1);
   CSAW_HIP(hipMemcpy(pool.data(), g->hub_pool, sizeof(int64_t) * pool.size(), hipMemcpyDeviceToHost));
   CSAW_HIP(device_malloc(&g->hub_cdf[kind], sizeof(uint64_t) * g->hub_entries));
   CSAW_TRY(hub_cdf_build(g->view(), g->hook_view(), kind, pool, g->hub_cdf[kind], g->stream, g->num_cu));
-  if (fits) CSAW_TRY(narrow_hubs(g));
   CSAW_HIP(hipStreamSynchronize(g->stream));
   return CSAW_OK;
 }
@@ -542,42 +536,59 @@ static int build_index(const T* C, int64_t E, T** out, hipStream_t stream, int n
 
 // The DEGREE hub CDFs as uint32, padded and indexed like the CDF cache, when
 // their totals fit (duplicate neighbours can total more than E), so do the hubs'
-// places among them (the batch build keeps a place beside its total in 64 bits),
-// and there is room for them; without them every entry keeps to the uint64 hubs.
-static int narrow_hubs(csaw_graph* g) {
+// places among them (the batch build keeps a place beside its total in 64 bits)
+// and the totals of the other vertices, and there is room for the copy; without
+// it every entry keeps to the uint64 hubs.  Where only the room was missing the
+// next plan asks again, but takes no more from the pools for it.
+int graph_prepare_build32(csaw_graph* g) {
+  if (g->build32 || g->wide_totals) return CSAW_OK;
+  CSAW_TRY(graph_prepare_bias(g, CSAW_BIAS_DEGREE));
   const int64_t n = g->hub_entries, npad = pad16(n);
-  if (n > (int64_t)UINT32_MAX) return CSAW_OK;
-  auto room = [](auto** p, int64_t count) -> bool {
-    if (device_malloc(p, sizeof(**p) * count) == hipSuccess) return true;
+  if (g->wide_int_cdf || g->max_deg * (int64_t)kHubMin >= ((int64_t)1 << 32) || n > (int64_t)UINT32_MAX) {
+    g->wide_totals = true;
+    return CSAW_OK;
+  }
+  if (g->n_hubs == 0) {
+    g->build32 = true;
+    return CSAW_OK;
+  }
+  uint32_t *cdf = nullptr, *idx = nullptr;
+  unsigned long long *d_max = nullptr, mx = 0;
+  auto room = [&](auto** p, int64_t count) -> bool {
+    const size_t bytes = sizeof(**p) * count;
+    if ((g->narrow_asked ? hipMalloc((void**)p, bytes) : device_malloc(p, bytes)) == hipSuccess) return true;
+    (void)hipGetLastError();
     *p = nullptr;
     return false;
   };
-  unsigned long long* d_max = nullptr;
-  if (!room(&d_max, 1)) return CSAW_OK;
-  unsigned long long mx = 0;
   auto body = [&]() -> int {
+    const bool got = room(&cdf, npad) && room(&idx, std::max<int64_t>(cdf_index_size(n), 16)) && room(&d_max, 1);
+    g->narrow_asked = true;
+    if (!got) return CSAW_OK;
     CSAW_HIP(hipMemsetAsync(d_max, 0, sizeof(unsigned long long), g->stream));
     k_max_u64<<<grid_for(n, 256, g->num_cu), 256, 0, g->stream>>>(g->hub_cdf[0], n, d_max);
     CSAW_LAUNCH_CHECK();
     CSAW_HIP(hipMemcpyAsync(&mx, d_max, sizeof(mx), hipMemcpyDeviceToHost, g->stream));
     CSAW_HIP(hipStreamSynchronize(g->stream));
-    if (mx >= (1ull << 32)) return CSAW_OK;
-    if (!room(&g->hub_cdf32, npad)) return CSAW_OK;
-    CSAW_HIP(hipMemsetAsync(g->hub_cdf32, 0, sizeof(uint32_t) * npad, g->stream));
-    k_narrow_u32<<<grid_for(n, 256, g->num_cu), 256, 0, g->stream>>>(g->hub_cdf[0], n, g->hub_cdf32);
-    CSAW_LAUNCH_CHECK();
-    if (!room(&g->hub_idx32, std::max<int64_t>(cdf_index_size(n), 16))) {
-      CSAW_HIP(hipStreamSynchronize(g->stream));
-      (void)hipFree(g->hub_cdf32);
-      g->hub_cdf32 = nullptr;
+    if (mx >= (1ull << 32)) {
+      g->wide_totals = true;
       return CSAW_OK;
     }
-    CSAW_TRY(build_index<uint32_t>(g->hub_cdf32, n, g->hub_idx32, g->stream, g->num_cu));
+    CSAW_HIP(hipMemsetAsync(cdf, 0, sizeof(uint32_t) * npad, g->stream));
+    k_narrow_u32<<<grid_for(n, 256, g->num_cu), 256, 0, g->stream>>>(g->hub_cdf[0], n, cdf);
+    CSAW_LAUNCH_CHECK();
+    CSAW_TRY(build_index<uint32_t>(cdf, n, idx, g->stream, g->num_cu));
+    g->hub_cdf32 = cdf;
+    g->hub_idx32 = idx;
     g->build32 = true;
     return CSAW_OK;
   };
   const int st = body();
   (void)hipFree(d_max);
+  if (!g->build32) {
+    (void)hipFree(cdf);
+    (void)hipFree(idx);
+  }
   return st;
 }
 

@@ -1,6 +1,7 @@
 // Device-resident CSR graph (replaces gpu_graph, non-stream/gpu_graph.cuh:10-65,
 // and the host loader graph<>, non-stream/graph.hpp:4-111).
 #pragma once
+#include <atomic>
 #include <memory>
 #include <mutex>
 #include <vector>
@@ -76,7 +77,9 @@ struct csaw_graph {
   uint64_t* hub_cdf[2] = {nullptr, nullptr};  // [DEGREE, USER]
   uint32_t* hub_cdf32 = nullptr;              // DEGREE, when every total fits
   uint32_t* hub_idx32 = nullptr;
-  bool build32 = false;                       // see GraphDev
+  std::atomic<bool> build32{false};           // see GraphDev
+  bool wide_totals = false;                   // build32 cannot become true
+  bool narrow_asked = false;
   uint64_t* int_cdf[2] = {nullptr, nullptr};  // full per-entry CDF cache [DEGREE, USER]
   // 16-ary search indexes over cdf and int_cdf (CDF arrays padded to 16)
   float* cdf_idx = nullptr;
@@ -95,6 +98,8 @@ struct csaw_graph {
   // (environment CSAW_INT_CDF_KEYS=64 at graph creation; covers the 64-bit
   // search paths on graphs whose totals are small)
   bool wide_int_cdf = false;
+  // held while a plan's or walk's preparations run (what they build is the graph's)
+  std::mutex prepare;
   // shared with the plans, which may outlive the graph
   std::shared_ptr<csaw::Workspace> work = std::make_shared<csaw::Workspace>();
 
@@ -110,6 +115,8 @@ int graph_prepare_vertex_records(csaw_graph* g, int32_t bias);
 // integer hub cache (CSAW_BIAS_DEGREE / CSAW_BIAS_USER).
 int graph_prepare_bias(csaw_graph* g, int32_t bias);
 int graph_prepare_int_cache(csaw_graph* g, int32_t bias);
+// 32-bit hub CDFs for degree bias without the CDF cache (GraphDev::build32)
+int graph_prepare_build32(csaw_graph* g);
 // Builds the search index of the CDF a bias uses from the cache (FP32 CDF for
 // CSAW_BIAS_WEIGHT, the integer CDF cache otherwise), building that CDF first.
 int graph_prepare_index(csaw_graph* g, int32_t bias);

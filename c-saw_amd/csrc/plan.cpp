@@ -652,10 +652,13 @@ static int plan_create(csaw_graph* g, const csaw_request* reqs, int32_t n_req, c
   else if (o.tuning && o.tuning->expand_per_cu > 0) p->L.frontier_per_cu = o.tuning->expand_per_cu;
   auto body = [&]() -> int {
     for (int i = 0; i < n_req; ++i) {
+      std::lock_guard<std::mutex> lock(g->prepare);
       CSAW_TRY(graph_prepare_bias(g, reqs[i].bias));
       if (o.cdf_cache) {
         CSAW_TRY(graph_prepare_index(g, reqs[i].bias));
         CSAW_TRY(graph_prepare_vertex_records(g, reqs[i].bias));
+      } else if (reqs[i].bias == CSAW_BIAS_DEGREE) {
+        CSAW_TRY(graph_prepare_build32(g));
       }
       p->reqs.push_back(reqs[i]);
       p->reqs.back().seeds = nullptr;

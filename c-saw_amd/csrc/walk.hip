@@ -201,8 +201,11 @@ extern "C" int csaw_walk_plan_create(csaw_graph* g, int32_t bias, uint64_t seed,
   for (int64_t i = 0; i < n_walkers; ++i)
     if (seeds[i] < 0 || seeds[i] >= g->V) return CSAW_ERR_INVALID_ARG;
   // walks search the CDF cache (FP32 CDF or integer cache) through its index
-  CSAW_TRY(graph_prepare_index(g, bias));
-  CSAW_TRY(graph_prepare_vertex_records(g, bias));
+  {
+    std::lock_guard<std::mutex> lock(g->prepare);
+    CSAW_TRY(graph_prepare_index(g, bias));
+    CSAW_TRY(graph_prepare_vertex_records(g, bias));
+  }
   csaw_walk_plan* p = new csaw_walk_plan();
   p->g = g;
   p->bias = bias;

@@ -264,6 +264,43 @@ static void pool_makes_room() {
   csaw_graph_destroy(g);
 }
 
+// The 32-bit copy of the hub CDFs is made for plans that read it (degree bias
+// without the CDF cache), and by a later plan where the first one found no room.
+static void narrow_hubs_when_read() {
+  const int32_t n = 4000;  // 13 MB a plan
+  const std::vector<int32_t> seeds(n, 0);
+  const csaw_request r = request(n, {25, 10}, CSAW_BIAS_DEGREE, seeds.data());
+  const int64_t entries = 5000 * 2000;  // 40 MB narrow
+  csaw_graph* g = regular_graph(5000, 2000);
+  auto asked = [&] {  // allocations of the copy's size
+    int k = 0;
+    for (size_t a : fake().allocs) k += a == sizeof(uint32_t) * entries;
+    return k;
+  };
+  auto batch_built = [&](int cache) {
+    csaw_plan_opts o;
+    memset(&o, 0, sizeof(o));
+    o.cdf_cache = cache;
+    csaw_plan* p = nullptr;
+    fake().allocs.clear();
+    NEED(csaw_plan_create(g, &r, 1, &o, &p) == CSAW_OK);
+    fake().log.clear();
+    NEED(csaw_plan_run(p, nullptr, 1) == CSAW_OK);
+    csaw_plan_destroy(p);
+    return fake().logged("k_expand_plainILi1ELb0ELi1ELb0ELb1E");
+  };
+  NEED(!batch_built(1) && asked() == 1);  // the CDF cache itself
+  NEED(!batch_built(1) && asked() == 0);
+  fake().limit = fake().used + (20 << 20);  // the plan fits, the copy does not
+  NEED(!batch_built(0));
+  NEED(!batch_built(0));
+  fake().limit = SIZE_MAX;
+  NEED(batch_built(0) && asked() == 1);
+  NEED(batch_built(0) && asked() == 0);
+  csaw_graph_destroy(g);
+  NEED(fake().used == 0);
+}
+
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> checks = {
       {"hub_positions", hub_positions},
@@ -272,6 +309,7 @@ int main(int argc, char** argv) {
       {"failed_copy_out", failed_copy_out},
       {"partial_streams", partial_streams},
       {"pool_makes_room", pool_makes_room},
+      {"narrow_hubs_when_read", narrow_hubs_when_read},
   };
   const auto it = checks.find(argc > 1 ? argv[1] : "");
   if (it == checks.end()) return 2;

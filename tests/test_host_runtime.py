@@ -50,3 +50,7 @@ def test_partly_made_streams_are_completed(host_check):
 
 def test_pooled_memory_makes_room_for_any_allocation(host_check):
     run(host_check, "pool_makes_room")
+
+
+def test_narrow_hubs_for_the_plans_that_read_them(host_check):
+    run(host_check, "narrow_hubs_when_read")
