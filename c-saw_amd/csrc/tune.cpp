@@ -61,7 +61,8 @@ extern "C" int csaw_plan_chunk_log(const csaw_plan* p, float* features, int32_t*
 
 // Tries workgroups-per-CU settings for each kernel family, then the tile
 // shapes (smallest chunk, smallest sub-wave group), one knob at a time
-// (coordinate descent), timing full runs of the plan with hipEvents.
+// (coordinate descent), timing full runs of the plan with hipEvents.  A knob that
+// no hop of the plan reads keeps its default: its runs would differ by noise only.
 extern "C" int csaw_autotune(csaw_graph* g, const csaw_request* reqs, int32_t n_req, const csaw_plan_opts* base,
                              csaw_tuning* best, double* best_ms) {
   if (!g || !best) return CSAW_ERR_INVALID_ARG;
@@ -79,10 +80,13 @@ extern "C" int csaw_autotune(csaw_graph* g, const csaw_request* reqs, int32_t n_
   cur.block_per_cu = def.block_per_cu;
   cur.chunk_min = def.chunk_min;
   cur.group_min = def.group_min;
+  bool binned = false, whole = false;  // some hop bins its entries, is expanded whole
   auto measure = [&](const csaw_tuning& t, double* ms) -> int {
     o.tuning = &t;
     csaw_plan* p = nullptr;
     CSAW_TRY(csaw_plan_create(g, reqs, n_req, &o, &p));
+    for (const Unit& u : p->units)
+      for (char b : u.bin) (b ? binned : whole) = true;
     int st = csaw_plan_run(p, nullptr, 1);  // warm-up (and graph capture)
     double acc = 0;
     const int reps = 3;
@@ -99,14 +103,26 @@ extern "C" int csaw_autotune(csaw_graph* g, const csaw_request* reqs, int32_t n_
   const std::vector<int> per_cu = {1, 2, 4, 8, 16};
   const std::vector<int> chunk = {8, 16, 32, 64, 128, 256};
   const std::vector<int> group = {4, 8, 16};
-  const std::pair<int32_t*, const std::vector<int>*> knobs[] = {
-      {&cur.expand_per_cu, &per_cu}, {&cur.thread_per_cu, &per_cu}, {&cur.block_per_cu, &per_cu},
-      {&cur.count_per_cu, &per_cu},  {&cur.chunk_min, &chunk},       {&cur.group_min, &group}};
+  // whole-hop kernels of a batched plan: 32 workgroups per CU unless this is set
+  const std::vector<int> grid = {8 * g->num_cu, 16 * g->num_cu, 64 * g->num_cu};
+  const bool batched = o.mode == CSAW_MODE_BATCHED;
+  const struct {
+    int32_t* value;
+    const std::vector<int>* tries;
+    bool read;
+  } knobs[] = {{&cur.expand_per_cu, &per_cu, binned || !batched},
+               {&cur.thread_per_cu, &per_cu, binned},
+               {&cur.block_per_cu, &per_cu, binned},
+               {&cur.grid_override, &grid, batched && whole},
+               {&cur.count_per_cu, &per_cu, true},
+               {&cur.chunk_min, &chunk, binned},
+               {&cur.group_min, &group, true}};
   for (const auto& kn : knobs) {
-    int32_t* f = kn.first;
+    if (!kn.read) continue;
+    int32_t* f = kn.value;
     const int32_t keep = *f;
     int32_t bv = keep;
-    for (int c : *kn.second) {
+    for (int c : *kn.tries) {
       if (c == keep) continue;
       *f = c;
       double ms = 0;

@@ -166,13 +166,18 @@ int csaw_random_walk(csaw_graph *g, int32_t bias, uint64_t seed, uint32_t reques
 
 /* Launch shapes (workgroups per CU per kernel family), chosen by
  * csaw_autotune.  Replaces the fixed <<<n_blocks, n_threads>>> of the
- * reference's run.sh:2 (400 x 128). */
+ * reference's run.sh:2 (400 x 128).  A batched plan expands a hop whole, a kernel
+ * per bias kind in frontier order, or bins it into chunks (csaw_plan_opts);
+ * expand_per_cu is read by plain plans and binned hops, thread_per_cu,
+ * block_per_cu and chunk_min by binned hops, the others by every plan. */
 typedef struct csaw_tuning {
   int32_t count_per_cu;
   int32_t expand_per_cu;
   int32_t thread_per_cu;
   int32_t block_per_cu;
-  int32_t grid_override; /* fixed grid for the plain expand kernel (0: auto) */
+  int32_t grid_override; /* fixed grid of the whole-hop expand kernels (0: at */
+                         /*  most expand_per_cu workgroups per CU in a plain  */
+                         /*  plan, 32 in a batched one)                       */
   /* Tile shapes (0: default).  chunk_min: smallest chunk of frontier
    * entries a queue hands out (a power of two, 8 .. 1024; chunks grow to
    * whole 1024-entry buckets when the hop is large).  group_min: smallest
@@ -294,8 +299,9 @@ int csaw_plan_destroy(csaw_plan *p);
 int csaw_plan_chunk_log(const csaw_plan *p, float *features, int32_t *variant, float *log2_ticks,
                         uint64_t *keys, int64_t max_n, int64_t *n);
 /* Tries launch and tile shapes (coordinate descent over workgroups per CU
- * of each kernel family, chunk_min and group_min) on the given requests and
- * returns the fastest; best_ms is its mean device time per run. */
+ * of each kernel family, grid_override, chunk_min and group_min) on the given
+ * requests and returns the fastest; best_ms is its mean device time per run.
+ * What no hop of these requests reads is returned at its default. */
 int csaw_autotune(csaw_graph *g, const csaw_request *reqs, int32_t n_req, const csaw_plan_opts *base,
                   csaw_tuning *best, double *best_ms);
 

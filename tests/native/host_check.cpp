@@ -301,6 +301,39 @@ static void narrow_hubs_when_read() {
   NEED(fake().used == 0);
 }
 
+// The autotuner tries what the plan's hops read and leaves the rest at its
+// default.  Every run takes less time than the one before it here, so that the
+// last of the values tried is kept.
+static void autotune_reads() {
+  csaw_graph* g = regular_graph(100, 8);
+  const std::vector<int32_t> seeds(50, 1);
+  const csaw_request r = request(50, {4, 4}, CSAW_BIAS_UNIFORM, seeds.data());
+  auto tune = [&](int mode, int sched) {
+    csaw_plan_opts o;
+    memset(&o, 0, sizeof(o));
+    o.mode = mode;
+    o.sched = sched;
+    o.variant = CSAW_VAR_THREAD;
+    csaw_tuning t;
+    double ms = 0;
+    fake().ms = 1000.0f;
+    fake().ms_step = 1.0f;
+    NEED(csaw_autotune(g, &r, 1, &o, &t, &ms) == CSAW_OK);
+    NEED(t.count_per_cu == 16 && t.group_min == 16);
+    return t;
+  };
+  csaw_tuning t = tune(CSAW_MODE_BATCHED, CSAW_SCHED_HEURISTIC);  // hops expanded whole
+  NEED(t.expand_per_cu == 8 && t.thread_per_cu == 4 && t.block_per_cu == 2 && t.chunk_min == 8);
+  NEED(t.grid_override == 64 * 256);
+  t = tune(CSAW_MODE_PLAIN, CSAW_SCHED_HEURISTIC);
+  NEED(t.expand_per_cu == 16 && t.thread_per_cu == 4 && t.block_per_cu == 2 && t.chunk_min == 8);
+  NEED(t.grid_override == 0);
+  t = tune(CSAW_MODE_BATCHED, CSAW_SCHED_FORCED);  // binned
+  NEED(t.expand_per_cu == 16 && t.thread_per_cu == 16 && t.block_per_cu == 16 && t.chunk_min == 256);
+  NEED(t.grid_override == 0);
+  csaw_graph_destroy(g);
+}
+
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> checks = {
       {"hub_positions", hub_positions},
@@ -310,6 +343,7 @@ int main(int argc, char** argv) {
       {"partial_streams", partial_streams},
       {"pool_makes_room", pool_makes_room},
       {"narrow_hubs_when_read", narrow_hubs_when_read},
+      {"autotune_reads", autotune_reads},
   };
   const auto it = checks.find(argc > 1 ? argv[1] : "");
   if (it == checks.end()) return 2;

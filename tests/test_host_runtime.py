@@ -54,3 +54,7 @@ def test_pooled_memory_makes_room_for_any_allocation(host_check):
 
 def test_narrow_hubs_for_the_plans_that_read_them(host_check):
     run(host_check, "narrow_hubs_when_read")
+
+
+def test_autotune_tries_what_the_hops_read(host_check):
+    run(host_check, "autotune_reads")
