@@ -524,6 +524,7 @@ def main():
         "speedup_parts": {"cdf_cache (plain -> plain+cache)": t_plain / (runs["plain_cdf_cache"]["ms_per_step"] * 1e-3),
                           "batching (plain+cache -> batched+heuristic)":
                               runs["plain_cdf_cache"]["ms_per_step"] / runs["batched_heuristic"]["ms_per_step"],
+                          # (level: no hop of this mix is binned, so both run the same kernels)
                           "learned schedule (batched+heuristic -> batched+learned)":
                               runs["batched_heuristic"]["ms_per_step"] / runs["batched_learned"]["ms_per_step"],
                           "learned schedule vs the best fixed variant (batched, wave bitmap forced)":

@@ -126,8 +126,9 @@ __global__ __launch_bounds__(kWave) void k_mlp_rows(const uint16_t* __restrict__
 // A against all WB columns of B; NA = 0: biases, the sums of B's columns) and
 // stages kParamRows rows of it in LDS with wide coalesced loads, the next rows'
 // loads in flight while the lanes run their chains from LDS.
-// Bound: the latency of the first tile (the rows were written by other XCDs)
-// and the 256-deep chain.  For 256 rows: 88 us with a lane's pairs loaded from
+// Bound: latency, of the first tile (the rows were written by other XCDs) and of
+// each tile's round of store, barrier and sum; the 256 dependent FMAs of a chain
+// are about 1 us of it.  For 256 rows: 88 us with a lane's pairs loaded from
 // memory one by one, 26 us with 32 pairs loaded ahead, 15 us from LDS with the
 // tile widths as run-time values, 12.3 us as constants, 10.9 us staged by sixteen
 // waves (one wave a workgroup, four times the workgroups: 28 us).

@@ -429,7 +429,15 @@ __global__ __launch_bounds__(256, KEYS == kKeys32 && !REMAP ? 4 : 1) void k_expa
   // end those sooner.  (Uniform draws collide too rarely for that: groups
   // throughout.)  On RMAT-22, groups and whole waves: region remap of 8,191 seeds
   // {10, 10} 542 and 469 us, degree bias {25, 10} from 40,000 with the CDF cache
-  // 609 and 534 us, without 854 and 735; beyond the line the groups are level.
+  // 609 and 534 us, without 854 and 735.
+  // One hop of entries drawn by degree, groups / whole waves in us at a half, one
+  // and twice the line: fanout 5, cached degree bias 44/36, 46/46, 50/64, FP32
+  // 29/29, 32/41, 36/58; fanout 10 79/68, 82/89, 105/125 and 44/46, 52/62, 67/91;
+  // 15 95/107, 136/140, 198/202 and 58/58, 77/86, 102/137; 20 192/165, 257/214,
+  // 414/360 and 75/74, 108/114, 178/197; 25 297/243, 504/389, 787/636 and 136/114,
+  // 196/184, 338/321; 32 440/349, 630/517, 967/840 and 176/145, 275/241, 439/390.
+  // So the line is where fanouts up to 15 cross; from 20 on whole waves stay ahead
+  // beyond it under degree bias.
   const int gs = hop_gs > 0 && KIND != kUniform && n * (kWave / hop_gs) <= kWideHopEntries ? kWave : hop_gs;
   // batch size adapts to the frontier: one entry (one group round) per wave
   // when it is small (all waves busy), up to 64 entries per metadata round

@@ -558,8 +558,8 @@ __device__ void wave_expand_batch(const GraphDev& G, const csaw_graph_view& hv, 
 // 64/GS entries in flight per wave instead of one.  Every shuffle reads lanes
 // of the shuffling group only, and all lanes of a group follow the same path.
 // ---------------------------------------------------------------------------
-// One frontier entry as the group path keeps it (16 dwords, so a batch of 64
-// costs 16 registers per lane, and one shuffle per dword to fetch).
+// One frontier entry as the group path keeps it (16 dwords; a batch's selecting
+// entries wait in LDS, store_gentry below).
 struct GEntry {
   int32_t v, d;
   int64_t o;
@@ -567,7 +567,7 @@ struct GEntry {
   int64_t pos;
   uint32_t c1, c2, c3, k0, k1;
   uint32_t flags;  // bit 0 dedup, bit 1 user-bias cache, bit 2 region remap, bits 4-7 PickMode
-  uint64_t T;      // integer CDF total, or the FP32 total's bits
+  uint64_t T;      // integer CDF total, or the FP32 total's bits (BUILD: group_select)
 };
 
 // Entry + its ITS state.  For KIND == kInt the CDF cache of the entry's bias

@@ -64,7 +64,8 @@ typedef enum csaw_variant {
 
 typedef enum csaw_sched {
   CSAW_SCHED_HEURISTIC = 0, /* C-SAW degree thresholds (util.h:19-20)         */
-  CSAW_SCHED_MLP = 1,       /* learned cost model, heuristic as fallback      */
+  CSAW_SCHED_MLP = 1,       /* learned cost model, heuristic as fallback; it  */
+                            /*  picks for the hops that are binned           */
   CSAW_SCHED_FORCED = 2,    /* one variant for every chunk it is valid for    */
   CSAW_SCHED_RANDOM = 3     /* random valid variant per chunk (training data) */
 } csaw_sched;
@@ -248,6 +249,14 @@ typedef struct csaw_request {
   const int32_t *seeds; /* host, `samples` entries */
 } csaw_request;
 
+/* A batched plan under the heuristic or learned schedule expands a hop whole,
+ * in frontier order with one kernel per bias kind, where no entry would gain from
+ * a variant: uniform and FP32 biases, integer biases over 32-bit CDFs (the cache;
+ * without it degree bias, unless its collisions are resolved by region remap), and
+ * hops of at most 65,536 entries.  Other hops,
+ * and every hop under forced or random variants or with log_chunks, are binned
+ * into chunks, each run by the variant that `sched` picks.  The edges are the
+ * same; a cost model given for CSAW_SCHED_MLP is consulted for binned hops only. */
 typedef struct csaw_plan_opts {
   int32_t mode;      /* csaw_mode                                          */
   int32_t sched;     /* csaw_sched                                         */
@@ -260,9 +269,10 @@ typedef struct csaw_plan_opts {
   const struct csaw_tuning *tuning; /* launch shapes (or NULL: defaults)   */
   int32_t cdf_cache; /* integer-bias draws use the per-graph CDF cache (the */
                      /* reference's Cp, functions.cuh:329-341; off there)   */
-  int32_t serial_expand; /* batched: run a hop's variant kernels one after */
-                         /* another on one stream (default: side by side  */
-                         /* on four streams)                               */
+  int32_t serial_expand; /* batched: run a hop's kernels (one per bias     */
+                         /* kind, or the variants) one after another on    */
+                         /* one stream (default: side by side on up to     */
+                         /* four streams)                                  */
 } csaw_plan_opts;
 
 typedef struct csaw_plan csaw_plan;
