@@ -228,6 +228,7 @@ hipError_t device_malloc(void** p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
   if (e == hipSuccess) return e;
   (void)hipGetLastError();
+  if (e != hipErrorOutOfMemory) return e;  // (a stream being captured, for one: frees are refused then too)
   std::vector<Workspace::Block> out;
   {
     Pools& P = pools();

@@ -75,8 +75,8 @@ int mlp_upload_bf16(const csaw_mlp* m, uint16_t* dst);
 // until the call has waited for it.  A call that does not wait, or whose launch or
 // wait fails, leaves its count.
 struct InFlight {
-  std::atomic<int>& n;
-  explicit InFlight(std::atomic<int>& count) : n(count) { ++n; }
+  std::atomic<int64_t>& n;
+  explicit InFlight(std::atomic<int64_t>& count) : n(count) { ++n; }
   void waited() { --n; }
 };
 
@@ -99,7 +99,7 @@ struct csaw_plan {
   // every device array below and the units' (one allocation)
   std::shared_ptr<csaw::Workspace> work;
   csaw::Workspace::Block slab;
-  mutable std::atomic<int> unwaited{0};  // calls whose work may still use it (InFlight)
+  mutable std::atomic<int64_t> unwaited{0};  // calls whose work may still use it (InFlight)
   int32_t* staging = nullptr;         // csaw_sample: the result, packed for one copy
   // counter block, then the requests' edge bounds (kCtrBytes + n_req *
   // kBoundsBytes): one copy into h_state after a synchronised run brings the

@@ -11,6 +11,7 @@
 
 #include <cstdint>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <string>
@@ -121,6 +122,7 @@ hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) {
 }
 hipError_t hipMalloc(void** p, size_t n) {
   FakeHip& f = fake();
+  if (f.fails("hipMalloc as unsupported")) return hipErrorStreamCaptureUnsupported;
   if (f.fails("hipMalloc") || n > f.limit - f.used) return hipErrorOutOfMemory;
   void* q = mmap(nullptr, n, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
   if (q == MAP_FAILED) return hipErrorOutOfMemory;

@@ -258,6 +258,14 @@ static void pool_makes_room() {
   const csaw_request big = request(4000, {64, 64}, CSAW_BIAS_UNIFORM, seeds.data());
   csaw_plan* p = nullptr;
   NEED(csaw_plan_create(g, &big, 1, nullptr, &p) == CSAW_ERR_OOM);
+  // an allocation refused for another reason (a stream is being captured) leaves the
+  // pools as they are
+  fill();
+  fake().limit = SIZE_MAX;
+  fake().log.clear();
+  fake().fail_in["hipMalloc as unsupported"] = 1;
+  NEED(csaw_seeds(g, 1, 0, 100, out.data()) == CSAW_ERR_HIP);
+  NEED(!fake().logged("free on"));
   csaw_mlp_destroy(m);
   csaw_host_graph_destroy(hg);
   csaw_graph_destroy(hubs);
